@@ -1,0 +1,719 @@
+// Many tokens through one weight matrix on the matrix cores, every GGUF format (gfx950):
+//   hh_mmg_amax                 per token the power of two that its f16 operands are scaled by
+//   hh_mmg_conv                 tokens [b][n] f32 -> token stages (below)
+//   hh_mmg_<fmt>_<mode>         Y[t][r] = W[r] . X[t] (execute_quant_gemv_batched, crates/
+//                               hayai-core/src/orchestrator.rs:240-269)
+//   hh_mmg_<fmt>_<mode>_gu      h[t][r] = act(W_gate[r] . X[t]) * (W_up[r] . X[t]) (prefill_
+//                               batched's gate/up, crates/hayai-core/src/prefill_wave.rs:569-584)
+//   hh_mmg_sum, hh_mmg_sum_act  the sums of split columns, in split order
+// (Compiled after mm_common.hip: its vector types and hh_split_f16.)
+//
+// Arithmetic.  Weights enter the f16 matrix cores as the exact integers of their format and
+// meet their f32 scale after the products: w = d * code, code = q - 8 (Q4_0), q (Q8_0), sc q
+// (Q4_K, <= 945), (2 s + 1) * +-grid (IQ2_XXS <= 1333, IQ3_XXS <= 1922), and for Q6_K sc (q - 32)
+// up to 4096 as its f16 rounding plus the remainder (-1, 0 or 1), each exact.  A token's
+// elements are scaled by one power of two (its largest magnitude into [512, 1024)) and split
+// into two f16, hi + lo, which carry 22 bits; products are summed in f32 by the matrix cores
+// over one scale block (32 or 256 columns), then d times that is added to the running sum.
+// Measured against 64 bits: 1e-7 to 4e-7, as the one-token f32 kernels.
+// The Q4_K minimum is dmin * sum_j m_j X_j with X_j the f32 sum of the token's 32 elements of
+// sub-block j, as hi + lo f16: one MFMA per superblock (k slots 0..7 hi, 8..15 lo).
+//
+// MFMA mapping (v_mfma_f32_32x32x16_f16): A = 32 token rows, B = 32 weight rows, so that lane l
+// holds outputs of weight row l % 32 only and d is one register per lane.  Lane l supplies k
+// slots 8 (l / 32) .. + 7 of its token / its weight row.  A 32-column group takes two steps;
+// half h = l / 32 of a weight row's lanes decodes 16 of the group's 32 columns from bytes that
+// are contiguous in the block, and the stage is written in the order that gives:
+//   columns 16 h + 8 step + e  (Q8_0, Q4_K, Q6_K, IQ)   or   16 step + 8 h + e  (Q4_0),
+//   e natural (Q8_0, IQ) or 0 2 1 3 4 6 5 7 (nibble pairs of a dword).
+// Weights go from global memory to registers to the matrix core; only tokens pass through LDS,
+// shared by the workgroup's four waves.  A wave owns 64 weight rows (32 of gate and the same 32
+// of up), so each 1 KB token fragment read from LDS feeds two MFMAs.
+//
+// Modes (chosen by the token count alone, plan_mmg): h<TT>: TT tiles of 32 tokens, hi and lo as two MFMAs; s16: 16 tokens, hi in A rows
+// 0..15 and lo in rows 16..31 of one MFMA, added at the end.
+//
+// What bounds it: at hundreds of tokens the matrix cores with the weight decode beside them (8B
+// FFN, 512 tokens, 2 x 180 GFLOP of hi and lo: 0.52 ms IQ2_XXS .. 0.78 ms Q8_0, 460 .. 690 TFLOP/s;
+// one token at a time these took 12 .. 39 ms); at 4..16 tokens the weight stream's latency (8B
+// Q6_K FFN, 16 tokens: 106 us against 779 us).
+//
+// Token stages: [tile][128-column chunk][group 0..3][step 0..1][hi, lo][lane][8 f16], for Q4_K
+// followed after every second chunk by the sums [lane][8 f16] (lane half 0: hi of sub-blocks
+// 0..7, half 1: lo).
+typedef float hh_f16v __attribute__((ext_vector_type(16)));
+
+enum { HH_MMG_H = 0, HH_MMG_S16 = 1 };
+
+struct hh_mmg_args {
+    const uint8_t* w0;       // GEMM: W; gate/up: W_gate
+    const uint8_t* w1;       // GEMM: W; gate/up: W_up
+    const uint8_t* xs;       // token stages
+    const float* down;       // per token: the power of two that undoes its scaling
+    float* y;                // kc == 1: Y [b][m] or h [b][m]; else the splits' sums
+    uint64_t row_bytes;
+    uint64_t tile_bytes;     // stage bytes of one token tile
+    uint64_t part_stride;    // kc > 1: floats between two splits' sums
+    uint64_t up_stride;      // kc > 1, gate/up: floats from gate's sums to up's
+    uint32_t m, n, b;
+    uint32_t nch;            // 128-column chunks (the last may be partly past n)
+    uint32_t cpk;            // chunks per split (even for formats of 256-column blocks)
+    uint32_t kc;             // splits
+    uint32_t groups;         // row groups
+    uint32_t ttiles;         // token tile groups
+    int32_t act;
+    uint32_t pad;
+};
+
+// Bytes at any address (2-byte aligned in GGUF formats): the hardware takes unaligned loads.
+HH_DEV uint4 hh_ldu16(const uint8_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+HH_DEV uint2 hh_ldu8(const uint8_t* p) {
+    uint2 v;
+    __builtin_memcpy(&v, p, 8);
+    return v;
+}
+HH_DEV uint32_t hh_ldu4(const uint8_t* p) {
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+
+HH_DEV hh_h2 hh_h2_all(float v) { return hh_h2{(_Float16)v, (_Float16)v}; }
+HH_DEV hh_h8 hh_h8_of(hh_h2 a, hh_h2 b, hh_h2 c, hh_h2 d) { return hh_h8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y}; }
+// bytes i and j of v as the f16 pair 1024 + byte
+template <uint32_t I, uint32_t J>
+HH_DEV hh_h2 hh_bytes_h2(uint32_t v) {
+    return hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, v, I | (4u << 8) | (J << 16) | (4u << 24)));
+}
+
+// ---- weight formats -------------------------------------------------------------------
+// Raw: one chunk's bytes of one row as loaded; load(p, ch, ...) of chunk ch of the row at p
+// (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
+// the d of the block that group g closes.  NB: B operands per step.
+struct hh_mmg_q4_0 {
+    static constexpr bool SUPER = false, MINS = false, TABLES = false;
+    static constexpr int NB = 1;
+    struct Raw {
+        uint2 q[4];
+        uint32_t d[4];
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++) {
+            const uint32_t k = 4 * ch + g;
+            const uint8_t* b = p + min(k, nblk - 1) * 18u;
+            r.q[g] = hh_ldu8(b + 2 + 8 * h);
+            r.d[g] = k < nblk ? hh_ld_u16(b) : 0u;
+        }
+    }
+    HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+        const uint32_t v[4] = {r.q[g].x, r.q[g].x >> 8, r.q[g].y, r.q[g].y >> 8};
+        hh_h2 o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (s == 0)  // 1024 + q, q - 8
+                o[i] = hh_h2_bits((v[i] & 0x000F000Fu) | 0x64006400u) - hh_h2_all(1032.f);
+            else  // 1024 + 16 q, q - 8 (exact: the FMA rounds only its result)
+                o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & 0x00F000F0u) | 0x64006400u), hh_h2_all(0.0625f),
+                                                 hh_h2_all(-72.f));
+        }
+        f[0] = hh_h8_of(o[0], o[1], o[2], o[3]);
+    }
+};
+
+struct hh_mmg_q8_0 {
+    static constexpr bool SUPER = false, MINS = false, TABLES = false;
+    static constexpr int NB = 1;
+    struct Raw {
+        uint4 q[4];
+        uint32_t d[4];
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++) {
+            const uint32_t k = 4 * ch + g;
+            const uint8_t* b = p + min(k, nblk - 1) * 34u;
+            r.q[g] = hh_ldu16(b + 2 + 16 * h);
+            r.d[g] = k < nblk ? hh_ld_u16(b) : 0u;
+        }
+    }
+    HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+        const uint32_t a = (s ? r.q[g].z : r.q[g].x) ^ 0x80808080u, b = (s ? r.q[g].w : r.q[g].y) ^ 0x80808080u;
+        const hh_h2 z = hh_h2_all(1152.f);  // 1024 + (q + 128)
+        f[0] = hh_h8_of(hh_bytes_h2<0, 1>(a) - z, hh_bytes_h2<2, 3>(a) - z, hh_bytes_h2<0, 1>(b) - z,
+                        hh_bytes_h2<2, 3>(b) - z);
+    }
+};
+
+struct hh_mmg_q4_k {
+    static constexpr bool SUPER = true, MINS = true, TABLES = false;
+    static constexpr int NB = 1;
+    struct Raw {
+        uint4 q[2];
+        uint4 hd;
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t) {
+        const uint8_t* b = p + (ch >> 1) * 144u;
+        r.hd = hh_ld16(b);
+        r.q[0] = hh_ld16(b + 16 + 64 * HALF + 16 * h);
+        r.q[1] = hh_ld16(b + 48 + 64 * HALF + 16 * h);
+    }
+    HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.hd.x & 0xFFFFu); }
+    HH_DEV static float min_scale(const Raw& r) { return hh_f16(r.hd.x >> 16); }
+    // the minima m_0 .. m_7 (get_scale_min_k4, q4k.rs:34-43), the same in both lane halves
+    HH_DEV static hh_h8 mins(const Raw& r) {
+        const uint32_t lo = r.hd.z & 0x3F3F3F3Fu, hi = ((r.hd.w >> 4) & 0x0F0F0F0Fu) | ((r.hd.z >> 2) & 0x30303030u);
+        const hh_h2 z = hh_h2_all(1024.f);
+        return hh_h8_of(hh_bytes_h2<0, 1>(lo) - z, hh_bytes_h2<2, 3>(lo) - z, hh_bytes_h2<0, 1>(hi) - z,
+                        hh_bytes_h2<2, 3>(hi) - z);
+    }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+        // the chunk's four sub-block scales; sub-blocks 2p (low nibbles) and 2p + 1 (high) of
+        // the 32 qs bytes p
+        const uint32_t sch =
+            HALF ? (r.hd.w & 0x0F0F0F0Fu) | ((r.hd.y >> 2) & 0x30303030u) : r.hd.y & 0x3F3F3F3Fu;
+        const uint4 q = r.q[g >> 1];
+        const uint32_t a = s ? q.z : q.x, b = s ? q.w : q.y;
+        const uint32_t v[4] = {a, a >> 8, b, b >> 8};
+        const uint32_t sel = (uint32_t)g | (4u << 8) | ((uint32_t)g << 16) | (4u << 24);
+        const hh_h2 sc = hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, sch, sel)) - hh_h2_all(1024.f);
+        const hh_h2 mul = (g & 1) ? sc * hh_h2_all(0.0625f) : sc;
+        const hh_h2 off = mul * hh_h2_all(-1024.f);
+        const uint32_t mask = (g & 1) ? 0x00F000F0u : 0x000F000Fu;
+        hh_h2 o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & mask) | 0x64006400u), mul, off);
+        f[0] = hh_h8_of(o[0], o[1], o[2], o[3]);
+    }
+};
+
+struct hh_mmg_q6_k {
+    static constexpr bool SUPER = true, MINS = false, TABLES = false;
+    static constexpr int NB = 2;
+    struct Raw {
+        uint4 a, b, qh;
+        uint2 sc;
+        uint32_t d;
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t) {
+        const uint8_t* b = p + (ch >> 1) * 210u;
+        const uint32_t n = HALF;
+        r.a = hh_ldu16(b + 64 * n + 16 * h);
+        r.b = hh_ldu16(b + 64 * n + 32 + 16 * h);
+        r.qh = hh_ldu16(b + 128 + 32 * n + 16 * h);
+        r.sc = hh_ldu8(b + 192 + 8 * n);
+        r.d = hh_ld_u16(b + 208);
+    }
+    HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d); }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char*, hh_h8* f) {
+        const uint4 l = (g & 1) ? r.b : r.a;
+        const uint32_t la = s ? l.z : l.x, lb = s ? l.w : l.y, ha = s ? r.qh.z : r.qh.x, hb = s ? r.qh.w : r.qh.y;
+        // scale byte 2 g + h of the chunk's eight
+        const uint32_t sw = (g & 2) ? r.sc.y : r.sc.x;
+        const float scf = (float)(int8_t)(sw >> (16 * (g & 1) + 8 * h));
+        const hh_h2 sc = hh_h2_all(scf);
+        const uint32_t q[2] = {((g & 2) ? (la >> 4) & 0x0F0F0F0Fu : la & 0x0F0F0F0Fu) | (((ha >> (2 * g)) & 0x03030303u) << 4),
+                               ((g & 2) ? (lb >> 4) & 0x0F0F0F0Fu : lb & 0x0F0F0F0Fu) | (((hb >> (2 * g)) & 0x03030303u) << 4)};
+        hh_h2 hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t v = q[i >> 1];
+            const hh_h2 t = ((i & 1) ? hh_bytes_h2<2, 3>(v) : hh_bytes_h2<0, 1>(v)) - hh_h2_all(1056.f);
+            hi[i] = t * sc;                                        // rounded to f16
+            lo[i] = __builtin_elementwise_fma(t, sc, -hi[i]);      // the rest, exact
+        }
+        f[0] = hh_h8_of(hi[0], hi[1], hi[2], hi[3]);
+        f[1] = hh_h8_of(lo[0], lo[1], lo[2], lo[3]);
+    }
+};
+
+// IQ tables as f16: the codebook entries' magnitudes, and per sign index a mask of sign bits.
+constexpr uint16_t hh_f16_of_small(uint32_t v) {  // an integer below 2048 as f16 bits
+    uint32_t e = 0;
+    while ((v >> (e + 1)) != 0) e++;
+    return v == 0 ? (uint16_t)0 : (uint16_t)(((e + 15) << 10) | ((v << (10 - e)) & 0x3FFu));
+}
+struct hh_mmg_iq2_tab {
+    uint16_t grid[256 * 8];
+    uint16_t sign[128 * 8];
+};
+struct hh_mmg_iq3_tab {
+    uint16_t grid[256 * 4];
+    uint16_t sign[128 * 8];
+};
+constexpr void hh_mmg_signs(uint16_t* s) {
+    for (uint32_t i = 0; i < 128; i++) {
+        uint32_t par = 0;
+        for (uint32_t k = 0; k < 7; k++) par ^= (i >> k) & 1u;
+        for (uint32_t k = 0; k < 8; k++) s[8 * i + k] = ((k < 7 ? (i >> k) & 1u : par) != 0) ? 0x8000u : 0u;
+    }
+}
+constexpr hh_mmg_iq2_tab hh_mmg_make_iq2() {
+    constexpr uint64_t g[256] = {HH_IQ2XXS_GRID_VALUES};
+    hh_mmg_iq2_tab t{};
+    for (uint32_t i = 0; i < 256; i++)
+        for (uint32_t k = 0; k < 8; k++) t.grid[8 * i + k] = hh_f16_of_small((uint32_t)(g[i] >> (8 * k)) & 0xFFu);
+    hh_mmg_signs(t.sign);
+    return t;
+}
+constexpr hh_mmg_iq3_tab hh_mmg_make_iq3() {
+    constexpr uint32_t g[256] = {HH_IQ3XXS_GRID_VALUES};
+    hh_mmg_iq3_tab t{};
+    for (uint32_t i = 0; i < 256; i++)
+        for (uint32_t k = 0; k < 4; k++) t.grid[4 * i + k] = hh_f16_of_small((g[i] >> (8 * k)) & 0xFFu);
+    hh_mmg_signs(t.sign);
+    return t;
+}
+__device__ const __attribute__((aligned(16))) hh_mmg_iq2_tab hh_mmg_iq2_table = hh_mmg_make_iq2();
+__device__ const __attribute__((aligned(16))) hh_mmg_iq3_tab hh_mmg_iq3_table = hh_mmg_make_iq3();
+
+HH_DEV hh_h8 hh_mmg_iq_frag(uint4 grid, uint4 sign, uint32_t aux) {
+    const hh_h2 sc = hh_h2_all((float)(2u * (aux >> 28) + 1u));
+    return hh_h8_of(hh_h2_bits(grid.x ^ sign.x) * sc, hh_h2_bits(grid.y ^ sign.y) * sc,
+                    hh_h2_bits(grid.z ^ sign.z) * sc, hh_h2_bits(grid.w ^ sign.w) * sc);
+}
+
+struct hh_mmg_iq2_xxs {
+    static constexpr bool SUPER = true, MINS = false, TABLES = true;
+    static constexpr int NB = 1;
+    static constexpr uint32_t TAB = sizeof(hh_mmg_iq2_tab);
+    HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq2_table; }
+    struct Raw {
+        uint2 q[4];
+        uint32_t d;
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t, uint32_t) {
+        const uint8_t* b = p + (ch >> 1) * 66u;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++) r.q[g] = hh_ldu8(b + 2 + 8 * (4 * HALF + g));
+        r.d = hh_ld_u16(b);
+    }
+    // d * (0.5 + s) * 0.25 = d / 8 * (2 s + 1)
+    HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d) * 0.125f; }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, hh_h8* f) {
+        const uint32_t l = 2 * h + (uint32_t)s, aux = r.q[g].y;
+        const uint32_t idx = (r.q[g].x >> (8 * l)) & 0xFFu, sg = (aux >> (7 * l)) & 127u;
+        f[0] = hh_mmg_iq_frag(*reinterpret_cast<const uint4*>(tab + idx * 16),
+                              *reinterpret_cast<const uint4*>(tab + 4096 + sg * 16), aux);
+    }
+};
+
+struct hh_mmg_iq3_xxs {
+    static constexpr bool SUPER = true, MINS = false, TABLES = true;
+    static constexpr int NB = 1;
+    static constexpr uint32_t TAB = sizeof(hh_mmg_iq3_tab);
+    HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq3_table; }
+    struct Raw {
+        uint32_t q[4];
+        uint4 aux;
+        uint32_t d;
+    };
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t) {
+        const uint8_t* b = p + (ch >> 1) * 98u;
+        const uint32_t n = HALF;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; g++) r.q[g] = hh_ldu4(b + 2 + 8 * (4 * n + g) + 4 * h);
+        r.aux = hh_ldu16(b + 66 + 16 * n);
+        r.d = hh_ld_u16(b);
+    }
+    // d * (0.5 + s) * 0.5 = d / 4 * (2 s + 1)
+    HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d) * 0.25f; }
+    template <uint32_t HALF>
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, hh_h8* f) {
+        const uint32_t l = 2 * h + (uint32_t)s;
+        const uint32_t aux = g == 0 ? r.aux.x : g == 1 ? r.aux.y : g == 2 ? r.aux.z : r.aux.w;
+        const uint32_t i0 = (r.q[g] >> (16 * s)) & 0xFFu, i1 = (r.q[g] >> (16 * s + 8)) & 0xFFu;
+        const uint2 a = *reinterpret_cast<const uint2*>(tab + i0 * 8), b = *reinterpret_cast<const uint2*>(tab + i1 * 8);
+        f[0] = hh_mmg_iq_frag(make_uint4(a.x, a.y, b.x, b.y),
+                              *reinterpret_cast<const uint4*>(tab + 2048 + ((aux >> (7 * l)) & 127u) * 16), aux);
+    }
+};
+
+// ---- tokens -> stages -----------------------------------------------------------------
+
+struct hh_mmg_conv_args {
+    const float* x;        // [b][n]
+    uint8_t* xs;           // stages
+    const float* up;       // per token: its power of two
+    uint64_t tile_bytes;
+    uint32_t b, n, nch;
+    uint32_t rows;         // tokens per tile: 32, or 16 (mode s16)
+    uint32_t mins;         // write the sub-block sums
+    uint32_t half_major;   // column order 16 h + 8 step + e (else 16 step + 8 h + e)
+    uint32_t paired;       // e in the order 0 2 1 3 4 6 5 7
+    uint32_t pad;
+};
+
+struct hh_mmg_amax_args {
+    const float* x;  // [b][n]
+    float* up;
+    float* down;
+    uint32_t n, pad;
+};
+
+// One workgroup per token.  amax in [2^(k-1), 2^k) -> up = 2^(10 - k): the largest magnitude
+// into [512, 1024), so that a sum of 32 elements stays below f16's largest value.  A token
+// without a finite, non-zero maximum keeps the factor 1 (its infinities stay infinities).
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_amax(const hh_mmg_amax_args a) {
+    __shared__ float red[4];
+    const float* x = a.x + (size_t)blockIdx.x * a.n;
+    float v = 0.f;
+    for (uint32_t i = threadIdx.x; i < a.n; i += 256) v = fmaxf(v, fabsf(x[i]));
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+        int e = 0;
+        if (v > 0.f && v < __builtin_inff()) {
+            int k;
+            (void)frexpf(v, &k);
+            e = min(max(10 - k, -120), 120);
+        }
+        a.up[blockIdx.x] = ldexpf(1.f, e);
+        a.down[blockIdx.x] = ldexpf(1.f, -e);
+    }
+}
+
+HH_DEV void hh_mmg_split(float v, _Float16& hi, _Float16& lo) {
+    hi = (_Float16)v;
+    const float r = v - (float)hi;
+    lo = (_Float16)(r == r ? r : 0.f);  // an infinite v: hi carries it alone
+}
+
+// One workgroup per (token tile, chunk); tokens past b and columns past n are zeros.
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_conv(const hh_mmg_conv_args a) {
+    const uint32_t tile = blockIdx.x / a.nch, ch = blockIdx.x % a.nch;
+    const bool s16 = a.rows == 16;
+    const uint32_t chunk_bytes = (s16 ? 8u : 16u) * 1024u;
+    uint8_t* st = a.xs + tile * a.tile_bytes +
+                  (a.mins ? (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + (ch & 1u) * chunk_bytes
+                          : (size_t)ch * chunk_bytes);
+    const bool vec = ((uintptr_t)a.x & 15u) == 0;
+    for (uint32_t p = threadIdx.x; p < (s16 ? 256u : 512u); p += 256) {
+        // piece p: group, step, lane half, token
+        const uint32_t tok = p % a.rows, h = (p / a.rows) & 1u, step = (p / a.rows >> 1) & 1u, g = p / a.rows >> 2;
+        const uint32_t t = tile * a.rows + tok;
+        const uint32_t col = 128 * ch + 32 * g + (a.half_major ? 16 * h + 8 * step : 16 * step + 8 * h);
+        float v[8];
+        if (t < a.b && col < a.n) {
+            const float* src = a.x + (size_t)t * a.n + col;
+            const float up = a.up[t];
+            if (vec) {
+                const float4 u0 = reinterpret_cast<const float4*>(src)[0], u1 = reinterpret_cast<const float4*>(src)[1];
+                v[0] = u0.x, v[1] = u0.y, v[2] = u0.z, v[3] = u0.w, v[4] = u1.x, v[5] = u1.y, v[6] = u1.z, v[7] = u1.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = src[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] *= up;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = 0.f;
+        }
+        if (a.paired) {
+            float s = v[1];
+            v[1] = v[2], v[2] = s;
+            s = v[5];
+            v[5] = v[6], v[6] = s;
+        }
+        hh_h8 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            _Float16 x0, x1;
+            hh_mmg_split(v[e], x0, x1);
+            hi[e] = x0;
+            lo[e] = x1;
+        }
+        const uint32_t gs = g * 2 + step;
+        if (s16) {
+            *reinterpret_cast<hh_h8*>(st + gs * 1024u + (32 * h + tok) * 16u) = hi;
+            *reinterpret_cast<hh_h8*>(st + gs * 1024u + (32 * h + 16 + tok) * 16u) = lo;
+        } else {
+            *reinterpret_cast<hh_h8*>(st + gs * 2048u + (32 * h + tok) * 16u) = hi;
+            *reinterpret_cast<hh_h8*>(st + gs * 2048u + 1024u + (32 * h + tok) * 16u) = lo;
+        }
+    }
+    if (!a.mins) return;
+    uint8_t* sums = a.xs + tile * a.tile_bytes + (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + 2 * chunk_bytes;
+    const uint32_t q = threadIdx.x;  // token row, group
+    if (q >= 128) return;
+    const uint32_t row = q % 32, g = q / 32, j = 4 * (ch & 1u) + g, t = tile * a.rows + row;
+    float s = 0.f;
+    if (row < a.rows && t < a.b) {
+        const float* src = a.x + (size_t)t * a.n + 128 * ch + 32 * g;
+        const float up = a.up[t];
+        for (int e = 0; e < 32; e++) s += src[e] * up;
+    }
+    _Float16 hi, lo;
+    hh_mmg_split(s, hi, lo);
+    *reinterpret_cast<_Float16*>(sums + row * 16 + j * 2) = hi;         // s16: rows 16..31 are zeros
+    *reinterpret_cast<_Float16*>(sums + 512 + row * 16 + j * 2) = lo;
+}
+
+template <uint32_t V>
+struct hh_uint_c {
+    static constexpr uint32_t value = V;
+};
+
+// ---- the product ----------------------------------------------------------------------
+
+// Tokens' LDS copies in flight and all LDS reads of this wave done, then the workgroup meets.
+HH_DEV void hh_mmg_sync() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <class F, int MODE, int TT, bool GU>
+HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
+    constexpr int NA = MODE == HH_MMG_H ? 2 : 1;
+    constexpr uint32_t CB = 8u * NA * 1024u;            // stage bytes of a (tile, chunk)
+    constexpr uint32_t SUMS = F::MINS ? 1024u : 0u;
+    constexpr uint32_t BUF = TT * (CB + SUMS);
+    constexpr uint32_t ROWS = MODE == HH_MMG_S16 ? 16 : 32;  // tokens per tile
+    extern __shared__ __attribute__((aligned(16))) char hh_smem[];
+    const uint32_t tid = threadIdx.x, lane = tid % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const uint32_t r = lane & 31u, h = lane >> 5;
+    // workgroup -> (row group, split, token tiles): the token tiles of one (row group, split) sit
+    // on one XCD one after another, so its weights come from memory once and from L2 after
+    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const uint32_t unit = slot / a.ttiles * 8u + xcd, tg = slot % a.ttiles;
+    if (unit >= a.groups * a.kc) return;
+    const uint32_t grp = unit / a.kc, kci = unit % a.kc;
+    const uint32_t c0 = kci * a.cpk, c1 = min(c0 + a.cpk, a.nch);
+    const uint32_t nblk = a.n / 32;
+
+    uint32_t row[2];
+    const uint8_t* wp[2];
+    row[0] = GU ? grp * 128 + wave * 32 + r : grp * 256 + wave * 64 + r;
+    row[1] = GU ? row[0] : row[0] + 32;
+    wp[0] = a.w0 + (size_t)min(row[0], a.m - 1) * a.row_bytes;
+    wp[1] = a.w1 + (size_t)min(row[1], a.m - 1) * a.row_bytes;
+
+    if constexpr (F::TABLES) {
+        char* tab = hh_smem + 2 * BUF;
+        for (uint32_t i = tid; i < F::TAB / 16; i += 256)
+            reinterpret_cast<uint4*>(tab)[i] = reinterpret_cast<const uint4*>(F::table())[i];
+    }
+    const char* const tab = hh_smem + 2 * BUF;
+
+    auto copy = [&](uint32_t ch, auto buf_c) {
+        constexpr uint32_t buf = decltype(buf_c)::value;
+        const size_t at = F::MINS ? (size_t)(ch >> 1) * (2 * CB + SUMS) + buf * CB : (size_t)ch * CB;
+#pragma unroll
+        for (uint32_t i = 0; i < TT * CB / 4096u; i++) {
+            const uint32_t u = i * 4 + wave, tt = u / (CB / 1024u), o = u % (CB / 1024u);
+            const uint8_t* src = a.xs + (size_t)(tg * TT + tt) * a.tile_bytes + at + o * 1024u + lane * 16u;
+            char* dst = hh_smem + buf * BUF + tt * (CB + SUMS) + o * 1024u;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+        }
+        if constexpr (F::MINS && buf == 1) {
+            if (wave < TT) {
+                const uint8_t* src = a.xs + (size_t)(tg * TT + wave) * a.tile_bytes + at + CB + lane * 16u;
+                char* dst = hh_smem + buf * BUF + wave * (CB + SUMS) + CB;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                                 (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+            }
+        }
+    };
+
+    hh_f16v sum[2][TT], part[2][TT];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum[q][tt][i] = part[q][tt][i] = 0.f;
+
+    // one chunk out of LDS buffer `buf`: for formats of 256-column blocks the first or second
+    // half of one (splits start at even chunks)
+    auto compute = [&](const typename F::Raw* raw, auto buf_c) {
+        constexpr uint32_t buf = decltype(buf_c)::value;
+        constexpr bool open = buf == 0, close = buf == 1;
+        const char* st = hh_smem + buf * BUF + lane * 16u;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                hh_h8 wf[2][F::NB];
+#pragma unroll
+                for (int q = 0; q < 2; q++) F::template frag<buf>(raw[q], g, s, h, tab, wf[q]);
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) {
+                    const char* p = st + tt * (CB + SUMS) + (g * 2 + s) * (NA * 1024);
+                    const hh_h8 x0 = *reinterpret_cast<const hh_h8*>(p);
+                    hh_h8 x1;
+                    if constexpr (NA == 2) x1 = *reinterpret_cast<const hh_h8*>(p + 1024);
+                    const bool fresh = s == 0 && (F::SUPER ? open && g == 0 : true);
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        hh_f16v c = part[q][tt];
+                        if (fresh) {
+#pragma unroll
+                            for (int i = 0; i < 16; i++) c[i] = 0.f;
+                        }
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x0, wf[q][0], c, 0, 0, 0);
+                        if constexpr (NA == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x1, wf[q][0], c, 0, 0, 0);
+                        if constexpr (F::NB == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x0, wf[q][1], c, 0, 0, 0);
+                        part[q][tt] = c;
+                    }
+                }
+            }
+            if (!F::SUPER || (close && g == 3)) {
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const float d = F::scale(raw[q], g);
+#pragma unroll
+                    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) sum[q][tt][i] = fmaf(d, part[q][tt][i], sum[q][tt][i]);
+                }
+            }
+        }
+        if constexpr (F::MINS) {
+            if (close) {
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const hh_h8 mf = F::mins(raw[q]);
+                    const float dm = -F::min_scale(raw[q]);
+#pragma unroll
+                    for (int tt = 0; tt < TT; tt++) {
+                        const hh_h8 xs = *reinterpret_cast<const hh_h8*>(st + tt * (CB + SUMS) + CB);
+                        hh_f16v c;
+#pragma unroll
+                        for (int i = 0; i < 16; i++) c[i] = 0.f;
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, mf, c, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 16; i++) sum[q][tt][i] = fmaf(dm, c[i], sum[q][tt][i]);
+                    }
+                }
+            }
+        }
+    };
+
+    typename F::Raw raw[2][2];  // [buffer][row tile]
+    constexpr hh_uint_c<0> B0{};
+    constexpr hh_uint_c<1> B1{};
+    copy(c0, B0);
+#pragma unroll
+    for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], c0, h, nblk);
+    for (uint32_t ch = c0; ch < c1; ch += 2) {
+        // chunk ch's tokens have landed for every wave, and buffer 1 is free
+        hh_mmg_sync();
+        const bool two = F::SUPER || ch + 1 < c1;
+        if (two) {
+            copy(ch + 1, B1);
+#pragma unroll
+            for (int q = 0; q < 2; q++) F::template load<1>(raw[1][q], wp[q], ch + 1, h, nblk);
+        }
+        compute(raw[0], B0);
+        if (!two) break;
+        hh_mmg_sync();
+        if (ch + 2 < c1) {
+            copy(ch + 2, B0);
+#pragma unroll
+            for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], ch + 2, h, nblk);
+        }
+        compute(raw[1], B1);
+    }
+
+    // outputs: lane's weight row, tokens 8 (i / 4) + 4 h + i % 4 of each tile
+    float* const out = a.y + (a.kc > 1 ? kci * a.part_stride : 0);
+    const bool fuse = GU && a.kc == 1;
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++) {
+#pragma unroll
+        for (int i4 = 0; i4 < (MODE == HH_MMG_S16 ? 2 : 4); i4++) {
+            const uint32_t t0 = (tg * TT + tt) * ROWS + 8 * i4 + 4 * h;
+            const float4 d4 = *reinterpret_cast<const float4*>(a.down + t0);  // padded to whole tiles
+            const float dn[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint32_t t = t0 + k;
+                if (t >= a.b) continue;
+                float v[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    v[q] = sum[q][tt][4 * i4 + k];
+                    if constexpr (MODE == HH_MMG_S16) v[q] += sum[q][tt][4 * i4 + k + 8];
+                    v[q] *= dn[k];
+                }
+                if (fuse) {
+                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = hh_act_mul(v[0], v[1], a.act);
+                } else {
+                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = v[0];
+                    if (row[1] < a.m) out[(GU ? a.up_stride : 0) + (size_t)t * a.m + row[1]] = v[1];
+                }
+            }
+        }
+    }
+}
+
+struct hh_mmg_sum_args {
+    const float* part;     // [kc][count] (gate/up: gate's, then up's at up_stride)
+    float* y;              // [count]
+    uint64_t stride;       // floats between two splits
+    uint64_t up_stride;
+    uint64_t count;        // floats (a multiple of 4)
+    uint32_t kc;
+    int32_t act;
+};
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum(const hh_mmg_sum_args a) {
+    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+    if (i >= a.count) return;
+    float s = 0.f;
+    for (uint32_t k = 0; k < a.kc; k++) s += a.part[k * a.stride + i];
+    a.y[i] = s;
+}
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_sum_args a) {
+    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x);
+    if (i >= a.count) return;
+    float g = 0.f, u = 0.f;
+    for (uint32_t k = 0; k < a.kc; k++) {
+        g += a.part[k * a.stride + i];
+        u += a.part[k * a.stride + a.up_stride + i];
+    }
+    a.y[i] = hh_act_mul(g, u, a.act);
+}
+
+#define HH_MMG_KERNEL(FMT, NAME, MODE, TT, WPE)                                                                  \
+    extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_##FMT##_##NAME(const hh_mmg_args a) {          \
+        hh_mmg_body<hh_mmg_##FMT, MODE, TT, false>(a);                                                          \
+    }                                                                                                           \
+    extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_##FMT##_##NAME##_gu(const hh_mmg_args a) {     \
+        hh_mmg_body<hh_mmg_##FMT, MODE, TT, true>(a);                                                           \
+    }
+#define HH_MMG_FORMAT(FMT, WPE)               \
+    HH_MMG_KERNEL(FMT, s16, HH_MMG_S16, 1, WPE) \
+    HH_MMG_KERNEL(FMT, h1, HH_MMG_H, 1, WPE)    \
+    HH_MMG_KERNEL(FMT, h2, HH_MMG_H, 2, 2)
+HH_MMG_FORMAT(q4_0, 2)
+HH_MMG_FORMAT(q8_0, 2)
+HH_MMG_FORMAT(q4_k, 3)
+HH_MMG_FORMAT(q6_k, 3)
+HH_MMG_FORMAT(iq2_xxs, 3)
+HH_MMG_FORMAT(iq3_xxs, 3)

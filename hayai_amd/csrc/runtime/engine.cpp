@@ -738,17 +738,25 @@ struct SffnArgs {  // the small FFN kernels' scalar parameters (small_ffn.hip)
     int32_t act;
 };
 
+static int small_team(size_t units) { return units <= 16 ? 16 : (units <= 32 ? 32 : 64); }
+
+bool hh_engine::small_ffn_shape(const hh_ffn_desc* d) const {
+    const size_t dm = d->d_model, df = d->d_ff, G = (size_t)props.multiProcessorCount;
+    return small_ffn && d->type_gate == d->type_up && d->type_up == d->type_down &&
+           (d->type_gate == HH_TYPE_Q4_0 || d->type_gate == HH_TYPE_Q8_0) && dm % 32 == 0 && df % 32 == 0 &&
+           dm / 32 <= 64 && df / 32 <= 64 && (df + G - 1) / G <= 2 * (256 / (size_t)small_team(dm / 32)) &&
+           (dm + G - 1) / G <= 2 * (256 / (size_t)small_team(df / 32));
+}
+
 // A small Q4_0 / Q8_0 FFN in one launch (small_ffn.hip): every workgroup's rows fit its teams
 // (at most two rows per team and phase), one workgroup per CU, a grid barrier between gate/up
 // and down.
 hh_status hh_engine::enqueue_small_ffn(const hh_ffn_desc* d, const uint8_t* wg, const uint8_t* wu, const uint8_t* wd,
                                        const float* x, float* y) {
     const size_t dm = d->d_model, df = d->d_ff, G = (size_t)props.multiProcessorCount;
-    auto team_of = [](size_t units) { return units <= 16 ? 16 : (units <= 32 ? 32 : 64); };
-    const int t1 = team_of(dm / 32), t2 = team_of(df / 32);
-    if (!small_ffn || dm % 32 || df % 32 || dm / 32 > 64 || df / 32 > 64 ||
-        (df + G - 1) / G > 2 * (256 / (size_t)t1) || (dm + G - 1) / G > 2 * (256 / (size_t)t2) ||
-        (((uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd) & 1u) || ((uintptr_t)x & 3u) || ((uintptr_t)y & 3u))
+    const int t1 = small_team(dm / 32), t2 = small_team(df / 32);
+    if (!small_ffn_shape(d) || (((uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd) & 1u) || ((uintptr_t)x & 3u) ||
+        ((uintptr_t)y & 3u))
         return HH_ERR_UNSUPPORTED_DEVICE;
     const std::string name = std::string("hh_sffn_") + (d->type_gate == HH_TYPE_Q4_0 ? "q4_0" : "q8_0") + "_t" +
                              std::to_string(t1) + "_" + std::to_string(t2);
@@ -1115,12 +1123,241 @@ hh_status hh_engine::enqueue_q4k_mmi(bool ffn, size_t m, size_t n, const uint8_t
     return HH_OK;
 }
 
+// ---- many tokens, every format (mmg.hip) ----
+
+// Kernel argument blocks of mmg.hip (same layout).
+struct MmgArgs {
+    const uint8_t* w0;
+    const uint8_t* w1;
+    const uint8_t* xs;
+    const float* down;
+    float* y;
+    uint64_t row_bytes, tile_bytes, part_stride, up_stride;
+    uint32_t m, n, b, nch, cpk, kc, groups, ttiles;
+    int32_t act;
+    uint32_t pad;
+};
+struct MmgConvArgs {
+    const float* x;
+    uint8_t* xs;
+    const float* up;
+    uint64_t tile_bytes;
+    uint32_t b, n, nch, rows, mins, half_major, paired, pad;
+};
+struct MmgAmaxArgs {
+    const float* x;
+    float* up;
+    float* down;
+    uint32_t n, pad;
+};
+struct MmgSumArgs {
+    const float* part;
+    float* y;
+    uint64_t stride, up_stride, count;
+    uint32_t kc;
+    int32_t act;
+};
+constexpr size_t kMmgMaxTokens = 1024;  // tokens per pass (bounds the workspaces)
+// From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
+// 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
+// one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
+// against 32, 6 tokens 43 against 32).
+constexpr size_t kMmgMinTokens = 4, kMmgMinTokensSmallFfn = 5;
+
+struct MmgFmt {
+    int type;
+    bool super, mins, half_major, paired;
+    uint32_t align;      // of the weights
+    uint32_t tab_bytes;  // LDS tables
+    double work;         // MFMAs per step, relative
+};
+static const MmgFmt kMmgFmts[] = {
+    {HH_TYPE_Q4_0, false, false, false, true, 2, 0, 1.0},   {HH_TYPE_Q8_0, false, false, true, false, 2, 0, 1.0},
+    {HH_TYPE_Q4_K, true, true, true, true, 16, 0, 1.0},     {HH_TYPE_Q6_K, true, false, true, false, 2, 0, 1.5},
+    {HH_TYPE_IQ2_XXS, true, false, true, false, 2, 6144, 1.0}, {HH_TYPE_IQ3_XXS, true, false, true, false, 2, 4096, 1.0},
+};
+static const MmgFmt* mmg_fmt(int type) {
+    for (const MmgFmt& f : kMmgFmts)
+        if (f.type == type) return &f;
+    return nullptr;
+}
+
+// How a product of b tokens runs: tokens per MFMA tile (16: hi and lo as rows of one tile),
+// tiles per workgroup, and the split of the columns.
+struct MmgPlan {
+    const char* mode;
+    size_t rows, tt, tiles, ttiles, groups, nch, cpk, kc, stage, tile_bytes, smem;
+};
+static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus) {
+    MmgPlan p{};
+    const size_t pad2 = (b + 63) / 64 * 64, pad1 = (b + 31) / 32 * 32;
+    double us;  // of one chunk of one workgroup beside the others of its CU
+    if (b <= 16) {
+        p.mode = "s16", p.rows = 16, p.tt = 1, us = 0.7;
+    } else if ((double)pad1 * 1.2 <= (double)pad2) {
+        p.mode = "h1", p.rows = 32, p.tt = 1, us = 1.3;
+    } else {
+        p.mode = "h2", p.rows = 32, p.tt = 2, us = 2.2;
+    }
+    us *= f->work;
+    p.ttiles = (b + p.rows * p.tt - 1) / (p.rows * p.tt);
+    p.tiles = p.ttiles * p.tt;
+    p.groups = gu ? (m + 127) / 128 : (m + 255) / 256;
+    p.nch = (n + 127) / 128;
+    const size_t chunk = (p.rows == 16 ? 8 : 16) * 1024, sums = f->mins ? 1024 : 0;
+    p.tile_bytes = p.nch * chunk + p.nch / 2 * sums;
+    p.smem = 2 * p.tt * (chunk + sums) + f->tab_bytes;
+    // splits: rounds of two workgroups per CU against the sums' traffic (8 bytes per output and
+    // split at about 3 TB/s, and a launch)
+    const size_t step = f->super ? 2 : 1, slots = 2 * cus;
+    double best = 1e300;
+    for (size_t kc = 1; kc <= std::min<size_t>(p.nch / step, 64); kc++) {
+        size_t cpk = (p.nch + kc - 1) / kc;
+        cpk = (cpk + step - 1) / step * step;
+        const size_t real = (p.nch + cpk - 1) / cpk;
+        if (real != kc) continue;
+        const size_t wgs = p.groups * p.ttiles * kc, rounds = (wgs + slots - 1) / slots;
+        double cost = (double)rounds * ((double)cpk * us + 3.0);
+        if (kc > 1) cost += 3.0 + (double)(kc * b * m * (gu ? 2 : 1)) * 8.0 / 3e6;
+        if (cost < best) {
+            best = cost;
+            p.kc = kc;
+            p.cpk = cpk;
+        }
+    }
+    return p;
+}
+
+bool hh_engine::mmg_ok(int type, size_t m, size_t n, const void* w) const {
+    const MmgFmt* f = mmg_fmt(type);
+    const Format* g = format_of(type);
+    // rows no wider than the one-token kernels take, so that what they refuse stays refused
+    return mmg && f && g && m >= 1 && n >= 32 && n % g->block == 0 && m <= UINT32_MAX / 2 && n <= UINT32_MAX / 2 &&
+           pick_team(n / g->unit) && ((uintptr_t)w & (f->align - 1)) == 0;
+}
+
+// The workspaces of products (types, ms, ns, gate/up) over b tokens, in turn on one stream.
+hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus,
+                              int count) {
+    size_t s = 0, pb = 0;
+    for (int i = 0; i < count; i++) {
+        const MmgPlan p = plan_mmg(mmg_fmt(types[i]), gus[i], ms[i], ns[i], b, (size_t)props.multiProcessorCount);
+        s = std::max(s, p.tiles * p.tile_bytes);
+        if (p.kc > 1) pb = std::max(pb, p.kc * b * ms[i] * (gus[i] ? 2 : 1) * sizeof(float));
+    }
+    hh_status st = grow(&ws_mg_s, &ws_mg_s_cap, s);
+    if (st == HH_OK && pb) st = grow(&ws_mg_p, &ws_mg_p_cap, pb);
+    if (st == HH_OK) st = grow(&ws_mg_f, &ws_mg_f_cap, 2 * (kMmgMaxTokens + 64) * sizeof(float));
+    return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
+}
+
+hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b) {
+    const MmgFmt* f = mmg_fmt(type);
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
+    float* up = (float*)ws_mg_f;
+    float* down = up + kMmgMaxTokens + 64;
+    hipFunction_t fn;
+    HH_TRY(kernel("hh_mmg_amax", &fn));
+    HH_TRY(launch(fn, (uint32_t)b, 256, MmgAmaxArgs{x, up, down, (uint32_t)n, 0}));
+    HH_TRY(kernel("hh_mmg_conv", &fn));
+    return launch(fn, (uint32_t)(p.tiles * p.nch), 256,
+                  MmgConvArgs{x, (uint8_t*)ws_mg_s, up, p.tile_bytes, (uint32_t)b, (uint32_t)n, (uint32_t)p.nch,
+                              (uint32_t)p.rows, f->mins, f->half_major, f->paired, 0});
+}
+
+hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b,
+                                 float* y, int act) {
+    const MmgFmt* f = mmg_fmt(type);
+    const bool gu = w1 != nullptr;
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
+    size_t rb;
+    HH_TRY(row_bytes(type, n, &rb));
+    hipFunction_t fn;
+    HH_TRY(kernel(std::string("hh_mmg_") + format_of(type)->name + "_" + p.mode + (gu ? "_gu" : ""), &fn));
+    MmgArgs a{};
+    a.w0 = w0;
+    a.w1 = gu ? w1 : w0;
+    a.xs = (const uint8_t*)ws_mg_s;
+    a.down = (const float*)ws_mg_f + kMmgMaxTokens + 64;
+    a.y = p.kc > 1 ? (float*)ws_mg_p : y;
+    a.row_bytes = rb;
+    a.tile_bytes = p.tile_bytes;
+    a.part_stride = b * m * (gu ? 2 : 1);
+    a.up_stride = gu ? b * m : 0;
+    a.m = (uint32_t)m;
+    a.n = (uint32_t)n;
+    a.b = (uint32_t)b;
+    a.nch = (uint32_t)p.nch;
+    a.cpk = (uint32_t)p.cpk;
+    a.kc = (uint32_t)p.kc;
+    a.groups = (uint32_t)p.groups;
+    a.ttiles = (uint32_t)p.ttiles;
+    a.act = act;
+    const size_t units = (p.groups * p.kc + 7) / 8 * 8;
+    void* params[] = {&a};
+    HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)(units * p.ttiles), 1, 1, 256, 1, 1, (unsigned)p.smem, stream, params,
+                                     nullptr),
+               "hipModuleLaunchKernel(mmg)");
+    if (p.kc == 1) return HH_OK;
+    HH_TRY(kernel(gu ? "hh_mmg_sum_act" : "hh_mmg_sum", &fn));
+    const size_t count = b * m;
+    return launch(fn, (uint32_t)((count + 255) / 256), 256,
+                  MmgSumArgs{(const float*)ws_mg_p, y, a.part_stride, a.up_stride, count, (uint32_t)p.kc, act});
+}
+
+hh_status hh_engine::enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b,
+                                      float* y) {
+    if (b < kMmgMinTokens || !mmg_ok(type, m, n, w)) return HH_ERR_UNSUPPORTED_DEVICE;
+    const bool gu = false;
+    for (size_t nb : {std::min(b, kMmgMaxTokens), b % kMmgMaxTokens})  // a full pass and the last
+        if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1));
+    for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
+        const size_t nb = std::min(kMmgMaxTokens, b - b0);
+        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb));
+        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0));
+    }
+    return HH_OK;
+}
+
+hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y) {
+    const size_t dm = d->d_model, df = d->d_ff;
+    const uint8_t* wg = pack + d->gate_off;
+    const uint8_t* wu = pack + d->up_off;
+    const uint8_t* wd = pack + d->down_off;
+    if (b < (small_ffn_shape(d) ? kMmgMinTokensSmallFfn : kMmgMinTokens) || d->type_gate != d->type_up || !mmg_ok(d->type_gate, df, dm, wg) ||
+        !mmg_ok(d->type_up, df, dm, wu) || !mmg_ok(d->type_down, dm, df, wd))
+        return HH_ERR_UNSUPPORTED_DEVICE;
+    const int types[] = {d->type_gate, d->type_down};
+    const size_t ms[] = {df, dm}, ns[] = {dm, df};
+    const bool gus[] = {true, false};
+    const size_t most = std::min(b, kMmgMaxTokens);
+    for (size_t nb : {most, b % kMmgMaxTokens})  // a full pass and the last
+        if (nb) HH_TRY(mmg_grow(nb, types, ms, ns, gus, 2));
+    const hh_status st = grow(&ws_mg_h, &ws_mg_h_cap, most * df * sizeof(float));
+    if (st != HH_OK) return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
+    for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
+        const size_t nb = std::min(kMmgMaxTokens, b - b0);
+        float* h = (float*)ws_mg_h;
+        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb));
+        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act));
+        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb));
+        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0));
+    }
+    ffn_stage_valid = false;
+    ffn_calls += 3 * b;
+    return HH_OK;
+}
+
 hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t batch,
                                           float* y) {
     if (batch == 0) return HH_OK;
     const bool mfma = type == HH_TYPE_Q4_K && batch >= 2 && !q4k_generic && ((uintptr_t)w & 15u) == 0 &&
                       ((uintptr_t)x & 15u) == 0 && m <= 0xFFFFFFFFu && n <= 0xFFFFFFFFu;
     if (!mfma) {
+        if (type != HH_TYPE_Q4_K) {
+            const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y);
+            if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+        }
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_gemv(type, m, n, w, x + b * n, y + b * m));
         return HH_OK;
     }
@@ -1162,6 +1399,10 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
                       batch >= 4 && batch <= kMmrMaxTokens && df % 512 == 0 && !capturing &&
                       mmr_ok(df, dm, batch, wg, wg, x) && mmr_ok(df, dm, batch, wu, wu, x) &&
                       (((uintptr_t)wd | (uintptr_t)x) & 15u) == 0;
+    if (!mfma && !(d->type_gate == HH_TYPE_Q4_K && d->type_up == HH_TYPE_Q4_K && d->type_down == HH_TYPE_Q4_K)) {
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
     if (q4km) {
         HH_TRY(grow(&ws_g, &ws_g_cap, batch * df * sizeof(float)));
         HH_TRY(grow(&ws_u, &ws_u_cap, batch * df * sizeof(float)));
@@ -1492,6 +1733,11 @@ static std::vector<std::string> required_kernels() {
         for (const char* f : {"_d2_w", "_d4_w", "_d2_r", "_d4_r"}) k.push_back("hh_q4k_mmi_t" + std::to_string(t) + f);
     for (const char* f : {"t1_d2_w", "t1_d2_r", "t2_d2_w", "t2_d2_r", "t4_d2_w", "t4_d2_r"})
         k.push_back(std::string("hh_q4k_mmi_gu_") + f);
+    for (const char* f : {"hh_mmg_amax", "hh_mmg_conv", "hh_mmg_sum", "hh_mmg_sum_act"}) k.push_back(f);
+    for (const MmgFmt& f : kMmgFmts)
+        for (const char* mode : {"s16", "h1", "h2"})
+            for (const char* gu : {"", "_gu"})
+                k.push_back(std::string("hh_mmg_") + format_of(f.type)->name + "_" + mode + gu);
     k.push_back("hh_lut_gemv");
     for (const char* f : {"gu_ring_g1", "gu_ring_g2", "gu_ring_g1_n", "gu_ring_g2_n", "dn_ring_d1", "dn_ring_d2", "dn_ring_d4", "dn_ring_d8"})
         k.push_back(std::string("hh_q4k_") + f);
@@ -1581,6 +1827,7 @@ hh_status engine_create(int device, hh_engine** out) {
     if (const char* f = getenv("HAYAI_HIP_RING_GU_PER_CU")) e->ring_gu_per_cu = std::max(1, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_RING_DN_PER_CU")) e->ring_dn_per_cu = std::max(1, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMR")) e->mmr = atoi(f) != 0;
+    if (const char* f = getenv("HAYAI_HIP_MMG")) e->mmg = atoi(f) != 0;
     if (const char* f = getenv("HAYAI_HIP_MMI_MIN")) e->mmi_min = (size_t)std::max(2, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_D")) e->mmi_d = atoi(f);
     err = hipMalloc(&e->grid_sync, kBarBytes);
@@ -1598,7 +1845,7 @@ void engine_destroy(hh_engine* e) {
     if (e->copy_stream) (void)hipStreamSynchronize(e->copy_stream);
     if (e->copy_stream2) (void)hipStreamSynchronize(e->copy_stream2);
     for (void* p : {e->ws_x, e->ws_y, e->ws_h, e->ws_g, e->ws_u, e->ws_w, e->ws_hq, e->ws_xop, e->ws_hop, e->ws_part,
-                    e->ws_cnt, e->ws_moe_h, e->ws_moe_ids, e->ws_moe_w, e->ws_moe_hx, e->ws_xn, e->ws_f, e->ws_xq, e->ws_moe_yp, e->ws_moe_grp, e->ws_moe_q, e->ws_stk, e->grid_sync})
+                    e->ws_mg_s, e->ws_mg_h, e->ws_mg_p, e->ws_mg_f, e->ws_cnt, e->ws_moe_h, e->ws_moe_ids, e->ws_moe_w, e->ws_moe_hx, e->ws_xn, e->ws_f, e->ws_xq, e->ws_moe_yp, e->ws_moe_grp, e->ws_moe_q, e->ws_stk, e->grid_sync})
         if (p) (void)hipFree(p);
     for (void* p : e->ws_retired) (void)hipFree(p);
     if (e->stream) (void)hipStreamDestroy(e->stream);

@@ -129,6 +129,16 @@ struct hh_engine {
     size_t ws_part_cap = 0;
     void* ws_cnt = nullptr;  // zeroed when allocated; every launch leaves it zero
     size_t ws_cnt_cap = 0;
+    // Many-token path of every format (mmg.hip): token stages, the FFN intermediate, split
+    // sums, per-token scaling factors.
+    void* ws_mg_s = nullptr;
+    size_t ws_mg_s_cap = 0;
+    void* ws_mg_h = nullptr;
+    size_t ws_mg_h_cap = 0;
+    void* ws_mg_p = nullptr;
+    size_t ws_mg_p_cap = 0;
+    void* ws_mg_f = nullptr;
+    size_t ws_mg_f_cap = 0;
     // MoE: expert intermediates [T][k][d_ff], ids and weights of hh_moe_dev.
     void* ws_moe_h = nullptr;
     size_t ws_moe_h_cap = 0;
@@ -158,6 +168,7 @@ struct hh_engine {
     int ring_dn_per_cu = 1;     // HAYAI_HIP_RING_DN_PER_CU: ring down workgroups per CU
     bool mmr = true;            // HAYAI_HIP_MMR=0: batched Q4_K (<= 16 tokens) one token at a time
     bool mmq = true;            // HAYAI_HIP_MMQ=0: batched Q4_K (>= 17 tokens) one token at a time, no int8
+    bool mmg = true;            // HAYAI_HIP_MMG=0: other formats' batches one token at a time
     size_t mmi_min = 17;        // HAYAI_HIP_MMI_MIN: fewest tokens per pass on the int8 kernels (>= 2)
     int mmi_d = 0;              // HAYAI_HIP_MMI_D: ring depth of the int8 f16-MFMA kernels (0: chosen)
     int blocks_per_cu_override = 0;  // HAYAI_HIP_BLOCKS_PER_CU
@@ -200,6 +211,7 @@ struct hh_engine {
     hh_status enqueue_gateup(int type_g, int type_u, size_t d_ff, size_t d_model, const uint8_t* wg,
                              const uint8_t* wu, const float* x, float* h, int act, float* gu_ws = nullptr);
     hh_status enqueue_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, float* y);
+    bool small_ffn_shape(const hh_ffn_desc* d) const;  // the layer fits the one-launch FFN
     hh_status enqueue_small_ffn(const hh_ffn_desc* d, const uint8_t* wg, const uint8_t* wu, const uint8_t* wd,
                                 const float* x, float* y);
     hh_status enqueue_ffn_block(const hh_ffn_desc* d, const uint8_t* pack, const float* x, const float* norm,
@@ -237,12 +249,14 @@ struct hh_engine {
     hh_status enqueue_ring_gemv(int type, size_t m, size_t n, const uint8_t* w, const float* x, float* y,
                                 void* xq_ws = nullptr);
     // Batched GEMV Y[b][m] = W . X[b] (x, y device pointers, row-major by token).  Q4_K with
-    // 2 <= batch uses the MFMA kernels in chunks of up to 64 tokens; other formats (and
-    // batch 1) run one GEMV per token, as the reference's orchestrator does
+    // 2 <= batch uses the MFMA kernels in chunks of up to 64 tokens; the other quantized
+    // formats run on the matrix cores from 4 tokens on (mmg.hip, passes of up to 1024);
+    // fewer tokens and F32 / F16 run one GEMV per token, as the reference's orchestrator does
     // (orchestrator.rs:258-260).
     hh_status enqueue_gemv_batched(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t batch,
                                    float* y);
-    // Batched FFN: per token y[b] = FFN(x[b]); all-Q4_K FFNs run gate/up and down on MFMA.
+    // Batched FFN: per token y[b] = FFN(x[b]); all-Q4_K FFNs run gate/up and down on the Q4_K
+    // MFMA kernels, other layers of one gate/up format on mmg.hip's.
     hh_status enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t batch, float* y);
     // Tokens [b][n] f32 -> operand stages in ws_xop for 16 * tt token slots.
     hh_status enqueue_mm_prep(const float* x, size_t b, size_t n, size_t tt);
@@ -262,6 +276,17 @@ struct hh_engine {
                               size_t b, float* y, void* hs, int act, size_t tiles = 0);
     hh_status enqueue_q4k_mmr(int kind, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, const void* x,
                               size_t b, float* y, int act);
+    // Many tokens on the matrix cores, any format (mmg.hip).  HH_ERR_UNSUPPORTED_DEVICE (before
+    // any launch) when shape, type or alignment does not fit or the workspaces cannot be had.
+    bool mmg_ok(int type, size_t m, size_t n, const void* w) const;
+    hh_status mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus, int count);
+    // x [b][n] -> stages of `type`'s order, with the factors of each token
+    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b);
+    // the product of the staged tokens: GEMM (w1 null) into y [b][m], or gate/up + act into y
+    hh_status mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b, float* y,
+                          int act);
+    hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y);
+    hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y);
     // MoE routing of T tokens (device pointers) and the grouped expert FFN.
     hh_status enqueue_moe_route(const hh_moe_desc* d, const float* logits, const float* bias, size_t T,
                                 int32_t* ids, float* wts);

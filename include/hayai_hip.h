@@ -172,7 +172,9 @@ void hh_pending_destroy(hh_pending* p);
  * type, as execute_quant_gemv_batched does (crates/hayai-core/src/orchestrator.rs:240-269):
  * outputs[b*m + r] = W[r] . inputs[b*n .. b*n+n) for b < batch.  Host weights and
  * activations, blocking.  Q4_K with batch >= 2 runs on the matrix cores in passes of up to
- * 64 tokens; other types loop over tokens.  Precision of the Q4_K passes:
+ * 64 tokens; the other quantized types with batch >= 4 in passes of up to 1024 tokens at f32
+ * accuracy (measured within 4e-7 of the 64-bit product); F32 and F16 loop over tokens.
+ * Precision of the Q4_K passes:
  *   - passes of 2..16 tokens: f32 activations (as f16 hi + lo pairs), f32 accumulation:
  *     within ~1e-6 of the f32 product;
  *   - passes of 17..64 tokens: each token's activations are first quantized to int8 per
@@ -290,8 +292,9 @@ hh_status hh_ffn_block_stack_dev(hh_engine* e, const hh_ffn_desc* d, const hh_bu
  * precision hh_gemv_batched states: passes of 17..64 tokens quantize x, and then h, to
  * int8 per 32-element block, which moves the FFN output by 3-13% of max|y| per token on
  * N(0,1) inputs (h is heavy-tailed; the tests bound it at 25%); passes of 2..16 tokens stay
- * within 1e-3 of the f32 FFN (h enters down as f16).  Other formats run the single-token op
- * per token.  _dev: device buffers, enqueue only; without: host x / y, blocking. */
+ * within 1e-3 of the f32 FFN (h enters down as f16).  Other layers of quantized types (gate
+ * and up alike) run gate/up(+act) and down on the matrix cores at f32 accuracy from 4 or 5
+ * tokens on; what is left runs the single-token op per token.  _dev: device buffers, enqueue only; without: host x / y, blocking. */
 hh_status hh_ffn_batched_dev(hh_engine* e, const hh_ffn_desc* d, const hh_buf* pack, size_t pack_off,
                              const hh_buf* x, size_t x_off, size_t batch, hh_buf* y, size_t y_off);
 hh_status hh_ffn_batched(hh_engine* e, const hh_ffn_desc* d, const hh_buf* pack, size_t pack_off,

@@ -1,0 +1,112 @@
+"""Many tokens through one matrix on the matrix cores, every quantized format (mmg.hip).
+
+Held to a 64-bit product of the oracle's dequantized weights.  Bound per output, with
+S = sum |w| |x|: the two-f16 split of x leaves at most 2^-22 of each |x|, and every f32
+addition of the matrix cores (n / 16 steps, hi and lo) and of the running sum (at most n / 32)
+at most 2^-23 of S.
+"""
+import numpy as np
+import pytest
+
+import hayai_amd
+import oracle
+from hayai_amd import synth
+
+pytestmark = pytest.mark.gpu
+Q4_0, Q8_0, Q4_K, Q6_K, IQ2, IQ3 = 2, 8, 12, 14, 16, 18
+FORMATS = [Q4_0, Q8_0, Q6_K, IQ2, IQ3]
+
+
+def check(t, m, n, w, X, Y):
+    W = oracle.dequant(t, w, m * n).reshape(m, n).astype(np.float64)
+    X = X.astype(np.float64)
+    bound = (np.abs(X) @ np.abs(W).T) * (2.0 ** -22 + (n / 8 + n / 32) * 2.0 ** -23) + 1e-300
+    worst = float(np.max(np.abs(Y - X @ W.T) / bound))
+    print(f"  worst error / bound {worst:.3e}", flush=True)
+    assert np.isfinite(Y).all() and worst <= 1.0
+
+
+# rows and tokens around the tiles (256 rows a workgroup, 64 a wave; 16, 32 and 64 tokens),
+# columns of one block, odd block counts, a partial 128-column chunk, and split columns
+SHAPES = [(1, 256, 4), (33, 256, 16), (255, 768, 17), (257, 512, 32), (300, 1280, 33), (64, 2048, 64),
+          (1000, 256, 65), (512, 2304, 97), (100, 14336, 5)]
+
+
+@pytest.mark.parametrize("m,n,batch", SHAPES)
+@pytest.mark.parametrize("t", FORMATS)
+def test_products(engine, t, m, n, batch):
+    print(f"[case] many tokens type={t} m={m} n={n} batch={batch}", flush=True)
+    w = synth.matrix(t, m, n, synth.seed_for(51, batch, t))
+    X = synth.normal(synth.seed_for(51, n, m), batch * n).reshape(batch, n)
+    Y = engine.ggml_gemv_batched(t, m, n, w, X, batch).reshape(batch, m)
+    check(t, m, n, w, X, Y)
+
+
+@pytest.mark.parametrize("n", [32, 96, 576, 1056])
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+def test_short_blocks_end_inside_a_chunk(engine, t, n):
+    print(f"[case] many tokens type={t} n={n}", flush=True)
+    m, batch = 70, 21
+    w = synth.matrix(t, m, n, 52)
+    X = synth.normal(53, batch * n).reshape(batch, n)
+    check(t, m, n, w, X, engine.ggml_gemv_batched(t, m, n, w, X, batch).reshape(batch, m))
+
+
+@pytest.mark.parametrize("t", FORMATS)
+def test_tokens_of_any_size(engine, t):
+    # each token has its own power of two: tiny, huge, zero and mixed tokens do not disturb
+    # one another, and an infinite one only itself
+    print(f"[case] token sizes type={t}", flush=True)
+    m, n = 96, 512
+    w = synth.matrix(t, m, n, 54)
+    X = synth.normal(55, 6 * n).reshape(6, n)
+    X[0] *= np.float32(1e-30)
+    X[1] *= np.float32(1e30)
+    X[2] = 0
+    X[3, ::2] *= np.float32(1e-6)
+    X[4, 7] = np.inf
+    Y = engine.ggml_gemv_batched(t, m, n, w, X, 6).reshape(6, m)
+    fine = [0, 1, 2, 3, 5]
+    check(t, m, n, w, X[fine], Y[fine])
+    assert not np.isfinite(Y[4]).any()
+
+
+def make_pack(engine, types, d_model, d_ff, cfg):
+    shapes = [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]
+    mats = [hayai_amd.QuantMatrix("m", c, r, t) for t, (r, c) in zip(types, shapes)]
+    lay = hayai_amd.LayerPackLayout.ffn_only(*mats)
+    ws = [synth.matrix(t, r, c, synth.seed_for(cfg, 0, i)) for i, (t, (r, c)) in enumerate(zip(types, shapes))]
+    pack = engine.alloc(lay.total)
+    for w, off in zip(ws, (lay.gate_off, lay.up_off, lay.down_off)):
+        pack.write(w, off)
+    return lay, ws, pack
+
+
+@pytest.mark.parametrize("types,d_model,d_ff,batch,act", [
+    ((Q4_0,) * 3, 576, 1536, 5, 0), ((Q8_0,) * 3, 96, 160, 40, 0), ((Q6_K,) * 3, 768, 1280, 33, 1),
+    ((Q4_K, Q4_K, Q6_K), 512, 1536, 70, 0), ((IQ2,) * 3, 512, 768, 16, 0), ((IQ3, IQ3, Q8_0), 256, 512, 17, 0),
+    ((Q4_K, Q4_K, Q6_K), 256, 512, 1029, 0),  # more than one pass, the last of five tokens
+])
+def test_ffn(engine, types, d_model, d_ff, batch, act):
+    print(f"[case] many tokens ffn {types} {d_model}x{d_ff} batch={batch}", flush=True)
+    lay, ws, pack = make_pack(engine, types, d_model, d_ff, 56)
+    desc = engine.ffn_desc(types, d_model, d_ff, lay, act)
+    X = synth.normal(57, batch * d_model).reshape(batch, d_model)
+    Y = engine.ffn_batched(desc, pack, 0, X)
+    for b in list(range(min(batch, 40))) + list(range(max(40, batch - 8), batch)):
+        ref = oracle.ffn(types, d_model, d_ff, *ws, X[b], act=act)
+        # the oracle sums in f32 itself; both are within 1e-5 of max |y| at these widths
+        assert np.max(np.abs(Y[b] - ref)) <= 2e-5 * np.max(np.abs(ref)), b
+
+
+def test_in_place_and_unaligned_activations(engine):
+    # x read and y written at 4-byte offsets, and y over x
+    t, d_model, d_ff, batch = Q8_0, 160, 96, 9
+    lay, ws, pack = make_pack(engine, (t,) * 3, d_model, d_ff, 58)
+    desc = engine.ffn_desc((t,) * 3, d_model, d_ff, lay)
+    X = synth.normal(59, batch * d_model).reshape(batch, d_model)
+    want = engine.ffn_batched(desc, pack, 0, X)
+    buf = engine.alloc(4 + X.nbytes)
+    buf.write(X, 4)
+    engine.ffn_batched_dev(desc, pack, 0, buf, 4, batch, buf, 4)
+    np.testing.assert_array_equal(buf.read(np.float32, X.size, 4).reshape(X.shape), want)
