@@ -1,5 +1,6 @@
 // Many tokens through one weight matrix on the matrix cores, every GGUF format (gfx950):
-//   hh_mmg_amax                 per token the power of two that its f16 operands are scaled by
+//   hh_mmg_amax                 per token its largest magnitude, which its f16 operands' power of
+//                               two is made of (h's is collected by gate/up as it stores h)
 //   hh_mmg_conv                 tokens [b][n] f32 -> token stages (below)
 //   hh_mmg_<fmt>_<mode>         Y[t][r] = W[r] . X[t] (execute_quant_gemv_batched, crates/
 //                               hayai-core/src/orchestrator.rs:240-269)
@@ -38,18 +39,25 @@
 // one token at a time these took 12 .. 39 ms); at 4..16 tokens the weight stream's latency (8B
 // Q6_K FFN, 16 tokens: 106 us against 779 us).
 //
+// MoE (hh_mmg_moe_*): the (token, slot) pairs of an expert in tiles of 16 or 32, one launch over
+// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 259 us a layer.
+//
 // Token stages: [tile][128-column chunk][group 0..3][step 0..1][hi, lo][lane][8 f16], for Q4_K
 // followed after every second chunk by the sums [lane][8 f16] (lane half 0: hi of sub-blocks
 // 0..7, half 1: lo).
 typedef float hh_f16v __attribute__((ext_vector_type(16)));
 
+#ifndef HH_MMG_VALU
+#define HH_MMG_VALU 0
+#endif
 enum { HH_MMG_H = 0, HH_MMG_S16 = 1 };
 
 struct hh_mmg_args {
     const uint8_t* w0;       // GEMM: W; gate/up: W_gate
     const uint8_t* w1;       // GEMM: W; gate/up: W_up
     const uint8_t* xs;       // token stages
-    const float* down;       // per token: the power of two that undoes its scaling
+    const float* amax;       // per token: what its scaling was made of
+    float* pmax;             // gate/up: [row group][ldt] the group's largest magnitude of each token's h
     float* y;                // kc == 1: Y [b][m] or h [b][m]; else the splits' sums
     uint64_t row_bytes;
     uint64_t tile_bytes;     // stage bytes of one token tile
@@ -62,7 +70,11 @@ struct hh_mmg_args {
     uint32_t groups;         // row groups
     uint32_t ttiles;         // token tile groups
     int32_t act;
-    uint32_t pad;
+    uint32_t ldt;
+    // MoE: tiles of one expert's pairs (hh_mmg_moe_args); w0 / w1 are expert 0's matrices
+    const int4* trec;
+    const int32_t* order;
+    uint64_t expert_stride;
 };
 
 // Bytes at any address (2-byte aligned in GGUF formats): the hardware takes unaligned loads.
@@ -90,6 +102,19 @@ HH_DEV hh_h2 hh_bytes_h2(uint32_t v) {
     return hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, v, I | (4u << 8) | (J << 16) | (4u << 24)));
 }
 
+// Masks and exponent bits of the decodes, held in registers: a gfx9 VOP3 instruction takes no
+// literal, so only so is (v & mask) | bits one v_and_or_b32.
+struct hh_mmg_k {
+    uint32_t lo, hi, magic;  // 0x000F000F, 0x00F000F0 (scalar), 0x64006400 (vector)
+    uint32_t b30;            // 0x30303030 (scalar)
+    HH_DEV void set() {
+        asm volatile("s_mov_b32 %0, 0x000F000F" : "=s"(lo));
+        asm volatile("s_mov_b32 %0, 0x00F000F0" : "=s"(hi));
+        asm volatile("s_mov_b32 %0, 0x30303030" : "=s"(b30));
+        asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+    }
+};
+
 // ---- weight formats -------------------------------------------------------------------
 // Raw: one chunk's bytes of one row as loaded; load(p, ch, ...) of chunk ch of the row at p
 // (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
@@ -113,15 +138,15 @@ struct hh_mmg_q4_0 {
     }
     HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
         const uint32_t v[4] = {r.q[g].x, r.q[g].x >> 8, r.q[g].y, r.q[g].y >> 8};
         hh_h2 o[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             if (s == 0)  // 1024 + q, q - 8
-                o[i] = hh_h2_bits((v[i] & 0x000F000Fu) | 0x64006400u) - hh_h2_all(1032.f);
+                o[i] = hh_h2_bits((v[i] & k.lo) | k.magic) - hh_h2_all(1032.f);
             else  // 1024 + 16 q, q - 8 (exact: the FMA rounds only its result)
-                o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & 0x00F000F0u) | 0x64006400u), hh_h2_all(0.0625f),
+                o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & k.hi) | k.magic), hh_h2_all(0.0625f),
                                                  hh_h2_all(-72.f));
         }
         f[0] = hh_h8_of(o[0], o[1], o[2], o[3]);
@@ -147,7 +172,7 @@ struct hh_mmg_q8_0 {
     }
     HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
         const uint32_t a = (s ? r.q[g].z : r.q[g].x) ^ 0x80808080u, b = (s ? r.q[g].w : r.q[g].y) ^ 0x80808080u;
         const hh_h2 z = hh_h2_all(1152.f);  // 1024 + (q + 128)
         f[0] = hh_h8_of(hh_bytes_h2<0, 1>(a) - z, hh_bytes_h2<2, 3>(a) - z, hh_bytes_h2<0, 1>(b) - z,
@@ -179,7 +204,7 @@ struct hh_mmg_q4_k {
                         hh_bytes_h2<2, 3>(hi) - z);
     }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
         // the chunk's four sub-block scales; sub-blocks 2p (low nibbles) and 2p + 1 (high) of
         // the 32 qs bytes p
         const uint32_t sch =
@@ -191,11 +216,11 @@ struct hh_mmg_q4_k {
         const hh_h2 sc = hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, sch, sel)) - hh_h2_all(1024.f);
         const hh_h2 mul = (g & 1) ? sc * hh_h2_all(0.0625f) : sc;
         const hh_h2 off = mul * hh_h2_all(-1024.f);
-        const uint32_t mask = (g & 1) ? 0x00F000F0u : 0x000F000Fu;
+        const uint32_t mask = (g & 1) ? k.hi : k.lo;
         hh_h2 o[4];
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & mask) | 0x64006400u), mul, off);
+            o[i] = __builtin_elementwise_fma(hh_h2_bits((v[i] & mask) | k.magic), mul, off);
         f[0] = hh_h8_of(o[0], o[1], o[2], o[3]);
     }
 };
@@ -220,15 +245,18 @@ struct hh_mmg_q6_k {
     }
     HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d); }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char*, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char*, const hh_mmg_k& k, hh_h8* f) {
         const uint4 l = (g & 1) ? r.b : r.a;
         const uint32_t la = s ? l.z : l.x, lb = s ? l.w : l.y, ha = s ? r.qh.z : r.qh.x, hb = s ? r.qh.w : r.qh.y;
         // scale byte 2 g + h of the chunk's eight
         const uint32_t sw = (g & 2) ? r.sc.y : r.sc.x;
         const float scf = (float)(int8_t)(sw >> (16 * (g & 1) + 8 * h));
         const hh_h2 sc = hh_h2_all(scf);
-        const uint32_t q[2] = {((g & 2) ? (la >> 4) & 0x0F0F0F0Fu : la & 0x0F0F0F0Fu) | (((ha >> (2 * g)) & 0x03030303u) << 4),
-                               ((g & 2) ? (lb >> 4) & 0x0F0F0F0Fu : lb & 0x0F0F0F0Fu) | (((hb >> (2 * g)) & 0x03030303u) << 4)};
+        // bits 2 g, 2 g + 1 of each qh byte to bits 4, 5
+        const uint32_t ta = g == 0 ? ha << 4 : g == 1 ? ha << 2 : g == 2 ? ha : ha >> 2;
+        const uint32_t tb = g == 0 ? hb << 4 : g == 1 ? hb << 2 : g == 2 ? hb : hb >> 2;
+        const uint32_t q[2] = {(ta & k.b30) | (((g & 2) ? la >> 4 : la) & 0x0F0F0F0Fu),
+                               (tb & k.b30) | (((g & 2) ? lb >> 4 : lb) & 0x0F0F0F0Fu)};
         hh_h2 hi[4], lo[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -307,7 +335,7 @@ struct hh_mmg_iq2_xxs {
     // d * (0.5 + s) * 0.25 = d / 8 * (2 s + 1)
     HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d) * 0.125f; }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, const hh_mmg_k&, hh_h8* f) {
         const uint32_t l = 2 * h + (uint32_t)s, aux = r.q[g].y;
         const uint32_t idx = (r.q[g].x >> (8 * l)) & 0xFFu, sg = (aux >> (7 * l)) & 127u;
         f[0] = hh_mmg_iq_frag(*reinterpret_cast<const uint4*>(tab + idx * 16),
@@ -337,7 +365,7 @@ struct hh_mmg_iq3_xxs {
     // d * (0.5 + s) * 0.5 = d / 4 * (2 s + 1)
     HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.d) * 0.25f; }
     template <uint32_t HALF>
-    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, hh_h8* f) {
+    HH_DEV static void frag(const Raw& r, int g, int s, uint32_t h, const char* tab, const hh_mmg_k&, hh_h8* f) {
         const uint32_t l = 2 * h + (uint32_t)s;
         const uint32_t aux = g == 0 ? r.aux.x : g == 1 ? r.aux.y : g == 2 ? r.aux.z : r.aux.w;
         const uint32_t i0 = (r.q[g] >> (16 * s)) & 0xFFu, i1 = (r.q[g] >> (16 * s + 8)) & 0xFFu;
@@ -352,47 +380,65 @@ struct hh_mmg_iq3_xxs {
 struct hh_mmg_conv_args {
     const float* x;        // [b][n]
     uint8_t* xs;           // stages
-    const float* up;       // per token: its power of two
+    float* amax;           // per token: its largest magnitude
+    const float* pmax;     // h: gate/up's [pgroups][ldt] largest magnitudes over its row groups,
+                           // from which amax is made (and written) here; null: amax is given
     uint64_t tile_bytes;
     uint32_t b, n, nch;
     uint32_t rows;         // tokens per tile: 32, or 16 (mode s16)
     uint32_t mins;         // write the sub-block sums
     uint32_t half_major;   // column order 16 h + 8 step + e (else 16 step + 8 h + e)
     uint32_t paired;       // e in the order 0 2 1 3 4 6 5 7
+    uint32_t pgroups, ldt;
     uint32_t pad;
 };
 
 struct hh_mmg_amax_args {
     const float* x;  // [b][n]
-    float* up;
-    float* down;
+    float* amax;     // per token
     uint32_t n, pad;
 };
 
-// One workgroup per token.  amax in [2^(k-1), 2^k) -> up = 2^(10 - k): the largest magnitude
-// into [512, 1024), so that a sum of 32 elements stays below f16's largest value.  A token
-// without a finite, non-zero maximum keeps the factor 1 (its infinities stay infinities).
-extern "C" __global__ void __launch_bounds__(256) hh_mmg_amax(const hh_mmg_amax_args a) {
-    __shared__ float red[4];
-    const float* x = a.x + (size_t)blockIdx.x * a.n;
-    float v = 0.f;
-    for (uint32_t i = threadIdx.x; i < a.n; i += 256) v = fmaxf(v, fabsf(x[i]));
+// amax in [2^(k-1), 2^k) -> up = 2^(10 - k): the largest magnitude into [512, 1024), so that a
+// sum of 32 elements stays below f16's largest value.  A token without a finite, non-zero
+// maximum keeps the factor 1 (its infinities stay infinities).
+HH_DEV int hh_mmg_exp(float amax) {
+    if (!(amax > 0.f && amax < __builtin_inff())) return 0;
+    int k;
+    (void)frexpf(amax, &k);
+    return min(max(10 - k, -120), 120);
+}
+HH_DEV float hh_wave_max(float v) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// A workgroup of 256 threads: the largest magnitude of x[0, n) (NaN elements do not count).
+HH_DEV void hh_mmg_token_amax(const float* x, uint32_t n, float* amax) {
+    __shared__ float red[4];
+    float v = 0.f;
+    if ((((uintptr_t)x | n) & 3u) == 0 && ((uintptr_t)x & 15u) == 0) {
+        const float4* x4 = reinterpret_cast<const float4*>(x);
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < n / 4; i += 256) {
+            const float4 u = x4[i];
+            v = fmaxf(v, fmaxf(fmaxf(fabsf(u.x), fabsf(u.y)), fmaxf(fabsf(u.z), fabsf(u.w))));
+        }
+    } else {
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < n; i += 256) v = fmaxf(v, fabsf(x[i]));
+    }
+    v = hh_wave_max(v);
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        int e = 0;
-        if (v > 0.f && v < __builtin_inff()) {
-            int k;
-            (void)frexpf(v, &k);
-            e = min(max(10 - k, -120), 120);
-        }
-        a.up[blockIdx.x] = ldexpf(1.f, e);
-        a.down[blockIdx.x] = ldexpf(1.f, -e);
-    }
+    if (threadIdx.x == 0) *amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_amax(const hh_mmg_amax_args a) {
+    hh_mmg_token_amax(a.x + (size_t)blockIdx.x * a.n, a.n, a.amax + blockIdx.x);
+}
+HH_DEV float hh_mmg_up(float amax) { return ldexpf(1.f, hh_mmg_exp(amax)); }
+HH_DEV float hh_mmg_down(float amax) { return ldexpf(1.f, -hh_mmg_exp(amax)); }
 
 HH_DEV void hh_mmg_split(float v, _Float16& hi, _Float16& lo) {
     hi = (_Float16)v;
@@ -400,24 +446,24 @@ HH_DEV void hh_mmg_split(float v, _Float16& hi, _Float16& lo) {
     lo = (_Float16)(r == r ? r : 0.f);  // an infinite v: hi carries it alone
 }
 
-// One workgroup per (token tile, chunk); tokens past b and columns past n are zeros.
-extern "C" __global__ void __launch_bounds__(256) hh_mmg_conv(const hh_mmg_conv_args a) {
-    const uint32_t tile = blockIdx.x / a.nch, ch = blockIdx.x % a.nch;
+// One chunk of one tile, by a workgroup of `threads`.  row(tok, &src, &up): the tile's token tok
+// as its f32 row and factor, false past the tokens (zeros; columns past n are zeros too).
+template <class ROW>
+HH_DEV void hh_mmg_conv_chunk(uint8_t* tile, const hh_mmg_conv_args& a, uint32_t ch, bool vec, uint32_t threads,
+                              ROW row) {
     const bool s16 = a.rows == 16;
     const uint32_t chunk_bytes = (s16 ? 8u : 16u) * 1024u;
-    uint8_t* st = a.xs + tile * a.tile_bytes +
-                  (a.mins ? (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + (ch & 1u) * chunk_bytes
-                          : (size_t)ch * chunk_bytes);
-    const bool vec = ((uintptr_t)a.x & 15u) == 0;
-    for (uint32_t p = threadIdx.x; p < (s16 ? 256u : 512u); p += 256) {
+    uint8_t* st = tile + (a.mins ? (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + (ch & 1u) * chunk_bytes
+                                 : (size_t)ch * chunk_bytes);
+    for (uint32_t p = threadIdx.x; p < (s16 ? 256u : 512u); p += threads) {
         // piece p: group, step, lane half, token
         const uint32_t tok = p % a.rows, h = (p / a.rows) & 1u, step = (p / a.rows >> 1) & 1u, g = p / a.rows >> 2;
-        const uint32_t t = tile * a.rows + tok;
         const uint32_t col = 128 * ch + 32 * g + (a.half_major ? 16 * h + 8 * step : 16 * step + 8 * h);
         float v[8];
-        if (t < a.b && col < a.n) {
-            const float* src = a.x + (size_t)t * a.n + col;
-            const float up = a.up[t];
+        const float* src;
+        float up;
+        if (col < a.n && row(tok, src, up)) {
+            src += col;
             if (vec) {
                 const float4 u0 = reinterpret_cast<const float4*>(src)[0], u1 = reinterpret_cast<const float4*>(src)[1];
                 v[0] = u0.x, v[1] = u0.y, v[2] = u0.z, v[3] = u0.w, v[4] = u1.x, v[5] = u1.y, v[6] = u1.z, v[7] = u1.w;
@@ -455,20 +501,96 @@ extern "C" __global__ void __launch_bounds__(256) hh_mmg_conv(const hh_mmg_conv_
         }
     }
     if (!a.mins) return;
-    uint8_t* sums = a.xs + tile * a.tile_bytes + (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + 2 * chunk_bytes;
+    uint8_t* sums = tile + (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + 2 * chunk_bytes;
     const uint32_t q = threadIdx.x;  // token row, group
     if (q >= 128) return;
-    const uint32_t row = q % 32, g = q / 32, j = 4 * (ch & 1u) + g, t = tile * a.rows + row;
+    const uint32_t r = q % 32, g = q / 32, j = 4 * (ch & 1u) + g;
     float s = 0.f;
-    if (row < a.rows && t < a.b) {
-        const float* src = a.x + (size_t)t * a.n + 128 * ch + 32 * g;
-        const float up = a.up[t];
+    const float* src;
+    float up;
+    if (r < a.rows && row(r, src, up)) {
+        src += 128 * ch + 32 * g;
         for (int e = 0; e < 32; e++) s += src[e] * up;
     }
     _Float16 hi, lo;
     hh_mmg_split(s, hi, lo);
-    *reinterpret_cast<_Float16*>(sums + row * 16 + j * 2) = hi;         // s16: rows 16..31 are zeros
-    *reinterpret_cast<_Float16*>(sums + 512 + row * 16 + j * 2) = lo;
+    *reinterpret_cast<_Float16*>(sums + r * 16 + j * 2) = hi;  // s16: rows 16..31 are zeros
+    *reinterpret_cast<_Float16*>(sums + 512 + r * 16 + j * 2) = lo;
+}
+
+// The factors of a tile's rows into LDS; index(row): the row's place in amax / pmax.
+template <class IDX>
+HH_DEV void hh_mmg_ups(float* ups, const hh_mmg_conv_args& a, uint32_t count, bool store, IDX index) {
+    __shared__ float red[8][32];
+    const uint32_t row = threadIdx.x % 32, part = threadIdx.x / 32;
+    if (a.pmax) {
+        float v = 0.f;
+        if (row < count) {
+            const float* p = a.pmax + index(row);
+#pragma unroll 4
+            for (uint32_t g = part; g < a.pgroups; g += 8) v = fmaxf(v, p[(size_t)g * a.ldt]);
+        }
+        red[part][row] = v;
+        __syncthreads();
+    }
+    if (part == 0 && row < count) {
+        float v;
+        if (a.pmax) {
+            v = red[0][row];
+#pragma unroll
+            for (int k = 1; k < 8; k++) v = fmaxf(v, red[k][row]);
+            if (store) a.amax[index(row)] = v;
+        } else {
+            v = a.amax[index(row)];
+        }
+        ups[row] = hh_mmg_up(v);
+    }
+    __syncthreads();
+}
+
+// One workgroup per (token tile, chunk).
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_conv(const hh_mmg_conv_args a) {
+    __shared__ float ups[32];
+    const uint32_t tile = blockIdx.x / a.nch, ch = blockIdx.x % a.nch;
+    const uint32_t t0 = tile * a.rows, count = t0 < a.b ? min(a.rows, a.b - t0) : 0u;
+    hh_mmg_ups(ups, a, count, ch == 0, [&](uint32_t row) { return t0 + row; });
+    hh_mmg_conv_chunk(a.xs + tile * a.tile_bytes, a, ch, ((uintptr_t)a.x & 15u) == 0, 256,
+                      [&](uint32_t tok, const float*& src, float& up) {
+                          if (tok >= count) return false;
+                          src = a.x + (size_t)(t0 + tok) * a.n;
+                          up = ups[tok];
+                          return true;
+                      });
+}
+
+// MoE: tiles of one expert's (token, slot) pairs.  trec[0].x: how many; trec[1 + tile]: the
+// expert, the tile's first position in `order`, its pairs.
+struct hh_mmg_moe_args {
+    hh_mmg_conv_args c;      // x: tokens [T][n] and their amax; h: tile rows [tile][rows][n] and theirs
+    const int4* trec;
+    const int32_t* order;
+    float* amax_row;         // x: per tile row, its token's amax
+    uint32_t k, pad;         // slots per token; 0: h
+};
+// One workgroup per (tile, chunk).  x: each row is its pair's token; h: the row itself.
+extern "C" __global__ void __launch_bounds__(256) hh_mmg_moe_conv(const hh_mmg_moe_args a) {
+    __shared__ float ups[32];
+    const uint32_t tile = blockIdx.x / a.c.nch, ch = blockIdx.x % a.c.nch;
+    if (tile >= (uint32_t)a.trec[0].x) return;
+    const int4 rec = a.trec[1 + tile];
+    auto token = [&](uint32_t row) {
+        return a.k ? (uint32_t)a.order[rec.y + (int)row] / a.k : tile * a.c.rows + row;
+    };
+    hh_mmg_ups(ups, a.c, (uint32_t)rec.z, ch == 0, token);
+    hh_mmg_conv_chunk(a.c.xs + tile * a.c.tile_bytes, a.c, ch, true, 256,
+                      [&](uint32_t tok, const float*& src, float& up) {
+                          if ((int)tok >= rec.z) return false;
+                          src = a.c.x + (size_t)token(tok) * a.c.n;
+                          up = ups[tok];
+                          return true;
+                      });
+    if (a.k && ch == 0 && (int)threadIdx.x < rec.z)
+        a.amax_row[tile * a.c.rows + threadIdx.x] = a.c.amax[token(threadIdx.x)];
 }
 
 template <uint32_t V>
@@ -486,7 +608,7 @@ HH_DEV void hh_mmg_sync() {
     asm volatile("" ::: "memory");
 }
 
-template <class F, int MODE, int TT, bool GU>
+template <class F, int MODE, int TT, bool GU, bool MOE = false>
 HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     constexpr int NA = MODE == HH_MMG_H ? 2 : 1;
     constexpr uint32_t CB = 8u * NA * 1024u;            // stage bytes of a (tile, chunk)
@@ -500,9 +622,25 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     // workgroup -> (row group, split, token tiles): the token tiles of one (row group, split) sit
     // on one XCD one after another, so its weights come from memory once and from L2 after
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-    const uint32_t unit = slot / a.ttiles * 8u + xcd, tg = slot % a.ttiles;
-    if (unit >= a.groups * a.kc) return;
-    const uint32_t grp = unit / a.kc, kci = unit % a.kc;
+    uint32_t tg, grp, kci;
+    int4 rec{};
+    if constexpr (MOE) {
+        // each XCD takes a contiguous share of (tile, row group): the tiles of one expert run
+        // close together on one L2
+        const uint32_t all = (uint32_t)a.trec[0].x * a.groups, share = (all + 7u) / 8u;
+        const uint32_t i = xcd * share + slot;
+        if (slot >= share || i >= all) return;
+        tg = i / a.groups;
+        grp = i % a.groups;
+        kci = 0;
+        rec = a.trec[1 + tg];
+    } else {
+        const uint32_t unit = slot / a.ttiles * 8u + xcd;
+        tg = slot % a.ttiles;
+        if (unit >= a.groups * a.kc) return;
+        grp = unit / a.kc;
+        kci = unit % a.kc;
+    }
     const uint32_t c0 = kci * a.cpk, c1 = min(c0 + a.cpk, a.nch);
     const uint32_t nblk = a.n / 32;
 
@@ -510,8 +648,9 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     const uint8_t* wp[2];
     row[0] = GU ? grp * 128 + wave * 32 + r : grp * 256 + wave * 64 + r;
     row[1] = GU ? row[0] : row[0] + 32;
-    wp[0] = a.w0 + (size_t)min(row[0], a.m - 1) * a.row_bytes;
-    wp[1] = a.w1 + (size_t)min(row[1], a.m - 1) * a.row_bytes;
+    const size_t ex = MOE ? (size_t)rec.x * a.expert_stride : 0;
+    wp[0] = a.w0 + ex + (size_t)min(row[0], a.m - 1) * a.row_bytes;
+    wp[1] = a.w1 + ex + (size_t)min(row[1], a.m - 1) * a.row_bytes;
 
     if constexpr (F::TABLES) {
         char* tab = hh_smem + 2 * BUF;
@@ -541,6 +680,8 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         }
     };
 
+    hh_mmg_k kk;
+    kk.set();
     hh_f16v sum[2][TT], part[2][TT];
 #pragma unroll
     for (int q = 0; q < 2; q++)
@@ -561,27 +702,31 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             for (int s = 0; s < 2; s++) {
                 hh_h8 wf[2][F::NB];
 #pragma unroll
-                for (int q = 0; q < 2; q++) F::template frag<buf>(raw[q], g, s, h, tab, wf[q]);
+                for (int q = 0; q < 2; q++) F::template frag<buf>(raw[q], g, s, h, tab, kk, wf[q]);
+                const bool fresh = s == 0 && (F::SUPER ? open && g == 0 : true);
+                hh_h8 x[NA][TT];
 #pragma unroll
-                for (int tt = 0; tt < TT; tt++) {
-                    const char* p = st + tt * (CB + SUMS) + (g * 2 + s) * (NA * 1024);
-                    const hh_h8 x0 = *reinterpret_cast<const hh_h8*>(p);
-                    hh_h8 x1;
-                    if constexpr (NA == 2) x1 = *reinterpret_cast<const hh_h8*>(p + 1024);
-                    const bool fresh = s == 0 && (F::SUPER ? open && g == 0 : true);
+                for (int k = 0; k < NA; k++)
 #pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        hh_f16v c = part[q][tt];
-                        if (fresh) {
+                    for (int tt = 0; tt < TT; tt++)
+                        x[k][tt] = *reinterpret_cast<const hh_h8*>(st + tt * (CB + SUMS) + (g * 2 + s) * (NA * 1024) +
+                                                                   k * 1024);
+                // hi of every tile, then lo, then the weights' remainders: no product waits for
+                // the one before it
 #pragma unroll
-                            for (int i = 0; i < 16; i++) c[i] = 0.f;
+                for (int k = 0; k < NA + F::NB - 1; k++)
+#pragma unroll
+                    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                        for (int q = 0; q < 2; q++) {
+                            hh_f16v c = part[q][tt];
+                            if (fresh && k == 0) {
+#pragma unroll
+                                for (int i = 0; i < 16; i++) c[i] = 0.f;
+                            }
+                            part[q][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                k < NA ? x[k][tt] : x[0][tt], wf[q][k < NA ? 0 : 1], c, 0, 0, 0);
                         }
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x0, wf[q][0], c, 0, 0, 0);
-                        if constexpr (NA == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x1, wf[q][0], c, 0, 0, 0);
-                        if constexpr (F::NB == 2) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x0, wf[q][1], c, 0, 0, 0);
-                        part[q][tt] = c;
-                    }
-                }
             }
             if (!F::SUPER || (close && g == 3)) {
 #pragma unroll
@@ -615,6 +760,16 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         }
     };
 
+    // the matrix core's next operands are decoded while it works: one MFMA, then a few others
+    auto interleave = [&]() {
+        constexpr int N = 4 * 2 * 2 * TT * (NA + F::NB - 1);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, HH_MMG_VALU, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+    };
     typename F::Raw raw[2][2];  // [buffer][row tile]
     constexpr hh_uint_c<0> B0{};
     constexpr hh_uint_c<1> B1{};
@@ -631,6 +786,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             for (int q = 0; q < 2; q++) F::template load<1>(raw[1][q], wp[q], ch + 1, h, nblk);
         }
         compute(raw[0], B0);
+        if (HH_MMG_VALU) interleave();
         if (!two) break;
         hh_mmg_sync();
         if (ch + 2 < c1) {
@@ -639,22 +795,26 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], ch + 2, h, nblk);
         }
         compute(raw[1], B1);
+        if (HH_MMG_VALU) interleave();
     }
 
     // outputs: lane's weight row, tokens 8 (i / 4) + 4 h + i % 4 of each tile
     float* const out = a.y + (a.kc > 1 ? kci * a.part_stride : 0);
-    const bool fuse = GU && a.kc == 1;
+    const bool fuse = GU && (MOE || a.kc == 1);
+    float* const wmax = reinterpret_cast<float*>(hh_smem) + wave * 2 * (TT * ROWS);  // gate/up: per token
+    if (fuse) hh_mmg_sync();  // the token buffers are read
 #pragma unroll
     for (int tt = 0; tt < TT; tt++) {
 #pragma unroll
         for (int i4 = 0; i4 < (MODE == HH_MMG_S16 ? 2 : 4); i4++) {
-            const uint32_t t0 = (tg * TT + tt) * ROWS + 8 * i4 + 4 * h;
-            const float4 d4 = *reinterpret_cast<const float4*>(a.down + t0);  // padded to whole tiles
-            const float dn[4] = {d4.x, d4.y, d4.z, d4.w};
+            const uint32_t in = 8 * i4 + 4 * h, t0 = (tg * TT + tt) * ROWS + in;
+            const float4 d4 = *reinterpret_cast<const float4*>(a.amax + t0);  // padded to whole tiles
+            const float dn[4] = {hh_mmg_down(d4.x), hh_mmg_down(d4.y), hh_mmg_down(d4.z), hh_mmg_down(d4.w)};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const uint32_t t = t0 + k;
-                if (t >= a.b) continue;
+                uint32_t t = t0 + k;
+                const bool live = MOE ? (int)(in + k) < rec.z : t < a.b;
+                if constexpr (MOE && !GU) t = (uint32_t)a.order[rec.y + min((int)(in + k), rec.z - 1)];  // the pair
                 float v[2];
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
@@ -663,41 +823,73 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
                     v[q] *= dn[k];
                 }
                 if (fuse) {
-                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = hh_act_mul(v[0], v[1], a.act);
-                } else {
+                    float hv = hh_act_mul(v[0], v[1], a.act);
+                    if (live && row[0] < a.m) out[(size_t)t * a.m + row[0]] = hv;
+                    // over the wave's 32 rows (the token is the same in a lane half)
+                    // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
+                    hv = row[0] < a.m ? fabsf(hv) : 0.f;
+                    hv = fmaxf(hv, hh_dpp<0xB1>(hv));   // quad_perm [1,0,3,2]
+                    hv = fmaxf(hv, hh_dpp<0x4E>(hv));   // quad_perm [2,3,0,1]
+                    hv = fmaxf(hv, hh_dpp<0x124>(hv));  // row_ror:4
+                    hv = fmaxf(hv, hh_dpp<0x128>(hv));  // row_ror:8
+                    if ((r & 15u) == 0) wmax[(r >> 4) * (TT * ROWS) + tt * ROWS + in + k] = hv;
+                } else if (live) {
                     if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = v[0];
                     if (row[1] < a.m) out[(GU ? a.up_stride : 0) + (size_t)t * a.m + row[1]] = v[1];
                 }
             }
         }
     }
+    if (fuse) {
+        hh_mmg_sync();
+        if (tid < TT * ROWS) {
+            const float* w = reinterpret_cast<const float*>(hh_smem) + tid;
+            float v = w[0];
+#pragma unroll
+            for (int k = 1; k < 8; k++) v = fmaxf(v, w[k * (TT * ROWS)]);
+            a.pmax[(size_t)grp * a.ldt + tg * (TT * ROWS) + tid] = v;
+        }
+    }
 }
 
 struct hh_mmg_sum_args {
-    const float* part;     // [kc][count] (gate/up: gate's, then up's at up_stride)
-    float* y;              // [count]
+    const float* part;     // [kc][b][m] (gate/up: gate's, then up's at up_stride)
+    float* y;              // [b][m]
     uint64_t stride;       // floats between two splits
     uint64_t up_stride;
-    uint64_t count;        // floats (a multiple of 4)
+    float* pmax;           // sum_act: [256-row group][ldt] largest magnitudes of each token's h
+    uint32_t m;
     uint32_t kc;
     int32_t act;
+    uint32_t ldt;
 };
+// grid.y: tokens
 extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum(const hh_mmg_sum_args a) {
-    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x);
-    if (i >= a.count) return;
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= a.m) return;
+    const uint64_t i = (uint64_t)blockIdx.y * a.m + r;
     float s = 0.f;
+#pragma unroll 4
     for (uint32_t k = 0; k < a.kc; k++) s += a.part[k * a.stride + i];
     a.y[i] = s;
 }
 extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_sum_args a) {
-    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x);
-    if (i >= a.count) return;
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    const uint64_t i = (uint64_t)blockIdx.y * a.m + min(r, a.m - 1);
     float g = 0.f, u = 0.f;
+#pragma unroll 4
     for (uint32_t k = 0; k < a.kc; k++) {
         g += a.part[k * a.stride + i];
         u += a.part[k * a.stride + a.up_stride + i];
     }
-    a.y[i] = hh_act_mul(g, u, a.act);
+    const float h = hh_act_mul(g, u, a.act);
+    if (r < a.m) a.y[i] = h;
+    __shared__ float red[4];
+    const float v = hh_wave_max(r < a.m ? fabsf(h) : 0.f);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        a.pmax[(size_t)blockIdx.x * a.ldt + blockIdx.y] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 #define HH_MMG_KERNEL(FMT, NAME, MODE, TT, WPE)                                                                  \
@@ -717,3 +909,12 @@ HH_MMG_FORMAT(q4_k, 3)
 HH_MMG_FORMAT(q6_k, 3)
 HH_MMG_FORMAT(iq2_xxs, 3)
 HH_MMG_FORMAT(iq3_xxs, 3)
+#define HH_MMG_MOE(NAME, MODE, WPE)                                                                               \
+    extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_moe_##NAME(const hh_mmg_args a) {              \
+        hh_mmg_body<hh_mmg_q4_k, MODE, 1, false, true>(a);                                                      \
+    }                                                                                                           \
+    extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_moe_##NAME##_gu(const hh_mmg_args a) {         \
+        hh_mmg_body<hh_mmg_q4_k, MODE, 1, true, true>(a);                                                       \
+    }
+HH_MMG_MOE(s16, HH_MMG_S16, 3)
+HH_MMG_MOE(h1, HH_MMG_H, 3)

@@ -3,8 +3,8 @@
 // per (token, expert) pair.  Same results as the expert loop + combine of
 // crates/hayai-core/src/moe_infer.rs:342-455 (y[t] = sum over slots s of
 // w[t][s] * down_e(act(gate_e x_t) * up_e x_t), e = ids[t][s]):
-//   hh_moe_prep:         (token, slot) pairs p = t * k + s grouped by expert, in p order
-//                        within an expert, the active experts in ascending order, with one
+//   hh_moe_prep:         (token, slot) pairs p = t * k + s grouped by expert, the active
+//                        experts in ascending order, with one
 //                        record per active expert (hh_moeg_args::rec); and every token's x as
 //                        int8 digits (hh_moe_route_prep: the routing too)
 //   hh_moe_gu_grp_t<TM>: grid.y = active expert; every row of gate and up is read once and
@@ -34,6 +34,12 @@ struct hh_moeg_args {
     uint8_t* hq;             // [T * k] digit forms of h (d_ff elements)
     uint32_t T, k, d_model, d_ff, n_experts;
     int32_t act;
+    // many pairs (mmg.hip's kernels): instead of rec and xq, tiles of trows pairs of one expert
+    // (trec[0].x: how many; trec[1 + tile]: expert, first position in order, pairs) and each
+    // token's largest magnitude
+    int4* trec;
+    float* amax;
+    uint32_t trows, pad;
 };
 
 #define HH_MOEG_MAX_E 512     // experts the grouping kernel handles
@@ -65,12 +71,11 @@ HH_DEV int hh_moeg_valid(const hh_moeg_args& a, int e) { return (e < 0 || (uint3
 
 // Workgroup 0 groups the pairs; workgroup 1 + t turns token t's x into digits (global, read
 // by every expert's gate/up workgroups from L2).  Grouping: pair p's position is its expert's
-// start plus the number of earlier pairs with the same expert (its rank); an expert's start
-// is the sum of the counts of the experts before it.  The starts (and the list of active
-// experts) come from one exclusive scan over the counts; a rank is a few popcounts of the
-// expert's bitmask of pairs (built with atomicOr: order-free), or, when the masks would not
-// fit LDS, a count over the earlier pairs.  Every result is a pure function of ids.
-#define HH_MOEG_MASK_WORDS 4096  // LDS words for the per-expert pair bitmasks
+// start plus its rank among the expert's pairs, which is what an LDS counter returns as it
+// counts them.  The order inside an expert is therefore that of arrival; nothing depends on it
+// (every pair's row is computed by itself and written by its own number).  The starts (and the
+// list of active experts) come from one exclusive scan over the counts.  Counting earlier pairs
+// instead, in pair order, cost 470 us of a 1.23 ms layer at 4096 pairs.
 
 // Exclusive scan over the workgroup of (a, b) pairs, one pair per thread (256 threads):
 // returns the sums of the pairs of lower threads; *ta, *tb get the totals.
@@ -113,22 +118,14 @@ HH_DEV void hh_moeg_group(const hh_moeg_args& a) {
     __shared__ int cnt[HH_MOEG_MAX_E];
     __shared__ int first[HH_MOEG_MAX_E];
     __shared__ int apos[HH_MOEG_MAX_E];  // an active expert's position in ascending order
-    __shared__ int pid[HH_MOEG_MAX_P];
-    __shared__ uint32_t mask[HH_MOEG_MASK_WORDS];
+    __shared__ uint32_t pid[HH_MOEG_MAX_P];  // expert | rank << 16; 0xFFFF: no expert
     const uint32_t tid = threadIdx.x;
     const uint32_t E = a.n_experts, P = a.T * a.k;
-    const uint32_t PW = (P + 31) / 32;                     // mask words per expert
-    const bool masks = (size_t)E * PW <= HH_MOEG_MASK_WORDS;  // else: count earlier pairs
     for (uint32_t e = tid; e < E; e += 256) cnt[e] = 0;
-    if (masks)
-        for (uint32_t i = tid; i < E * PW; i += 256) mask[i] = 0u;
-    for (uint32_t p = tid; p < P; p += 256) pid[p] = hh_moeg_valid(a, a.ids[p]);
     __syncthreads();
     for (uint32_t p = tid; p < P; p += 256) {
-        const int e = pid[p];
-        if (e < 0) continue;
-        atomicAdd(&cnt[e], 1);  // counts and masks only: order-free
-        if (masks) atomicOr(&mask[(uint32_t)e * PW + p / 32], 1u << (p % 32));
+        const int e = hh_moeg_valid(a, a.ids[p]);
+        pid[p] = e < 0 ? 0xFFFFu : (uint32_t)e | (uint32_t)atomicAdd(&cnt[e], 1) << 16;
     }
     __syncthreads();
     // starts and active-expert positions: each thread owns experts 2 tid and 2 tid + 1
@@ -140,7 +137,7 @@ HH_DEV void hh_moeg_group(const hh_moeg_args& a) {
         const int2 ex = hh_moeg_scan256(c0 + c1, (c0 > 0) + (c1 > 0), &tot, &tot_a);
         if (e0 < E) {
             first[e0] = ex.x;
-            if (c0) {
+            if (c0 && a.rec) {
                 int* r = a.rec + (size_t)ex.y * HH_MOEG_REC;
                 r[0] = (int)e0;
                 r[1] = ex.x;
@@ -150,7 +147,7 @@ HH_DEV void hh_moeg_group(const hh_moeg_args& a) {
         }
         if (e1 < E) {
             first[e1] = ex.x + c0;
-            if (c1) {
+            if (c1 && a.rec) {
                 const int y = ex.y + (c0 > 0);
                 int* r = a.rec + (size_t)y * HH_MOEG_REC;
                 r[0] = (int)e1;
@@ -160,27 +157,36 @@ HH_DEV void hh_moeg_group(const hh_moeg_args& a) {
             }
         }
         // the records past the active experts, up to the grid's min(E, P) rows
-        for (uint32_t y = (uint32_t)tot_a + tid; y < min(E, P); y += 256) a.rec[(size_t)y * HH_MOEG_REC] = -1;
+        if (a.rec)
+            for (uint32_t y = (uint32_t)tot_a + tid; y < min(E, P); y += 256) a.rec[(size_t)y * HH_MOEG_REC] = -1;
+        if (a.trec) {
+            const int R = (int)a.trows, n0 = (c0 + R - 1) / R, n1 = (c1 + R - 1) / R;
+            __syncthreads();  // the scan's LDS words are read
+            int tiles, none;
+            const int at = hh_moeg_scan256(n0 + n1, 0, &tiles, &none).x;
+            for (int i = 0; i < n0; i++)
+                a.trec[1 + at + i] = make_int4((int)e0, first[e0] + i * R, min(R, c0 - i * R), 0);
+            for (int i = 0; i < n1; i++)
+                a.trec[1 + at + n0 + i] = make_int4((int)e1, first[e1] + i * R, min(R, c1 - i * R), 0);
+            if (tid == 0) a.trec[0] = make_int4(tiles, 0, 0, 0);
+        }
     }
     __syncthreads();
     for (uint32_t p = tid; p < P; p += 256) {
-        const int e = pid[p];
-        if (e < 0) continue;
-        int r = 0;
-        if (masks) {
-            const uint32_t* m = mask + (uint32_t)e * PW;
-            for (uint32_t wi = 0; wi < p / 32; wi++) r += __popc(m[wi]);
-            r += __popc(m[p / 32] & ((1u << (p % 32)) - 1u));
-        } else {
-            for (uint32_t q = 0; q < p; q++) r += pid[q] == e;
-        }
+        const uint32_t e = pid[p] & 0xFFFFu;
+        if (e == 0xFFFFu) continue;
+        const int r = (int)(pid[p] >> 16);
         a.order[first[e] + r] = (int)p;
-        if (r < HH_MOEG_NS) a.rec[(size_t)apos[e] * HH_MOEG_REC + 3 + r] = (int)p;
+        if (r < HH_MOEG_NS && a.rec) a.rec[(size_t)apos[e] * HH_MOEG_REC + 3 + r] = (int)p;
     }
 }
 
 // Token t's x -> digits (global, read by every expert's gate/up workgroups from L2).
 HH_DEV void hh_moeg_x_digits(const hh_moeg_args& a, uint32_t t) {
+    if (a.trec) {  // mmg.hip's kernels take x through hh_mmg_moe_conv
+        hh_mmg_token_amax(a.x + (size_t)t * a.d_model, a.d_model, a.amax + t);
+        return;
+    }
     hh_quantize_digits(a.x + (size_t)t * a.d_model, a.d_model,
                        hh_moe_digits((char*)a.xq + t * hh_digits_bytes_dev(a.d_model), a.d_model));
 }

@@ -1130,34 +1130,48 @@ struct MmgArgs {
     const uint8_t* w0;
     const uint8_t* w1;
     const uint8_t* xs;
-    const float* down;
+    const float* amax;
+    float* pmax;
     float* y;
     uint64_t row_bytes, tile_bytes, part_stride, up_stride;
     uint32_t m, n, b, nch, cpk, kc, groups, ttiles;
     int32_t act;
-    uint32_t pad;
+    uint32_t ldt;
+    const void* trec;
+    const int32_t* order;
+    uint64_t expert_stride;
 };
 struct MmgConvArgs {
     const float* x;
     uint8_t* xs;
-    const float* up;
+    float* amax;
+    const float* pmax;
     uint64_t tile_bytes;
-    uint32_t b, n, nch, rows, mins, half_major, paired, pad;
+    uint32_t b, n, nch, rows, mins, half_major, paired, pgroups, ldt, pad;
 };
 struct MmgAmaxArgs {
     const float* x;
-    float* up;
-    float* down;
+    float* amax;
     uint32_t n, pad;
+};
+struct MmgMoeArgs {
+    MmgConvArgs c;
+    const void* trec;
+    const int32_t* order;
+    float* amax_row;
+    uint32_t k, pad;
 };
 struct MmgSumArgs {
     const float* part;
     float* y;
-    uint64_t stride, up_stride, count;
-    uint32_t kc;
+    uint64_t stride, up_stride;
+    float* pmax;
+    uint32_t m, kc;
     int32_t act;
+    uint32_t ldt;
 };
 constexpr size_t kMmgMaxTokens = 1024;  // tokens per pass (bounds the workspaces)
+constexpr size_t kMmgLdt = kMmgMaxTokens + 64;  // tokens padded to whole tiles
 // From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
 // 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
 // one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
@@ -1247,26 +1261,33 @@ hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, cons
     }
     hh_status st = grow(&ws_mg_s, &ws_mg_s_cap, s);
     if (st == HH_OK && pb) st = grow(&ws_mg_p, &ws_mg_p_cap, pb);
-    if (st == HH_OK) st = grow(&ws_mg_f, &ws_mg_f_cap, 2 * (kMmgMaxTokens + 64) * sizeof(float));
+    // per token: x's and h's largest magnitudes, and those of h by row groups of gate/up
+    size_t pg = 0;
+    for (int i = 0; i < count; i++)
+        if (gus[i]) pg = std::max(pg, (ms[i] + 127) / 128);
+    if (st == HH_OK) st = grow(&ws_mg_f, &ws_mg_f_cap, (2 + pg) * kMmgLdt * sizeof(float));
     return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
 }
 
-hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b) {
+// h: the tokens are gate/up's output, whose largest magnitudes are there by so many row groups.
+hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h) {
     const MmgFmt* f = mmg_fmt(type);
     const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
-    float* up = (float*)ws_mg_f;
-    float* down = up + kMmgMaxTokens + 64;
+    float* amax = (float*)ws_mg_f + (h ? kMmgLdt : 0);
     hipFunction_t fn;
-    HH_TRY(kernel("hh_mmg_amax", &fn));
-    HH_TRY(launch(fn, (uint32_t)b, 256, MmgAmaxArgs{x, up, down, (uint32_t)n, 0}));
+    if (!h) {
+        HH_TRY(kernel("hh_mmg_amax", &fn));
+        HH_TRY(launch(fn, (uint32_t)b, 256, MmgAmaxArgs{x, amax, (uint32_t)n, 0}));
+    }
     HH_TRY(kernel("hh_mmg_conv", &fn));
     return launch(fn, (uint32_t)(p.tiles * p.nch), 256,
-                  MmgConvArgs{x, (uint8_t*)ws_mg_s, up, p.tile_bytes, (uint32_t)b, (uint32_t)n, (uint32_t)p.nch,
-                              (uint32_t)p.rows, f->mins, f->half_major, f->paired, 0});
+                  MmgConvArgs{x, (uint8_t*)ws_mg_s, amax, h ? (float*)ws_mg_f + 2 * kMmgLdt : nullptr, p.tile_bytes,
+                              (uint32_t)b, (uint32_t)n, (uint32_t)p.nch, (uint32_t)p.rows, f->mins, f->half_major,
+                              f->paired, (uint32_t)h, (uint32_t)kMmgLdt, 0});
 }
 
 hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b,
-                                 float* y, int act) {
+                                 float* y, int act, bool h) {
     const MmgFmt* f = mmg_fmt(type);
     const bool gu = w1 != nullptr;
     const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
@@ -1278,7 +1299,9 @@ hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0
     a.w0 = w0;
     a.w1 = gu ? w1 : w0;
     a.xs = (const uint8_t*)ws_mg_s;
-    a.down = (const float*)ws_mg_f + kMmgMaxTokens + 64;
+    a.amax = (const float*)ws_mg_f + (h ? kMmgLdt : 0);
+    a.pmax = (float*)ws_mg_f + 2 * kMmgLdt;
+    a.ldt = (uint32_t)kMmgLdt;
     a.y = p.kc > 1 ? (float*)ws_mg_p : y;
     a.row_bytes = rb;
     a.tile_bytes = p.tile_bytes;
@@ -1300,9 +1323,12 @@ hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0
                "hipModuleLaunchKernel(mmg)");
     if (p.kc == 1) return HH_OK;
     HH_TRY(kernel(gu ? "hh_mmg_sum_act" : "hh_mmg_sum", &fn));
-    const size_t count = b * m;
-    return launch(fn, (uint32_t)((count + 255) / 256), 256,
-                  MmgSumArgs{(const float*)ws_mg_p, y, a.part_stride, a.up_stride, count, (uint32_t)p.kc, act});
+    MmgSumArgs sa{(const float*)ws_mg_p, y, a.part_stride, a.up_stride, a.pmax, (uint32_t)m, (uint32_t)p.kc, act,
+                  (uint32_t)kMmgLdt};
+    void* sp[] = {&sa};
+    HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)((m + 255) / 256), (uint32_t)b, 1, 256, 1, 1, 0, stream, sp, nullptr),
+               "hipModuleLaunchKernel(mmg sums)");
+    return HH_OK;
 }
 
 hh_status hh_engine::enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b,
@@ -1313,8 +1339,8 @@ hh_status hh_engine::enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_
         if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1));
     for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
         const size_t nb = std::min(kMmgMaxTokens, b - b0);
-        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb));
-        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0));
+        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb, 0));
+        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0, false));
     }
     return HH_OK;
 }
@@ -1338,10 +1364,11 @@ hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, 
     for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
         const size_t nb = std::min(kMmgMaxTokens, b - b0);
         float* h = (float*)ws_mg_h;
-        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb));
-        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act));
-        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb));
-        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0));
+        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb, 0));
+        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act, false));
+        const size_t kc = plan_mmg(mmg_fmt(d->type_gate), true, df, dm, nb, (size_t)props.multiProcessorCount).kc;
+        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb, kc == 1 ? (df + 127) / 128 : (df + 255) / 256));
+        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0, true));
     }
     ffn_stage_valid = false;
     ffn_calls += 3 * b;
@@ -1513,10 +1540,166 @@ hh_status hh_engine::enqueue_moe_route(const hh_moe_desc* d, const float* logits
     return launch(fn, (uint32_t)((T + 3) / 4), kMoeBlock, a);
 }
 
+// Must match struct hh_moeg_args in kernels/moe_group.hip.
+struct MoegArgs {
+    const uint8_t* experts;
+    uint64_t expert_stride, gate_off, up_off, down_off, rb_in, rb_ff;
+    const int32_t* ids;
+    const float* wts;
+    const float* x;
+    float *h, *yp, *y;
+    int32_t *order, *rec;
+    uint8_t *xq, *hq;
+    uint32_t T, k, d_model, d_ff, n_experts;
+    int32_t act;
+    void* trec;
+    float* amax;
+    uint32_t trows, pad;
+};
+constexpr size_t kMoeMaxPairs = 4096;  // (token, slot) pairs of a grouping (HH_MOEG_MAX_P)
+
+// The pairs' grouping and x's per-token form.  With logits, routing, grouping and x in one
+// launch (hh_moe_route_prep): the last routing workgroup to finish groups the pairs; its
+// arrival counter is a word of the grid-barrier state that every launch leaves at zero.
+hh_status hh_engine::launch_moe_prep(const hh_moe_desc* d, const MoegArgs& g, const float* logits, const float* bias,
+                                     int32_t* ids, float* wts) {
+    const size_t T = g.T;
+    hipFunction_t fn;
+    if (!logits) {
+        HH_TRY(kernel("hh_moe_prep", &fn));
+        return launch(fn, (uint32_t)(1 + T), 256, g);
+    }
+    struct {
+        hh_route_args r;
+        MoegArgs m;
+        unsigned* arrivals;
+    } rp{route_args(d, logits, bias, T, ids, wts), g, (unsigned*)((char*)grid_sync + kBarMoeArrivalsOffset)};
+    HH_TRY(kernel("hh_moe_route_prep", &fn));
+    return launch(fn, (uint32_t)((T + 3) / 4 + T), kMoeBlock, rp);
+}
+
+// Many pairs per expert: the experts' products on the matrix cores (mmg.hip), in tiles of 16
+// or 32 pairs of one expert.  Workspaces: the stages of x's pairs, then of h's (in turn), h,
+// the pairs' outputs, the tiles' records and every factor.
+hh_status hh_engine::enqueue_moe_mmg(const hh_moe_desc* d, const uint8_t* experts, const float* x, size_t T,
+                                     int32_t* ids, float* wts, float* y, const float* logits, const float* bias) {
+    const size_t k = d->top_k, dm = d->d_model, df = d->d_ff, P = T * k, E = d->n_experts;
+    if (dm % 256 || df % 256) return HH_ERR_UNSUPPORTED_DEVICE;
+    // 16-pair tiles up to about 10 pairs an expert: fewer matrix-core steps are spent on padding
+    const size_t act = std::min(E, P), rows = P <= 10 * act ? 16 : 32;
+    const size_t tiles = P / rows + act;  // at most: every expert's last tile partly filled
+    auto stage = [&](size_t n) { return n / 128 * (rows == 16 ? 8192 : 16384) + n / 256 * 1024; };
+    const size_t s_bytes = tiles * std::max(stage(dm), stage(df));
+    const size_t f_count = T + (2 + df / 128) * tiles * rows + 64;
+    const size_t g_bytes = (1 + tiles) * 16 + P * 4;
+    hh_status st = grow(&ws_mg_s, &ws_mg_s_cap, s_bytes);
+    if (st == HH_OK) st = grow(&ws_mg_h, &ws_mg_h_cap, tiles * rows * df * sizeof(float));
+    if (st == HH_OK) st = grow(&ws_mg_f, &ws_mg_f_cap, f_count * sizeof(float));
+    if (st == HH_OK) st = grow(&ws_moe_yp, &ws_moe_yp_cap, P * dm * sizeof(float));
+    if (st == HH_OK) st = grow(&ws_moe_grp, &ws_moe_grp_cap, g_bytes);
+    if (st != HH_OK) return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
+    uint8_t* trec = (uint8_t*)ws_moe_grp;
+    int32_t* order = (int32_t*)(trec + (1 + tiles) * 16);
+    float* amax_x = (float*)ws_mg_f;  // per tile row, 16-byte aligned
+    float* amax_h = amax_x + tiles * rows;
+    float* pmax = amax_h + tiles * rows;
+    float* amax_tok = pmax + df / 128 * tiles * rows;
+    MoegArgs g{};
+    g.ids = ids;
+    g.wts = wts;
+    g.x = x;
+    g.yp = (float*)ws_moe_yp;
+    g.y = y;
+    g.order = order;
+    g.T = (uint32_t)T;
+    g.k = (uint32_t)k;
+    g.d_model = (uint32_t)dm;
+    g.d_ff = (uint32_t)df;
+    g.n_experts = (uint32_t)E;
+    g.act = d->act;
+    g.trec = trec;
+    g.amax = amax_tok;
+    g.trows = (uint32_t)rows;
+    HH_TRY(launch_moe_prep(d, g, logits, bias, ids, wts));
+    const MmgFmt* f = mmg_fmt(HH_TYPE_Q4_K);
+    hipFunction_t fn;
+    MmgMoeArgs c{MmgConvArgs{x, (uint8_t*)ws_mg_s, amax_tok, nullptr, stage(dm), 0, (uint32_t)dm,
+                             (uint32_t)(dm / 128), (uint32_t)rows, f->mins, f->half_major, f->paired, 0,
+                             (uint32_t)(tiles * rows), 0},
+                 trec, order, amax_x, (uint32_t)k, 0};
+    HH_TRY(kernel("hh_mmg_moe_conv", &fn));
+    HH_TRY(launch(fn, (uint32_t)(tiles * (dm / 128)), 256, c));
+    const std::string name = std::string("hh_mmg_moe_") + (rows == 16 ? "s16" : "h1");
+    const unsigned smem = 2 * ((rows == 16 ? 8192 : 16384) + 1024);
+    auto product = [&](bool gu, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, float* out) {
+        MmgArgs a{};
+        a.w0 = w0;
+        a.w1 = w1;
+        a.xs = (const uint8_t*)ws_mg_s;
+        a.amax = gu ? amax_x : amax_h;
+        a.pmax = pmax;
+        a.ldt = (uint32_t)(tiles * rows);
+        a.y = out;
+        a.row_bytes = n / 256 * 144;
+        a.tile_bytes = stage(n);
+        a.m = (uint32_t)m;
+        a.n = (uint32_t)n;
+        a.nch = a.cpk = (uint32_t)(n / 128);
+        a.kc = 1;
+        a.groups = (uint32_t)(gu ? (m + 127) / 128 : (m + 255) / 256);
+        a.ttiles = 1;
+        a.act = d->act;
+        a.trec = trec;
+        a.order = order;
+        a.expert_stride = d->expert_stride;
+        HH_TRY(kernel(name + (gu ? "_gu" : ""), &fn));
+        const size_t wgs = (tiles * a.groups + 7) / 8 * 8;
+        void* params[] = {&a};
+        HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)wgs, 1, 1, 256, 1, 1, smem, stream, params, nullptr),
+                   "hipModuleLaunchKernel(mmg moe)");
+        return HH_OK;
+    };
+    HH_TRY(product(true, df, dm, experts + d->gate_off, experts + d->up_off, (float*)ws_mg_h));
+    c.c.x = (const float*)ws_mg_h;
+    c.c.n = (uint32_t)df;
+    c.c.nch = (uint32_t)(df / 128);
+    c.c.tile_bytes = stage(df);
+    c.c.amax = amax_h;
+    c.c.pmax = pmax;
+    c.c.pgroups = (uint32_t)(df / 128);
+    c.k = 0;
+    HH_TRY(kernel("hh_mmg_moe_conv", &fn));
+    HH_TRY(launch(fn, (uint32_t)(tiles * (df / 128)), 256, c));
+    HH_TRY(product(false, dm, df, experts + d->down_off, experts + d->down_off, (float*)ws_moe_yp));
+    HH_TRY(kernel("hh_moe_combine", &fn));
+    void* gp[] = {&g};
+    HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)((dm + 255) / 256), (uint32_t)T, 1, 256, 1, 1, 0, stream, gp, nullptr),
+               "launch(moe combine)");
+    ffn_calls += 3 * T;
+    return HH_OK;
+}
+
 hh_status hh_engine::enqueue_moe_ffn(const hh_moe_desc* d, const uint8_t* experts, const float* x, size_t T,
                                      int32_t* ids, float* wts, float* y, const float* logits, const float* bias) {
     if (T == 0) return HH_OK;
     const size_t k = d->top_k, dm = d->d_model, df = d->d_ff;
+    const bool aligned =
+        ((d->expert_stride | d->gate_off | d->up_off | d->down_off | (uintptr_t)experts | (uintptr_t)x) & 15u) == 0;
+    const size_t P = T * k, E = d->n_experts;
+    const bool groups = moe_grouped && E <= 512 && k <= kMoeMaxPairs && aligned;
+    if (groups && P > kMoeMaxPairs && dm / 64 <= 64 && df / 64 <= 64) {
+        // more pairs than the grouping takes: passes of as many tokens as it does
+        const size_t per = kMoeMaxPairs / k;
+        for (size_t t0 = 0; t0 < T; t0 += per)
+            HH_TRY(enqueue_moe_ffn(d, experts, x + t0 * dm, std::min(per, T - t0), ids + t0 * k, wts + t0 * k,
+                                   y + t0 * dm, logits ? logits + t0 * E : nullptr, bias));
+        return HH_OK;
+    }
+    if (groups && mmg && P <= kMoeMaxPairs && dm / 64 <= 64 && df / 64 <= 64 && T > 1 &&
+        (double)P >= moe_mmg_min * (double)std::min(E, P)) {
+        const hh_status st = enqueue_moe_mmg(d, experts, x, T, ids, wts, y, logits, bias);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
     HH_TRY(grow(&ws_moe_h, &ws_moe_h_cap, T * k * df * sizeof(float)));
     hh_moe_args a{};
     a.experts = experts;
@@ -1576,48 +1759,18 @@ hh_status hh_engine::enqueue_moe_ffn(const hh_moe_desc* d, const uint8_t* expert
         return HH_OK;
     }
     // Several tokens: the grouped gather-GEMV (moe_group.hip), every selected expert read once.
-    const size_t P = T * k, E = d->n_experts;
-    if (moe_grouped && P <= 4096 && E <= 512 && dm / 64 <= 64 && df / 64 <= 64 &&
-        ((d->expert_stride | d->gate_off | d->up_off | d->down_off | (uintptr_t)experts | (uintptr_t)x) & 15u) == 0) {
+    if (groups && P <= kMoeMaxPairs && dm / 64 <= 64 && df / 64 <= 64) {
         HH_TRY(grow(&ws_moe_yp, &ws_moe_yp_cap, P * dm * sizeof(float)));
         const size_t gy = std::min(E, P);  // grid rows of the grouped kernels: the most active experts
         HH_TRY(grow(&ws_moe_grp, &ws_moe_grp_cap, (P + gy * kMoegRecInts) * sizeof(int32_t)));
         const size_t xqb = hh_digits_bytes(dm), hqb = hh_digits_bytes(df);
         HH_TRY(grow(&ws_moe_q, &ws_moe_q_cap, T * xqb + P * hqb));
-        struct {
-            const uint8_t* experts;
-            uint64_t expert_stride, gate_off, up_off, down_off, rb_in, rb_ff;
-            const int32_t* ids;
-            const float* wts;
-            const float* x;
-            float *h, *yp, *y;
-            int32_t *order, *rec;
-            uint8_t *xq, *hq;
-            uint32_t T, k, d_model, d_ff, n_experts;
-            int32_t act;
-        } g{experts, d->expert_stride, d->gate_off, d->up_off, d->down_off, a.rb_in, a.rb_ff, ids, wts, x,
-            (float*)ws_moe_h, (float*)ws_moe_yp, y, (int32_t*)ws_moe_grp + gy * kMoegRecInts,
-            (int32_t*)ws_moe_grp, (uint8_t*)ws_moe_q, (uint8_t*)ws_moe_q + T * xqb, (uint32_t)T,
-            (uint32_t)k, (uint32_t)dm, (uint32_t)df, (uint32_t)E, d->act};
+        MoegArgs g{experts, d->expert_stride, d->gate_off, d->up_off, d->down_off, a.rb_in, a.rb_ff, ids, wts, x,
+                   (float*)ws_moe_h, (float*)ws_moe_yp, y, (int32_t*)ws_moe_grp + gy * kMoegRecInts,
+                   (int32_t*)ws_moe_grp, (uint8_t*)ws_moe_q, (uint8_t*)ws_moe_q + T * xqb, (uint32_t)T,
+                   (uint32_t)k, (uint32_t)dm, (uint32_t)df, (uint32_t)E, d->act, nullptr, nullptr, 0, 0};
         hipFunction_t fn;
-        if (logits) {
-            // routing, grouping and x's digits in one launch (hh_moe_route_prep): the last
-            // routing workgroup to finish groups the pairs; its arrival counter is a word of
-            // the grid-barrier state that every launch leaves at zero
-            struct {
-                hh_route_args r;
-                decltype(g) m;
-                unsigned* arrivals;
-            } rp{route_args(d, logits, bias, T, ids, wts), g, (unsigned*)((char*)grid_sync + kBarMoeArrivalsOffset)};
-            HH_TRY(kernel("hh_moe_route_prep", &fn));
-            void* rpp[] = {&rp};
-            HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)((T + 3) / 4 + T), 1, 1, kMoeBlock, 1, 1, 0, stream, rpp,
-                                             nullptr),
-                       "launch(moe route + prep)");
-        } else {
-            HH_TRY(kernel("hh_moe_prep", &fn));
-            HH_TRY(launch(fn, (uint32_t)(1 + T), 256, g));
-        }
+        HH_TRY(launch_moe_prep(d, g, logits, bias, ids, wts));
         {
             const int team = moe_team(dm / 64);
             const size_t rows = (size_t)(kMoeBlock / team) * kMoegGuRows;
@@ -1733,7 +1886,9 @@ static std::vector<std::string> required_kernels() {
         for (const char* f : {"_d2_w", "_d4_w", "_d2_r", "_d4_r"}) k.push_back("hh_q4k_mmi_t" + std::to_string(t) + f);
     for (const char* f : {"t1_d2_w", "t1_d2_r", "t2_d2_w", "t2_d2_r", "t4_d2_w", "t4_d2_r"})
         k.push_back(std::string("hh_q4k_mmi_gu_") + f);
-    for (const char* f : {"hh_mmg_amax", "hh_mmg_conv", "hh_mmg_sum", "hh_mmg_sum_act"}) k.push_back(f);
+    for (const char* f : {"hh_mmg_amax", "hh_mmg_conv", "hh_mmg_sum", "hh_mmg_sum_act", "hh_mmg_moe_conv",
+                          "hh_mmg_moe_s16", "hh_mmg_moe_s16_gu", "hh_mmg_moe_h1", "hh_mmg_moe_h1_gu"})
+        k.push_back(f);
     for (const MmgFmt& f : kMmgFmts)
         for (const char* mode : {"s16", "h1", "h2"})
             for (const char* gu : {"", "_gu"})
@@ -1827,6 +1982,7 @@ hh_status engine_create(int device, hh_engine** out) {
     if (const char* f = getenv("HAYAI_HIP_RING_GU_PER_CU")) e->ring_gu_per_cu = std::max(1, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_RING_DN_PER_CU")) e->ring_dn_per_cu = std::max(1, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMR")) e->mmr = atoi(f) != 0;
+    if (const char* f = getenv("HAYAI_HIP_MOE_MMG_MIN")) e->moe_mmg_min = atof(f);
     if (const char* f = getenv("HAYAI_HIP_MMG")) e->mmg = atoi(f) != 0;
     if (const char* f = getenv("HAYAI_HIP_MMI_MIN")) e->mmi_min = (size_t)std::max(2, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_D")) e->mmi_d = atoi(f);

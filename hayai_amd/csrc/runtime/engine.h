@@ -84,6 +84,8 @@ struct hh_event {
     int device;
 };
 
+struct MoegArgs;
+
 struct hh_engine {
     int device = 0;
     hipDeviceProp_t props{};
@@ -169,6 +171,11 @@ struct hh_engine {
     bool mmr = true;            // HAYAI_HIP_MMR=0: batched Q4_K (<= 16 tokens) one token at a time
     bool mmq = true;            // HAYAI_HIP_MMQ=0: batched Q4_K (>= 17 tokens) one token at a time, no int8
     bool mmg = true;            // HAYAI_HIP_MMG=0: other formats' batches one token at a time
+    // HAYAI_HIP_MOE_MMG_MIN: (token, slot) pairs per expert from which MoE runs on mmg.hip.
+    // Against the grouped gather-GEMV, us: 128 experts 2048 x 768 4 pairs 161 : 148, 6.2 pairs
+    // 166 : 205; 64 experts 1024 x 1280 4 pairs 76 : 80; 16 experts 1024 x 512 4 pairs 41 : 33,
+    // 6 pairs 41 : 40, 8 pairs 42 : 45.
+    double moe_mmg_min = 6;
     size_t mmi_min = 17;        // HAYAI_HIP_MMI_MIN: fewest tokens per pass on the int8 kernels (>= 2)
     int mmi_d = 0;              // HAYAI_HIP_MMI_D: ring depth of the int8 f16-MFMA kernels (0: chosen)
     int blocks_per_cu_override = 0;  // HAYAI_HIP_BLOCKS_PER_CU
@@ -280,11 +287,12 @@ struct hh_engine {
     // any launch) when shape, type or alignment does not fit or the workspaces cannot be had.
     bool mmg_ok(int type, size_t m, size_t n, const void* w) const;
     hh_status mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus, int count);
-    // x [b][n] -> stages of `type`'s order, with the factors of each token
-    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b);
+    // x [b][n] -> stages of `type`'s order (h: x is gate/up's output, its
+    // largest magnitudes known by so many row groups)
+    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h);
     // the product of the staged tokens: GEMM (w1 null) into y [b][m], or gate/up + act into y
     hh_status mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b, float* y,
-                          int act);
+                          int act, bool h);
     hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y);
     hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y);
     // MoE routing of T tokens (device pointers) and the grouped expert FFN.
@@ -294,6 +302,10 @@ struct hh_engine {
     hh_status enqueue_moe_ffn(const hh_moe_desc* d, const uint8_t* experts, const float* x, size_t T,
                               int32_t* ids, float* wts, float* y, const float* logits = nullptr,
                               const float* bias = nullptr);
+    hh_status enqueue_moe_mmg(const hh_moe_desc* d, const uint8_t* experts, const float* x, size_t T, int32_t* ids,
+                              float* wts, float* y, const float* logits, const float* bias);
+    hh_status launch_moe_prep(const hh_moe_desc* d, const MoegArgs& g, const float* logits, const float* bias,
+                              int32_t* ids, float* wts);
     // The shared expert of an MoE layer (moe_infer.rs:456-493), after the routed experts:
     // y[t] += FFN_shared(x[t]).  Nothing when the descriptor has none.
     hh_status enqueue_moe_shared(const hh_moe_desc* d, const uint8_t* experts, const float* x, size_t T, float* y);

@@ -305,3 +305,45 @@ def test_moe_grouped_at_the_pair_limit(engine, T):
         worst = max(worst, float(np.max(np.abs(Y[t] - ref)) / np.max(np.abs(ref))))
     print(f"  worst token rel err {worst:.3e}", flush=True)
     assert worst <= REL_TOL
+
+
+@pytest.mark.parametrize("E,k,d_model,d_ff,T", [
+    (4, 2, 256, 256, 13),     # 6.5 pairs an expert: 16-pair tiles, some experts' second tile partly filled
+    (2, 2, 512, 256, 48),     # every expert has every token: 32-pair tiles, the last of 16
+    (3, 1, 256, 768, 200),    # uneven experts, row groups past the matrix
+    (4, 3, 256, 256, 1400),   # 4200 pairs: two passes of the grouping
+])
+def test_moe_on_the_matrix_cores(engine, E, k, d_model, d_ff, T):
+    # From 6 pairs per expert the experts' products run in tiles of one expert's pairs; routed
+    # on the GPU and from given ids with empty slots.
+    print(f"[case] moe tiles E={E} k={k} {d_model}x{d_ff} T={T}", flush=True)
+    buf, host, stride, offs = make_experts(engine, E, d_model, d_ff, 77)
+    d = engine.moe_desc(d_model, d_ff, E, k, stride, offs, norm_topk_prob=True)
+    rng = np.random.default_rng(T)
+    logits = (rng.standard_normal((T, E)) + np.arange(E)).astype(np.float32)
+    x = synth.normal(78, T * d_model).reshape(T, d_model)
+    lb, xb = engine.upload(logits), engine.upload(x)
+    ids_b, w_b = engine.alloc(4 * T * k), engine.alloc(4 * T * k)
+    y = engine.alloc(4 * T * d_model)
+    engine.route_experts_dev(d, lb, 0, None, 0, T, ids_b, 0, w_b, 0)
+    ids = ids_b.read(np.int32, T * k).reshape(T, k)
+    w = w_b.read(np.float32, T * k).reshape(T, k)
+    engine.moe_dev(d, buf, 0, lb, 0, None, 0, xb, 0, T, y, 0)
+    routed = y.read(np.float32, T * d_model).reshape(T, d_model)
+    holes = ids.copy()
+    holes[1, 0], holes[T - 1, k - 1] = -1, E
+    hb = engine.upload(holes)
+    engine.moe_ffn_dev(d, buf, 0, xb, 0, T, hb, 0, w_b, 0, y, 0)
+    given = y.read(np.float32, T * d_model).reshape(T, d_model)
+    for t in list(range(min(T, 24))) + [T - 2, T - 1]:
+        for got, chosen in ((routed, ids), (given, holes)):
+            keep = [(int(e), float(v)) for e, v in zip(chosen[t], w[t]) if 0 <= e < E]
+            if not keep:
+                assert not got[t].any()
+                continue
+            ref = oracle.moe_token(Q4_K, d_model, d_ff, host, stride, offs, [e for e, _ in keep], [v for _, v in keep],
+                                   x[t])
+            # f32 sums on both sides, as test_gpu_many_tokens.py
+            assert np.max(np.abs(got[t] - ref)) <= 2e-5 * np.max(np.abs(ref)), t
+    same = np.setdiff1d(np.arange(T), [1, T - 1])
+    np.testing.assert_array_equal(routed[same], given[same])
