@@ -50,7 +50,7 @@ typedef float hh_f16v __attribute__((ext_vector_type(16)));
 #ifndef HH_MMG_VALU
 #define HH_MMG_VALU 0
 #endif
-enum { HH_MMG_H = 0, HH_MMG_S16 = 1 };
+enum { HH_MMG_H = 0, HH_MMG_S16 = 1, HH_MMG_F = 2 };
 
 struct hh_mmg_args {
     const uint8_t* w0;       // GEMM: W; gate/up: W_gate
@@ -116,7 +116,7 @@ struct hh_mmg_k {
 };
 
 // ---- weight formats -------------------------------------------------------------------
-// Raw: one chunk's bytes of one row as loaded; load(p, ch, ...) of chunk ch of the row at p
+// Raw: one chunk's bytes of one row as loaded (ready: what is taken from them once); load(p, ch, ...) of chunk ch of the row at p
 // (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
 // the d of the block that group g closes.  NB: B operands per step.
 struct hh_mmg_q4_0 {
@@ -186,7 +186,12 @@ struct hh_mmg_q4_k {
     struct Raw {
         uint4 q[2];
         uint4 hd;
+        uint32_t sch;  // the chunk's four sub-block scales
     };
+    template <uint32_t HALF>
+    HH_DEV static void ready(Raw& r) {
+        r.sch = HALF ? (r.hd.w & 0x0F0F0F0Fu) | ((r.hd.y >> 2) & 0x30303030u) : r.hd.y & 0x3F3F3F3Fu;
+    }
     template <uint32_t HALF>
     HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t) {
         const uint8_t* b = p + (ch >> 1) * 144u;
@@ -205,15 +210,12 @@ struct hh_mmg_q4_k {
     }
     template <uint32_t HALF>
     HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
-        // the chunk's four sub-block scales; sub-blocks 2p (low nibbles) and 2p + 1 (high) of
-        // the 32 qs bytes p
-        const uint32_t sch =
-            HALF ? (r.hd.w & 0x0F0F0F0Fu) | ((r.hd.y >> 2) & 0x30303030u) : r.hd.y & 0x3F3F3F3Fu;
+        // sub-blocks 2p (low nibbles) and 2p + 1 (high) of the 32 qs bytes p
         const uint4 q = r.q[g >> 1];
         const uint32_t a = s ? q.z : q.x, b = s ? q.w : q.y;
         const uint32_t v[4] = {a, a >> 8, b, b >> 8};
         const uint32_t sel = (uint32_t)g | (4u << 8) | ((uint32_t)g << 16) | (4u << 24);
-        const hh_h2 sc = hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, sch, sel)) - hh_h2_all(1024.f);
+        const hh_h2 sc = hh_h2_bits(__builtin_amdgcn_perm(0x64646464u, r.sch, sel)) - hh_h2_all(1024.f);
         const hh_h2 mul = (g & 1) ? sc * hh_h2_all(0.0625f) : sc;
         const hh_h2 off = mul * hh_h2_all(-1024.f);
         const uint32_t mask = (g & 1) ? k.hi : k.lo;
@@ -390,7 +392,7 @@ struct hh_mmg_conv_args {
     uint32_t half_major;   // column order 16 h + 8 step + e (else 16 step + 8 h + e)
     uint32_t paired;       // e in the order 0 2 1 3 4 6 5 7
     uint32_t pgroups, ldt;
-    uint32_t pad;
+    uint32_t single;       // mode f: hi alone, the sums as two bf16
 };
 
 struct hh_mmg_amax_args {
@@ -440,6 +442,13 @@ extern "C" __global__ void __launch_bounds__(256) hh_mmg_amax(const hh_mmg_amax_
 HH_DEV float hh_mmg_up(float amax) { return ldexpf(1.f, hh_mmg_exp(amax)); }
 HH_DEV float hh_mmg_down(float amax) { return ldexpf(1.f, -hh_mmg_exp(amax)); }
 
+// f32 -> bf16 bits, to nearest even (infinities stay; a NaN keeps a set mantissa bit)
+HH_DEV uint32_t hh_bf16(float v) {
+    const uint32_t b = __float_as_uint(v);
+    if ((b & 0x7FFFFFFFu) >= 0x7F800000u) return (b >> 16) | ((b & 0x7FFFFFu) ? 0x40u : 0u);
+    return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
+}
+
 HH_DEV void hh_mmg_split(float v, _Float16& hi, _Float16& lo) {
     hi = (_Float16)v;
     const float r = v - (float)hi;
@@ -452,7 +461,7 @@ template <class ROW>
 HH_DEV void hh_mmg_conv_chunk(uint8_t* tile, const hh_mmg_conv_args& a, uint32_t ch, bool vec, uint32_t threads,
                               ROW row) {
     const bool s16 = a.rows == 16;
-    const uint32_t chunk_bytes = (s16 ? 8u : 16u) * 1024u;
+    const uint32_t chunk_bytes = (s16 || a.single ? 8u : 16u) * 1024u;
     uint8_t* st = tile + (a.mins ? (size_t)(ch >> 1) * (2 * chunk_bytes + 1024u) + (ch & 1u) * chunk_bytes
                                  : (size_t)ch * chunk_bytes);
     for (uint32_t p = threadIdx.x; p < (s16 ? 256u : 512u); p += threads) {
@@ -495,6 +504,8 @@ HH_DEV void hh_mmg_conv_chunk(uint8_t* tile, const hh_mmg_conv_args& a, uint32_t
         if (s16) {
             *reinterpret_cast<hh_h8*>(st + gs * 1024u + (32 * h + tok) * 16u) = hi;
             *reinterpret_cast<hh_h8*>(st + gs * 1024u + (32 * h + 16 + tok) * 16u) = lo;
+        } else if (a.single) {
+            *reinterpret_cast<hh_h8*>(st + gs * 1024u + (32 * h + tok) * 16u) = hi;
         } else {
             *reinterpret_cast<hh_h8*>(st + gs * 2048u + (32 * h + tok) * 16u) = hi;
             *reinterpret_cast<hh_h8*>(st + gs * 2048u + 1024u + (32 * h + tok) * 16u) = lo;
@@ -511,6 +522,12 @@ HH_DEV void hh_mmg_conv_chunk(uint8_t* tile, const hh_mmg_conv_args& a, uint32_t
     if (r < a.rows && row(r, src, up)) {
         src += 128 * ch + 32 * g;
         for (int e = 0; e < 32; e++) s += src[e] * up;
+    }
+    if (a.single) {
+        const uint32_t hi = hh_bf16(s), lo = hh_bf16(s - __uint_as_float(hi << 16));
+        *reinterpret_cast<uint16_t*>(sums + r * 16 + j * 2) = (uint16_t)hi;
+        *reinterpret_cast<uint16_t*>(sums + 512 + r * 16 + j * 2) = (uint16_t)lo;
+        return;
     }
     _Float16 hi, lo;
     hh_mmg_split(s, hi, lo);
@@ -608,6 +625,70 @@ HH_DEV void hh_mmg_sync() {
     asm volatile("" ::: "memory");
 }
 
+// The sums of a wave's 64 weight rows and TT token tiles to memory (gate/up: the activation,
+// and the row group's largest |h| of each token).
+template <int MODE, int TT, bool GU, bool MOE>
+HH_DEV void hh_mmg_store(const hh_mmg_args& a, const hh_f16v (&sum)[2][TT], const uint32_t (&row)[2], int4 rec,
+                         uint32_t tg, uint32_t grp, uint32_t kci) {
+    constexpr uint32_t ROWS = MODE == HH_MMG_S16 ? 16 : 32;  // tokens per tile
+    extern __shared__ __attribute__((aligned(16))) char hh_smem[];
+    const uint32_t tid = threadIdx.x, lane = tid % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const uint32_t r = lane & 31u, h = lane >> 5;
+    // outputs: lane's weight row, tokens 8 (i / 4) + 4 h + i % 4 of each tile
+    float* const out = a.y + (a.kc > 1 ? kci * a.part_stride : 0);
+    const bool fuse = GU && (MOE || a.kc == 1);
+    float* const wmax = reinterpret_cast<float*>(hh_smem) + wave * 2 * (TT * ROWS);  // gate/up: per token
+    if (fuse) hh_mmg_sync();  // the token buffers are read
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++) {
+#pragma unroll
+        for (int i4 = 0; i4 < (MODE == HH_MMG_S16 ? 2 : 4); i4++) {
+            const uint32_t in = 8 * i4 + 4 * h, t0 = (tg * TT + tt) * ROWS + in;
+            const float4 d4 = *reinterpret_cast<const float4*>(a.amax + t0);  // padded to whole tiles
+            const float dn[4] = {hh_mmg_down(d4.x), hh_mmg_down(d4.y), hh_mmg_down(d4.z), hh_mmg_down(d4.w)};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                uint32_t t = t0 + k;
+                const bool live = MOE ? (int)(in + k) < rec.z : t < a.b;
+                if constexpr (MOE && !GU) t = (uint32_t)a.order[rec.y + min((int)(in + k), rec.z - 1)];  // the pair
+                float v[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    v[q] = sum[q][tt][4 * i4 + k];
+                    if constexpr (MODE == HH_MMG_S16) v[q] += sum[q][tt][4 * i4 + k + 8];
+                    v[q] *= dn[k];
+                }
+                if (fuse) {
+                    float hv = hh_act_mul(v[0], v[1], a.act);
+                    if (live && row[0] < a.m) out[(size_t)t * a.m + row[0]] = hv;
+                    // over the wave's 32 rows (the token is the same in a lane half)
+                    // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
+                    hv = row[0] < a.m ? fabsf(hv) : 0.f;
+                    hv = fmaxf(hv, hh_dpp<0xB1>(hv));   // quad_perm [1,0,3,2]
+                    hv = fmaxf(hv, hh_dpp<0x4E>(hv));   // quad_perm [2,3,0,1]
+                    hv = fmaxf(hv, hh_dpp<0x124>(hv));  // row_ror:4
+                    hv = fmaxf(hv, hh_dpp<0x128>(hv));  // row_ror:8
+                    if ((r & 15u) == 0) wmax[(r >> 4) * (TT * ROWS) + tt * ROWS + in + k] = hv;
+                } else if (live) {
+                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = v[0];
+                    if (row[1] < a.m) out[(GU ? a.up_stride : 0) + (size_t)t * a.m + row[1]] = v[1];
+                }
+            }
+        }
+    }
+    if (fuse) {
+        hh_mmg_sync();
+        if (tid < TT * ROWS) {
+            const float* w = reinterpret_cast<const float*>(hh_smem) + tid;
+            float v = w[0];
+#pragma unroll
+            for (int k = 1; k < 8; k++) v = fmaxf(v, w[k * (TT * ROWS)]);
+            a.pmax[(size_t)grp * a.ldt + tg * (TT * ROWS) + tid] = v;
+        }
+    }
+}
+
 template <class F, int MODE, int TT, bool GU, bool MOE = false>
 HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     constexpr int NA = MODE == HH_MMG_H ? 2 : 1;
@@ -692,9 +773,13 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
 
     // one chunk out of LDS buffer `buf`: for formats of 256-column blocks the first or second
     // half of one (splits start at even chunks)
-    auto compute = [&](const typename F::Raw* raw, auto buf_c) {
+    auto compute = [&](typename F::Raw* raw, auto buf_c) {
         constexpr uint32_t buf = decltype(buf_c)::value;
         constexpr bool open = buf == 0, close = buf == 1;
+        if constexpr (F::MINS) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) F::template ready<buf>(raw[q]);
+        }
         const char* st = hh_smem + buf * BUF + lane * 16u;
 #pragma unroll
         for (int g = 0; g < 4; g++) {
@@ -798,58 +883,158 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         if (HH_MMG_VALU) interleave();
     }
 
-    // outputs: lane's weight row, tokens 8 (i / 4) + 4 h + i % 4 of each tile
-    float* const out = a.y + (a.kc > 1 ? kci * a.part_stride : 0);
-    const bool fuse = GU && (MOE || a.kc == 1);
-    float* const wmax = reinterpret_cast<float*>(hh_smem) + wave * 2 * (TT * ROWS);  // gate/up: per token
-    if (fuse) hh_mmg_sync();  // the token buffers are read
+    hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci);
+}
+
+// ---- Q4_K, one f16 per token element --------------------------------------------------
+// For all-Q4_K batches past 64 tokens, whose activations the 17..64-token kernels hold in 8
+// bits: here one f16 (11 bits), so half the matrix-core steps of mode h.  128 tokens per
+// workgroup; there is no room for a second accumulator per output at two waves per SIMD, so one
+// runs through all superblocks in units of the current superblock's d: at each new superblock it
+// is multiplied by d_before / d (f32), and the products stay those of exact integers sc q.  In
+// the same units the minimum is -(dmin / d) m_j X_j, whose factors enter the bf16 matrix core as
+// two bf16 each (f32's range, 16 bits).  8B FFN, 512 tokens: 558 us as 8 passes of 8-bit tokens,
+// 294 us here (613 TFLOP/s); error against 64 bits 1.2e-2 -> 5e-4.  A superblock with d = 0 keeps the unit before it and
+// zero scales.
+typedef __bf16 hh_b8 __attribute__((ext_vector_type(8)));
+
+template <bool GU>
+HH_DEV void hh_mmf_body(const hh_mmg_args& a) {
+    typedef hh_mmg_q4_k F;
+    constexpr int TT = 4;
+    constexpr uint32_t CB = 8192u, SUMS = 1024u, BUF = TT * (CB + SUMS);
+    extern __shared__ __attribute__((aligned(16))) char hh_smem[];
+    const uint32_t tid = threadIdx.x, lane = tid % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const uint32_t r = lane & 31u, h = lane >> 5;
+    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const uint32_t unit = slot / a.ttiles * 8u + xcd, tg = slot % a.ttiles;  // as hh_mmg_body
+    if (unit >= a.groups * a.kc) return;
+    const uint32_t grp = unit / a.kc, kci = unit % a.kc;
+    const uint32_t c0 = kci * a.cpk, c1 = min(c0 + a.cpk, a.nch);
+    uint32_t row[2];
+    const uint8_t* wp[2];
+    row[0] = GU ? grp * 128 + wave * 32 + r : grp * 256 + wave * 64 + r;
+    row[1] = GU ? row[0] : row[0] + 32;
+    wp[0] = a.w0 + (size_t)min(row[0], a.m - 1) * a.row_bytes;
+    wp[1] = a.w1 + (size_t)min(row[1], a.m - 1) * a.row_bytes;
+
+    auto copy = [&](uint32_t ch, auto buf_c) {
+        constexpr uint32_t buf = decltype(buf_c)::value;
+        const size_t at = (size_t)(ch >> 1) * (2 * CB + SUMS) + buf * CB;
+        // a wave copies one tile: 8 KB, and in the second half the superblock's sums
+        const uint8_t* src = a.xs + (size_t)(tg * TT + wave) * a.tile_bytes + at + lane * 16u;
+        char* dst = hh_smem + buf * BUF + wave * (CB + SUMS);
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++) {
+        for (uint32_t i = 0; i < (buf ? 9u : 8u); i++)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + i * 1024u),
+                                             (__attribute__((address_space(3))) void*)(dst + i * 1024u), 16, 0, 0);
+    };
+    hh_mmg_k kk;
+    kk.set();
+    hh_f16v acc[2][TT];
+    float u[2] = {1.f, 1.f};  // the accumulators' unit
 #pragma unroll
-        for (int i4 = 0; i4 < (MODE == HH_MMG_S16 ? 2 : 4); i4++) {
-            const uint32_t in = 8 * i4 + 4 * h, t0 = (tg * TT + tt) * ROWS + in;
-            const float4 d4 = *reinterpret_cast<const float4*>(a.amax + t0);  // padded to whole tiles
-            const float dn[4] = {hh_mmg_down(d4.x), hh_mmg_down(d4.y), hh_mmg_down(d4.z), hh_mmg_down(d4.w)};
+    for (int q = 0; q < 2; q++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                uint32_t t = t0 + k;
-                const bool live = MOE ? (int)(in + k) < rec.z : t < a.b;
-                if constexpr (MOE && !GU) t = (uint32_t)a.order[rec.y + min((int)(in + k), rec.z - 1)];  // the pair
-                float v[2];
+        for (int tt = 0; tt < TT; tt++)
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    v[q] = sum[q][tt][4 * i4 + k];
-                    if constexpr (MODE == HH_MMG_S16) v[q] += sum[q][tt][4 * i4 + k + 8];
-                    v[q] *= dn[k];
+            for (int i = 0; i < 16; i++) acc[q][tt][i] = 0.f;
+
+    // a new superblock: its unit, and zero scales where d is zero
+    uint32_t zero[2];  // mask of the scales: 0 where d is
+    auto open = [&](const typename F::Raw* raw) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const float d = F::scale(raw[q], 0);
+            const float n = d != 0.f ? d : u[q];
+            zero[q] = d != 0.f ? 0xFFFFFFFFu : 0u;
+            const float f = u[q] / n;
+            u[q] = n;
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[q][tt][i] *= f;
+        }
+    };
+    auto compute = [&](typename F::Raw* raw, auto buf_c) {
+        constexpr uint32_t buf = decltype(buf_c)::value;
+        const char* st = hh_smem + buf * BUF + lane * 16u;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            F::ready<buf>(raw[q]);
+            raw[q].sch &= zero[q];
+        }
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                hh_h8 wf[2], x[TT];
+#pragma unroll
+                for (int q = 0; q < 2; q++) F::template frag<buf>(raw[q], g, s, h, nullptr, kk, &wf[q]);
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++)
+                    x[tt] = *reinterpret_cast<const hh_h8*>(st + tt * (CB + SUMS) + (g * 2 + s) * 1024);
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                    for (int q = 0; q < 2; q++)
+                        acc[q][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt], wf[q], acc[q][tt], 0, 0, 0);
+            }
+        if constexpr (buf == 1) {
+            // the minima, in units of u
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const hh_h8 m = F::mins(raw[q]);
+                const float rho = -F::min_scale(raw[q]) / u[q];
+                union {
+                    uint16_t b[8];
+                    hh_b8 v;
+                } hi, lo;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float f = rho * (float)m[j];
+                    const uint32_t t = __float_as_uint(f) >> 16;  // truncated: the rest is exact
+                    hi.b[j] = (uint16_t)t;
+                    lo.b[j] = (uint16_t)(__float_as_uint(f - __uint_as_float(t << 16)) >> 16);
                 }
-                if (fuse) {
-                    float hv = hh_act_mul(v[0], v[1], a.act);
-                    if (live && row[0] < a.m) out[(size_t)t * a.m + row[0]] = hv;
-                    // over the wave's 32 rows (the token is the same in a lane half)
-                    // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
-                    hv = row[0] < a.m ? fabsf(hv) : 0.f;
-                    hv = fmaxf(hv, hh_dpp<0xB1>(hv));   // quad_perm [1,0,3,2]
-                    hv = fmaxf(hv, hh_dpp<0x4E>(hv));   // quad_perm [2,3,0,1]
-                    hv = fmaxf(hv, hh_dpp<0x124>(hv));  // row_ror:4
-                    hv = fmaxf(hv, hh_dpp<0x128>(hv));  // row_ror:8
-                    if ((r & 15u) == 0) wmax[(r >> 4) * (TT * ROWS) + tt * ROWS + in + k] = hv;
-                } else if (live) {
-                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = v[0];
-                    if (row[1] < a.m) out[(GU ? a.up_stride : 0) + (size_t)t * a.m + row[1]] = v[1];
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) {
+                    const hh_b8 xs = *reinterpret_cast<const hh_b8*>(st + tt * (CB + SUMS) + CB);
+                    acc[q][tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, hi.v, acc[q][tt], 0, 0, 0);
+                    acc[q][tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, lo.v, acc[q][tt], 0, 0, 0);
                 }
             }
         }
-    }
-    if (fuse) {
-        hh_mmg_sync();
-        if (tid < TT * ROWS) {
-            const float* w = reinterpret_cast<const float*>(hh_smem) + tid;
-            float v = w[0];
+    };
+    typename F::Raw raw[2][2];  // [half][row tile]
+    constexpr hh_uint_c<0> B0{};
+    constexpr hh_uint_c<1> B1{};
+    copy(c0, B0);
 #pragma unroll
-            for (int k = 1; k < 8; k++) v = fmaxf(v, w[k * (TT * ROWS)]);
-            a.pmax[(size_t)grp * a.ldt + tg * (TT * ROWS) + tid] = v;
+    for (int q = 0; q < 2; q++) F::load<0>(raw[0][q], wp[q], c0, h, 0);
+    for (uint32_t ch = c0; ch < c1; ch += 2) {
+        hh_mmg_sync();
+        copy(ch + 1, B1);
+#pragma unroll
+        for (int q = 0; q < 2; q++) F::load<1>(raw[1][q], wp[q], ch + 1, h, 0);
+        open(raw[0]);
+        compute(raw[0], B0);
+        hh_mmg_sync();
+        if (ch + 2 < c1) {
+            copy(ch + 2, B0);
+#pragma unroll
+            for (int q = 0; q < 2; q++) F::load<0>(raw[0][q], wp[q], ch + 2, h, 0);
         }
+        compute(raw[1], B1);
     }
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[q][tt][i] *= u[q];
+    hh_mmg_store<HH_MMG_F, TT, GU, false>(a, acc, row, int4{}, tg, grp, kci);
 }
 
 struct hh_mmg_sum_args {
@@ -918,3 +1103,5 @@ HH_MMG_FORMAT(iq3_xxs, 3)
     }
 HH_MMG_MOE(s16, HH_MMG_S16, 3)
 HH_MMG_MOE(h1, HH_MMG_H, 3)
+extern "C" __global__ void __launch_bounds__(256, 2) hh_mmg_q4_k_f4(const hh_mmg_args a) { hh_mmf_body<false>(a); }
+extern "C" __global__ void __launch_bounds__(256, 2) hh_mmg_q4_k_f4_gu(const hh_mmg_args a) { hh_mmf_body<true>(a); }

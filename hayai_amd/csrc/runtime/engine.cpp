@@ -1147,7 +1147,7 @@ struct MmgConvArgs {
     float* amax;
     const float* pmax;
     uint64_t tile_bytes;
-    uint32_t b, n, nch, rows, mins, half_major, paired, pgroups, ldt, pad;
+    uint32_t b, n, nch, rows, mins, half_major, paired, pgroups, ldt, single;
 };
 struct MmgAmaxArgs {
     const float* x;
@@ -1172,6 +1172,16 @@ struct MmgSumArgs {
 };
 constexpr size_t kMmgMaxTokens = 1024;  // tokens per pass (bounds the workspaces)
 constexpr size_t kMmgLdt = kMmgMaxTokens + 64;  // tokens padded to whole tiles
+// All-Q4_K batches as f16 tokens (mode f) against passes of 64 8-bit tokens: from how many
+// tokens, by the weights.  FFN: 1024 x 2816 97 tokens 57 : 69 us, 512 x 1536 128 tokens 61 : 52,
+// 160 tokens 62 : 70.  One matrix: 128256 x 2048 65 tokens 93 : 166, 32000 x 2048 97 tokens
+// 61 : 69, 4096 x 4096 128 tokens 43 : 39, 200 tokens 43 : 69.
+static size_t mmf_from(bool ffn, size_t m, size_t n) {
+    const size_t w = m * n;
+    if (ffn) return w >= (size_t)2 << 20 ? 97 : 144;
+    return w >= (size_t)100 << 20 ? 65 : w >= (size_t)48 << 20 ? 97 : 136;
+}
+
 // From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
 // 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
 // one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
@@ -1202,11 +1212,14 @@ struct MmgPlan {
     const char* mode;
     size_t rows, tt, tiles, ttiles, groups, nch, cpk, kc, stage, tile_bytes, smem;
 };
-static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus) {
+// single: one f16 per token element (mode f)
+static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus, bool single) {
     MmgPlan p{};
     const size_t pad2 = (b + 63) / 64 * 64, pad1 = (b + 31) / 32 * 32;
     double us;  // of one chunk of one workgroup beside the others of its CU
-    if (b <= 16) {
+    if (single) {
+        p.mode = "f4", p.rows = 32, p.tt = 4, us = 2.4;
+    } else if (b <= 16) {
         p.mode = "s16", p.rows = 16, p.tt = 1, us = 0.7;
     } else if ((double)pad1 * 1.2 <= (double)pad2) {
         p.mode = "h1", p.rows = 32, p.tt = 1, us = 1.3;
@@ -1218,7 +1231,7 @@ static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, 
     p.tiles = p.ttiles * p.tt;
     p.groups = gu ? (m + 127) / 128 : (m + 255) / 256;
     p.nch = (n + 127) / 128;
-    const size_t chunk = (p.rows == 16 ? 8 : 16) * 1024, sums = f->mins ? 1024 : 0;
+    const size_t chunk = (p.rows == 16 || single ? 8 : 16) * 1024, sums = f->mins ? 1024 : 0;
     p.tile_bytes = p.nch * chunk + p.nch / 2 * sums;
     p.smem = 2 * p.tt * (chunk + sums) + f->tab_bytes;
     // splits: rounds of two workgroups per CU against the sums' traffic (8 bytes per output and
@@ -1252,10 +1265,10 @@ bool hh_engine::mmg_ok(int type, size_t m, size_t n, const void* w) const {
 
 // The workspaces of products (types, ms, ns, gate/up) over b tokens, in turn on one stream.
 hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus,
-                              int count) {
+                              int count, bool single) {
     size_t s = 0, pb = 0;
     for (int i = 0; i < count; i++) {
-        const MmgPlan p = plan_mmg(mmg_fmt(types[i]), gus[i], ms[i], ns[i], b, (size_t)props.multiProcessorCount);
+        const MmgPlan p = plan_mmg(mmg_fmt(types[i]), gus[i], ms[i], ns[i], b, (size_t)props.multiProcessorCount, single);
         s = std::max(s, p.tiles * p.tile_bytes);
         if (p.kc > 1) pb = std::max(pb, p.kc * b * ms[i] * (gus[i] ? 2 : 1) * sizeof(float));
     }
@@ -1270,9 +1283,10 @@ hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, cons
 }
 
 // h: the tokens are gate/up's output, whose largest magnitudes are there by so many row groups.
-hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h) {
+hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h,
+                               bool single) {
     const MmgFmt* f = mmg_fmt(type);
-    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, single);
     float* amax = (float*)ws_mg_f + (h ? kMmgLdt : 0);
     hipFunction_t fn;
     if (!h) {
@@ -1283,14 +1297,14 @@ hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const floa
     return launch(fn, (uint32_t)(p.tiles * p.nch), 256,
                   MmgConvArgs{x, (uint8_t*)ws_mg_s, amax, h ? (float*)ws_mg_f + 2 * kMmgLdt : nullptr, p.tile_bytes,
                               (uint32_t)b, (uint32_t)n, (uint32_t)p.nch, (uint32_t)p.rows, f->mins, f->half_major,
-                              f->paired, (uint32_t)h, (uint32_t)kMmgLdt, 0});
+                              f->paired, (uint32_t)h, (uint32_t)kMmgLdt, single});
 }
 
 hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b,
-                                 float* y, int act, bool h) {
+                                 float* y, int act, bool h, bool single) {
     const MmgFmt* f = mmg_fmt(type);
     const bool gu = w1 != nullptr;
-    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount);
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, single);
     size_t rb;
     HH_TRY(row_bytes(type, n, &rb));
     hipFunction_t fn;
@@ -1332,20 +1346,21 @@ hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0
 }
 
 hh_status hh_engine::enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b,
-                                      float* y) {
+                                      float* y, bool single) {
     if (b < kMmgMinTokens || !mmg_ok(type, m, n, w)) return HH_ERR_UNSUPPORTED_DEVICE;
     const bool gu = false;
     for (size_t nb : {std::min(b, kMmgMaxTokens), b % kMmgMaxTokens})  // a full pass and the last
-        if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1));
+        if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1, single));
     for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
         const size_t nb = std::min(kMmgMaxTokens, b - b0);
-        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb, 0));
-        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0, false));
+        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb, 0, single));
+        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0, false, single));
     }
     return HH_OK;
 }
 
-hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y) {
+hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y,
+                                     bool single) {
     const size_t dm = d->d_model, df = d->d_ff;
     const uint8_t* wg = pack + d->gate_off;
     const uint8_t* wu = pack + d->up_off;
@@ -1358,17 +1373,17 @@ hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, 
     const bool gus[] = {true, false};
     const size_t most = std::min(b, kMmgMaxTokens);
     for (size_t nb : {most, b % kMmgMaxTokens})  // a full pass and the last
-        if (nb) HH_TRY(mmg_grow(nb, types, ms, ns, gus, 2));
+        if (nb) HH_TRY(mmg_grow(nb, types, ms, ns, gus, 2, single));
     const hh_status st = grow(&ws_mg_h, &ws_mg_h_cap, most * df * sizeof(float));
     if (st != HH_OK) return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
     for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
         const size_t nb = std::min(kMmgMaxTokens, b - b0);
         float* h = (float*)ws_mg_h;
-        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb, 0));
-        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act, false));
-        const size_t kc = plan_mmg(mmg_fmt(d->type_gate), true, df, dm, nb, (size_t)props.multiProcessorCount).kc;
-        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb, kc == 1 ? (df + 127) / 128 : (df + 255) / 256));
-        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0, true));
+        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb, 0, single));
+        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act, false, single));
+        const size_t kc = plan_mmg(mmg_fmt(d->type_gate), true, df, dm, nb, (size_t)props.multiProcessorCount, single).kc;
+        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb, kc == 1 ? (df + 127) / 128 : (df + 255) / 256, single));
+        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0, true, single));
     }
     ffn_stage_valid = false;
     ffn_calls += 3 * b;
@@ -1382,11 +1397,15 @@ hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const ui
                       ((uintptr_t)x & 15u) == 0 && m <= 0xFFFFFFFFu && n <= 0xFFFFFFFFu;
     if (!mfma) {
         if (type != HH_TYPE_Q4_K) {
-            const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y);
+            const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y, false);
             if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
         }
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_gemv(type, m, n, w, x + b * n, y + b * m));
         return HH_OK;
+    }
+    if (mmq && batch >= (mmf_min ? mmf_min : mmf_from(false, m, n))) {
+        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y, true);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     for (size_t b0 = 0; b0 < batch; b0 += kMmMaxTokens) {
         const size_t nb = std::min(kMmMaxTokens, batch - b0);
@@ -1427,7 +1446,7 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
                       mmr_ok(df, dm, batch, wg, wg, x) && mmr_ok(df, dm, batch, wu, wu, x) &&
                       (((uintptr_t)wd | (uintptr_t)x) & 15u) == 0;
     if (!mfma && !(d->type_gate == HH_TYPE_Q4_K && d->type_up == HH_TYPE_Q4_K && d->type_down == HH_TYPE_Q4_K)) {
-        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y);
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y, false);
         if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     if (q4km) {
@@ -1454,6 +1473,10 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
     if (!mfma) {
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_ffn(d, pack, x + b * dm, y + b * dm));
         return HH_OK;
+    }
+    if (mmq && batch >= (mmf_min ? mmf_min : mmf_from(true, df, dm))) {
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y, true);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     for (size_t b0 = 0; b0 < batch; b0 += kMmMaxTokens) {
         const size_t nb = std::min(kMmMaxTokens, batch - b0);
@@ -1886,7 +1909,7 @@ static std::vector<std::string> required_kernels() {
         for (const char* f : {"_d2_w", "_d4_w", "_d2_r", "_d4_r"}) k.push_back("hh_q4k_mmi_t" + std::to_string(t) + f);
     for (const char* f : {"t1_d2_w", "t1_d2_r", "t2_d2_w", "t2_d2_r", "t4_d2_w", "t4_d2_r"})
         k.push_back(std::string("hh_q4k_mmi_gu_") + f);
-    for (const char* f : {"hh_mmg_amax", "hh_mmg_conv", "hh_mmg_sum", "hh_mmg_sum_act", "hh_mmg_moe_conv",
+    for (const char* f : {"hh_mmg_amax", "hh_mmg_conv", "hh_mmg_sum", "hh_mmg_sum_act", "hh_mmg_moe_conv", "hh_mmg_q4_k_f4", "hh_mmg_q4_k_f4_gu",
                           "hh_mmg_moe_s16", "hh_mmg_moe_s16_gu", "hh_mmg_moe_h1", "hh_mmg_moe_h1_gu"})
         k.push_back(f);
     for (const MmgFmt& f : kMmgFmts)
@@ -1984,6 +2007,7 @@ hh_status engine_create(int device, hh_engine** out) {
     if (const char* f = getenv("HAYAI_HIP_MMR")) e->mmr = atoi(f) != 0;
     if (const char* f = getenv("HAYAI_HIP_MOE_MMG_MIN")) e->moe_mmg_min = atof(f);
     if (const char* f = getenv("HAYAI_HIP_MMG")) e->mmg = atoi(f) != 0;
+    if (const char* f = getenv("HAYAI_HIP_MMF_MIN")) e->mmf_min = (size_t)std::max(65, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_MIN")) e->mmi_min = (size_t)std::max(2, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_D")) e->mmi_d = atoi(f);
     err = hipMalloc(&e->grid_sync, kBarBytes);

@@ -176,6 +176,7 @@ struct hh_engine {
     // 166 : 205; 64 experts 1024 x 1280 4 pairs 76 : 80; 16 experts 1024 x 512 4 pairs 41 : 33,
     // 6 pairs 41 : 40, 8 pairs 42 : 45.
     double moe_mmg_min = 6;
+    size_t mmf_min = 0;         // HAYAI_HIP_MMF_MIN: all-Q4_K batches from which tokens are f16 (0: by the weights)
     size_t mmi_min = 17;        // HAYAI_HIP_MMI_MIN: fewest tokens per pass on the int8 kernels (>= 2)
     int mmi_d = 0;              // HAYAI_HIP_MMI_D: ring depth of the int8 f16-MFMA kernels (0: chosen)
     int blocks_per_cu_override = 0;  // HAYAI_HIP_BLOCKS_PER_CU
@@ -286,15 +287,19 @@ struct hh_engine {
     // Many tokens on the matrix cores, any format (mmg.hip).  HH_ERR_UNSUPPORTED_DEVICE (before
     // any launch) when shape, type or alignment does not fit or the workspaces cannot be had.
     bool mmg_ok(int type, size_t m, size_t n, const void* w) const;
-    hh_status mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus, int count);
+    hh_status mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus, int count,
+                       bool single);
     // x [b][n] -> stages of `type`'s order (h: x is gate/up's output, its
     // largest magnitudes known by so many row groups)
-    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h);
+    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h, bool single);
     // the product of the staged tokens: GEMM (w1 null) into y [b][m], or gate/up + act into y
     hh_status mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b, float* y,
-                          int act, bool h);
-    hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y);
-    hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y);
+                          int act, bool h, bool single);
+    // single: one f16 per token element (Q4_K)
+    hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y,
+                               bool single);
+    hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y,
+                              bool single);
     // MoE routing of T tokens (device pointers) and the grouped expert FFN.
     hh_status enqueue_moe_route(const hh_moe_desc* d, const float* logits, const float* bias, size_t T,
                                 int32_t* ids, float* wts);

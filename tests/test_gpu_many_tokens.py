@@ -110,3 +110,76 @@ def test_in_place_and_unaligned_activations(engine):
     buf.write(X, 4)
     engine.ffn_batched_dev(desc, pack, 0, buf, 4, batch, buf, 4)
     np.testing.assert_array_equal(buf.read(np.float32, X.size, 4).reshape(X.shape), want)
+
+
+# ---- all-Q4_K batches past 64 tokens: one f16 per activation -----------------------------
+
+
+@pytest.fixture(scope="module")
+def f16_engine():
+    import os
+    os.environ["HAYAI_HIP_MMF_MIN"] = "65"  # small shapes too
+    try:
+        eng = hayai_amd.HipEngine(0)
+    finally:
+        del os.environ["HAYAI_HIP_MMF_MIN"]
+    yield eng
+    eng.close()
+
+
+def parts(w, m, n):
+    """Q4_K weights in 64 bits, and per weight the error that a product with |x| may have: over
+    |d sc q| and |dmin m| apart (they cancel in w), f16 rounds x by at most 2^-11 of it, the
+    minima's 16-bit factors and sums of 32 x by 2^-14; f32 additions and unit changes as above."""
+    W = oracle.dequant(Q4_K, w, m * n).reshape(m, n).astype(np.float64)
+    nomin = w.reshape(-1, 144).copy()
+    nomin[:, 2:4] = 0
+    A = oracle.dequant(Q4_K, nomin.reshape(-1), m * n).reshape(m, n).astype(np.float64)
+    a, b = np.abs(A), np.abs(A - W)
+    return W, a * 2.0 ** -11 + b * 2.0 ** -14 + (a + b) * (n / 8) * 2.0 ** -23
+
+
+@pytest.mark.parametrize("m,n,batch", [(1, 256, 65), (300, 256, 128), (257, 768, 129), (512, 2304, 200),
+                                       (40, 14336, 97), (256, 512, 1100)])
+@pytest.mark.parametrize("blocks", ["plain", "zero d", "small d"])
+def test_f16_products(f16_engine, m, n, batch, blocks):
+    print(f"[case] f16 tokens m={m} n={n} batch={batch} {blocks}", flush=True)
+    w = synth.matrix(Q4_K, m, n, 61).reshape(-1, 144).copy()
+    some = np.random.default_rng(62).random(len(w)) < 0.4
+    if blocks == "zero d":  # the accumulator's unit stays the one before (or 1)
+        w[some, 0:2] = 0
+    if blocks == "small d":  # units 2^-24 beside ordinary ones, the minima as they were
+        w[some, 0:2] = [1, 0]
+    w = w.reshape(-1)
+    X = synth.normal(63, batch * n).reshape(batch, n)
+    X[1] *= np.float32(1e20)
+    X[2] = 0
+    Y = f16_engine.ggml_gemv_batched_q4_k(m, n, w, X, batch).reshape(batch, m)
+    W, wide = parts(w, m, n)
+    X = X.astype(np.float64)
+    bound = np.abs(X) @ wide.T + 1e-300
+    worst = float(np.max(np.abs(Y - X @ W.T) / bound))
+    print(f"  worst error / bound {worst:.3e}", flush=True)
+    assert np.isfinite(Y).all() and worst <= 1.0
+
+
+@pytest.mark.parametrize("d_model,d_ff,batch,act", [(256, 512, 65, 0), (512, 768, 130, 1), (768, 1280, 257, 0)])
+def test_f16_ffn(f16_engine, d_model, d_ff, batch, act):
+    print(f"[case] f16 tokens ffn {d_model}x{d_ff} batch={batch}", flush=True)
+    lay, ws, pack = make_pack(f16_engine, (Q4_K,) * 3, d_model, d_ff, 64)
+    desc = f16_engine.ffn_desc((Q4_K,) * 3, d_model, d_ff, lay, act)
+    X = synth.normal(65, batch * d_model).reshape(batch, d_model)
+    Y = f16_engine.ffn_batched(desc, pack, 0, X)
+    # the products' bounds carried through: |act'| <= 1.13, h's own rounding is in the last
+    (G, eg), (U, eu), (D, ed) = (parts(w, r, c) for w, (r, c) in
+                                 zip(ws, [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]))
+    X = X.astype(np.float64)
+    g, u, ax = X @ G.T, X @ U.T, np.abs(X)
+    inner = np.sqrt(2 / np.pi) * (g + 0.044715 * g ** 3)
+    f = 0.5 * g * (1 + np.tanh(inner)) if act else g / (1 + np.exp(-g))
+    dg, du = ax @ eg.T, ax @ eu.T
+    dh = 1.13 * dg * (np.abs(u) + du) + np.abs(f) * du
+    bound = dh @ np.abs(D).T + (np.abs(f * u) + dh) @ ed.T
+    worst = float(np.max(np.abs(Y - (f * u) @ D.T) / bound))
+    print(f"  worst error / bound {worst:.3e}", flush=True)
+    assert worst <= 1.0
