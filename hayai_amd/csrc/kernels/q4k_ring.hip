@@ -417,8 +417,10 @@ HH_DEV void hh_dn_ring_body(const hh_dnr_args& a) {
     const uint8_t* const wdp = a.wd;
     const typename F::lane_t lo = F::lane(u2);
     auto issue = [&](uint32_t k, typename F::data& s) {  // item k: local row team2 + k*TPW2
+        // padding re-reads the first row; a workgroup past the rows (fewer rows than workgroups)
+        // has none, and reads the last
         const uint32_t rl = team2 + k * TPW2;
-        F::issue(wdp + (size_t)drow(rl < nrows ? rl : 0u) * a.rb2, lo, s);  // padding re-reads the first row
+        F::issue(wdp + (size_t)min(drow(rl < nrows ? rl : 0u), dm - 1u) * a.rb2, lo, s);
     };
 
     // F::DIRECT_H (Q4_K, IQ): every compute lane loads its own unit's digits of the
