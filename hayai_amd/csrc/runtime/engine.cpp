@@ -277,8 +277,54 @@ hh_status hh_engine::enqueue_lut(size_t m, size_t n, const uint8_t* w, const flo
     return launch(f, (uint32_t)grid, 256, a);
 }
 
+// Must match struct hh_bst_args in kernels/block_stream.hip.
+struct BstArgs {
+    const uint8_t* w0;
+    const uint8_t* w1;
+    const float* x;
+    const float* norm;
+    const float* res;
+    float* y;
+    uint64_t row_bytes;
+    uint32_t m, n, waves, sb, depth, pad;
+    float eps;
+    int32_t act;
+};
+
+// One token through a Q8_0 / Q4_0 matrix (gate and up with w1) as a row stream through LDS
+// (block_stream.hip); rows of up to 1024 blocks whose x fits LDS beside two items a wave.
+hh_status hh_engine::enqueue_bst(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, const float* x,
+                                 float* y, int act, const float* norm, float eps, const float* res) {
+    const bool gu = w1 != nullptr;
+    if (!block_stream || (type != HH_TYPE_Q8_0 && type != HH_TYPE_Q4_0) || n % 32 || m > UINT32_MAX / 2 ||
+        (((uintptr_t)w0 | (uintptr_t)w1) & 1u) || (((uintptr_t)x | (uintptr_t)norm) & 15u) || ((uintptr_t)y & 3u))
+        return HH_ERR_UNSUPPORTED_DEVICE;
+    const size_t bb = type == HH_TYPE_Q8_0 ? 34 : 18, nblk = n / 32, rb = nblk * bb;
+    if (m * rb * (gu ? 2 : 1) < block_stream_min) return HH_ERR_UNSUPPORTED_DEVICE;
+    size_t W = 1;
+    while (W < 8 && W * 128 < nblk) W *= 2;
+    const size_t sb = (nblk + W - 1) / W;
+    if (sb > 128) return HH_ERR_UNSUPPORTED_DEVICE;
+    const bool pair = sb <= 64;
+    const size_t G = (size_t)props.multiProcessorCount, rows_max = (m + G - 1) / G;
+    const size_t fixed = nblk * 144 + rows_max * (gu ? 2 : 1) * W * 4 + 32, slot = (pair ? 2 : 1) * ((sb * bb + 45) & ~size_t(15));
+    const size_t lds = (size_t)props.sharedMemPerBlock - 64;  // less the static words
+    size_t depth = 4;
+    while (depth >= 2 && 8 * depth * slot + fixed > lds) depth--;
+    if (depth < 2) return HH_ERR_UNSUPPORTED_DEVICE;
+    hipFunction_t fn;
+    HH_TRY(kernel(std::string("hh_bst_") + format_of(type)->name + (pair ? "_pair" : "_wide") + (gu ? "_gu" : ""), &fn));
+    BstArgs a{w0, gu ? w1 : w0, x, norm, res, y, rb, (uint32_t)m, (uint32_t)n, (uint32_t)W, (uint32_t)sb,
+              (uint32_t)depth, 0, eps, act};
+    void* params[] = {&a};
+    HH_TRY_HIP(hipModuleLaunchKernel(fn, (uint32_t)G, 1, 1, 768, 1, 1, (unsigned)(8 * depth * slot + fixed), stream,
+                                     params, nullptr),
+               "hipModuleLaunchKernel(block stream)");
+    return HH_OK;
+}
+
 hh_status hh_engine::enqueue_gemv(int type, size_t m, size_t n, const uint8_t* w, const float* x, float* y,
-                                  void* xq_ws) {
+                                  void* xq_ws, bool stream_ok) {
     const Format* f = format_of(type);
     if (!f) return fail(HH_ERR_KERNEL_MISSING, "no GEMV kernel for GGML type %d", type);
     size_t rb;
@@ -298,6 +344,10 @@ hh_status hh_engine::enqueue_gemv(int type, size_t m, size_t n, const uint8_t* w
     }
     if (type == HH_TYPE_Q6_K || type == HH_TYPE_IQ2_XXS || type == HH_TYPE_IQ3_XXS) {
         hh_status st = enqueue_ring_gemv(type, m, n, w, x, y, xq_ws);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
+    if (stream_ok) {
+        const hh_status st = enqueue_bst(type, m, n, w, nullptr, x, y, 0, nullptr, 0.f, nullptr);
         if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     std::string name;
@@ -330,13 +380,18 @@ hh_status hh_engine::enqueue_gemv(int type, size_t m, size_t n, const uint8_t* w
 }
 
 hh_status hh_engine::enqueue_gateup(int tg, int tu, size_t d_ff, size_t d_model, const uint8_t* wg,
-                                    const uint8_t* wu, const float* x, float* h, int act, float* gu_ws) {
+                                    const uint8_t* wu, const float* x, float* h, int act, float* gu_ws,
+                                    bool stream_ok) {
     const Format* f = format_of(tg);
     if (!f || !format_of(tu)) return fail(HH_ERR_KERNEL_MISSING, "no GEMV kernel for GGML type %d/%d", tg, tu);
     size_t rb;
     HH_TRY(row_bytes(tg, d_model, &rb));
     if (tg == HH_TYPE_Q4_K && tu == HH_TYPE_Q4_K) {
         hh_status st = enqueue_q4k(d_ff, d_model, wg, wu, x, h, act, true, nullptr, nullptr);
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
+    if (tg == tu && stream_ok) {
+        const hh_status st = enqueue_bst(tg, d_ff, d_model, wg, wu, x, h, act, nullptr, 0.f, nullptr);
         if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     if (tg == tu && f->fused_gateup) {
@@ -612,6 +667,21 @@ hh_status hh_engine::enqueue_ffn_begin(const hh_ffn_desc* d, const uint8_t* pack
         ffn_calls += 2;
         return HH_OK;
     }
+    // (layers of the one-launch FFN keep its arithmetic: the team kernels)
+    const bool stream_ok = !small_layer(d);
+    if (norm && stream_ok && d->type_gate == d->type_up && !((uintptr_t)x & 3u)) {
+        // the Q8_0 / Q4_0 row stream normalizes x as it brings it in
+        st = enqueue_bst(d->type_gate, d->d_ff, d->d_model, wg, wu, x, (float*)ws_h, d->act, norm, eps, nullptr);
+        if (st == HH_OK) {
+            ffn_stage = *d;
+            ffn_stage_digits = false;
+            ffn_stage_ring = false;
+            ffn_stage_valid = true;
+            ffn_calls += 2;
+            return HH_OK;
+        }
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
     if (norm) {
         // other layouts: RMSNorm as its own kernel, then the plain begin step on its output
         HH_TRY(grow(&ws_xn, &ws_xn_cap, d->d_model * sizeof(float)));
@@ -628,7 +698,7 @@ hh_status hh_engine::enqueue_ffn_begin(const hh_ffn_desc* d, const uint8_t* pack
         digits = st == HH_OK;
     }
     if (st == HH_ERR_UNSUPPORTED_DEVICE)
-        st = enqueue_gateup(d->type_gate, d->type_up, d->d_ff, d->d_model, wg, wu, x, (float*)ws_h, d->act);
+        st = enqueue_gateup(d->type_gate, d->type_up, d->d_ff, d->d_model, wg, wu, x, (float*)ws_h, d->act, nullptr, stream_ok);
     if (st != HH_OK) return st;
     ffn_stage = *d;
     ffn_stage_digits = digits;
@@ -648,6 +718,12 @@ hh_status hh_engine::enqueue_ffn_finish(const hh_ffn_desc* d, const uint8_t* pac
         if (st == HH_OK) ffn_calls += 1;
         return st;
     }
+    if (res && !small_layer(d) && !ffn_stage_digits && !((uintptr_t)y & 3u)) {
+        const hh_status st = enqueue_bst(d->type_down, d->d_model, d->d_ff, wd, nullptr, (const float*)ws_h, y, 0, nullptr,
+                                         0.f, res);
+        if (st == HH_OK) ffn_calls += 1;
+        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    }
     float* out = y;
     if (res) {
         HH_TRY(grow(&ws_f, &ws_f_cap, d->d_model * sizeof(float)));
@@ -655,7 +731,8 @@ hh_status hh_engine::enqueue_ffn_finish(const hh_ffn_desc* d, const uint8_t* pac
     }
     hh_status st = HH_ERR_UNSUPPORTED_DEVICE;
     if (ffn_stage_digits) st = enqueue_q4k(d->d_model, d->d_ff, wd, nullptr, nullptr, out, 0, false, ws_hq, nullptr);
-    if (st == HH_ERR_UNSUPPORTED_DEVICE) st = enqueue_gemv(d->type_down, d->d_model, d->d_ff, wd, (const float*)ws_h, out);
+    if (st == HH_ERR_UNSUPPORTED_DEVICE) st = enqueue_gemv(d->type_down, d->d_model, d->d_ff, wd, (const float*)ws_h, out, nullptr,
+                                                         !small_layer(d));
     if (st != HH_OK) return st;
     ffn_calls += 1;
     if (!res) return HH_OK;
@@ -719,8 +796,8 @@ hh_status hh_engine::enqueue_ffn_noalloc(const hh_ffn_desc* d, const uint8_t* pa
                     dm, df, need, (unsigned)HH_NOALLOC_SCRATCH_BYTES);
     float* h = (float*)ws;
     float* gu = h + df;
-    HH_TRY(enqueue_gateup(d->type_gate, d->type_up, df, dm, wg, wu, x, h, d->act, gu));
-    HH_TRY(enqueue_gemv(d->type_down, dm, df, wd, h, y, (void*)(gu + 2 * df)));
+    HH_TRY(enqueue_gateup(d->type_gate, d->type_up, df, dm, wg, wu, x, h, d->act, gu, !small_layer(d)));
+    HH_TRY(enqueue_gemv(d->type_down, dm, df, wd, h, y, (void*)(gu + 2 * df), !small_layer(d)));
     ffn_calls += 3;
     return HH_OK;
 }
@@ -740,9 +817,9 @@ struct SffnArgs {  // the small FFN kernels' scalar parameters (small_ffn.hip)
 
 static int small_team(size_t units) { return units <= 16 ? 16 : (units <= 32 ? 32 : 64); }
 
-bool hh_engine::small_ffn_shape(const hh_ffn_desc* d) const {
+bool hh_engine::small_layer(const hh_ffn_desc* d) const {
     const size_t dm = d->d_model, df = d->d_ff, G = (size_t)props.multiProcessorCount;
-    return small_ffn && d->type_gate == d->type_up && d->type_up == d->type_down &&
+    return d->type_gate == d->type_up && d->type_up == d->type_down &&
            (d->type_gate == HH_TYPE_Q4_0 || d->type_gate == HH_TYPE_Q8_0) && dm % 32 == 0 && df % 32 == 0 &&
            dm / 32 <= 64 && df / 32 <= 64 && (df + G - 1) / G <= 2 * (256 / (size_t)small_team(dm / 32)) &&
            (dm + G - 1) / G <= 2 * (256 / (size_t)small_team(df / 32));
@@ -755,7 +832,7 @@ hh_status hh_engine::enqueue_small_ffn(const hh_ffn_desc* d, const uint8_t* wg, 
                                        const float* x, float* y) {
     const size_t dm = d->d_model, df = d->d_ff, G = (size_t)props.multiProcessorCount;
     const int t1 = small_team(dm / 32), t2 = small_team(df / 32);
-    if (!small_ffn_shape(d) || (((uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd) & 1u) || ((uintptr_t)x & 3u) ||
+    if (!small_ffn || !small_layer(d) || (((uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd) & 1u) || ((uintptr_t)x & 3u) ||
         ((uintptr_t)y & 3u))
         return HH_ERR_UNSUPPORTED_DEVICE;
     const std::string name = std::string("hh_sffn_") + (d->type_gate == HH_TYPE_Q4_0 ? "q4_0" : "q8_0") + "_t" +
@@ -872,6 +949,11 @@ hh_status hh_engine::enqueue_ffn_block(const hh_ffn_desc* d, const uint8_t* pack
         return HH_OK;
     }
     const size_t dm = d->d_model;
+    if (!small_layer(d)) {
+        // RMSNorm and the residual ride in the two halves where their kernels take them
+        HH_TRY(enqueue_ffn_begin(d, pack, x, norm, eps));
+        return enqueue_ffn_finish(d, pack, y, x);
+    }
     HH_TRY(grow(&ws_xn, &ws_xn_cap, dm * sizeof(float)));
     HH_TRY(grow(&ws_f, &ws_f_cap, dm * sizeof(float)));
     hipFunction_t fn;
@@ -1365,7 +1447,7 @@ hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, 
     const uint8_t* wg = pack + d->gate_off;
     const uint8_t* wu = pack + d->up_off;
     const uint8_t* wd = pack + d->down_off;
-    if (b < (small_ffn_shape(d) ? kMmgMinTokensSmallFfn : kMmgMinTokens) || d->type_gate != d->type_up || !mmg_ok(d->type_gate, df, dm, wg) ||
+    if (b < (small_ffn && small_layer(d) ? kMmgMinTokensSmallFfn : kMmgMinTokens) || d->type_gate != d->type_up || !mmg_ok(d->type_gate, df, dm, wg) ||
         !mmg_ok(d->type_up, df, dm, wu) || !mmg_ok(d->type_down, dm, df, wd))
         return HH_ERR_UNSUPPORTED_DEVICE;
     const int types[] = {d->type_gate, d->type_down};
@@ -1916,6 +1998,8 @@ static std::vector<std::string> required_kernels() {
         for (const char* mode : {"s16", "h1", "h2"})
             for (const char* gu : {"", "_gu"})
                 k.push_back(std::string("hh_mmg_") + format_of(f.type)->name + "_" + mode + gu);
+    for (const char* f : {"hh_bst_q8_0", "hh_bst_q4_0"})
+        for (const char* v : {"_pair", "_wide", "_pair_gu", "_wide_gu"}) k.push_back(std::string(f) + v);
     k.push_back("hh_lut_gemv");
     for (const char* f : {"gu_ring_g1", "gu_ring_g2", "gu_ring_g1_n", "gu_ring_g2_n", "dn_ring_d1", "dn_ring_d2", "dn_ring_d4", "dn_ring_d8"})
         k.push_back(std::string("hh_q4k_") + f);
@@ -2007,6 +2091,8 @@ hh_status engine_create(int device, hh_engine** out) {
     if (const char* f = getenv("HAYAI_HIP_MMR")) e->mmr = atoi(f) != 0;
     if (const char* f = getenv("HAYAI_HIP_MOE_MMG_MIN")) e->moe_mmg_min = atof(f);
     if (const char* f = getenv("HAYAI_HIP_MMG")) e->mmg = atoi(f) != 0;
+    if (const char* f = getenv("HAYAI_HIP_BLOCK_STREAM")) e->block_stream = atoi(f) != 0;
+    if (const char* f = getenv("HAYAI_HIP_BLOCK_STREAM_MIN")) e->block_stream_min = (size_t)atoll(f);
     if (const char* f = getenv("HAYAI_HIP_MMF_MIN")) e->mmf_min = (size_t)std::max(65, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_MIN")) e->mmi_min = (size_t)std::max(2, atoi(f));
     if (const char* f = getenv("HAYAI_HIP_MMI_D")) e->mmi_d = atoi(f);

@@ -170,6 +170,10 @@ struct hh_engine {
     int ring_dn_per_cu = 1;     // HAYAI_HIP_RING_DN_PER_CU: ring down workgroups per CU
     bool mmr = true;            // HAYAI_HIP_MMR=0: batched Q4_K (<= 16 tokens) one token at a time
     bool mmq = true;            // HAYAI_HIP_MMQ=0: batched Q4_K (>= 17 tokens) one token at a time, no int8
+    bool block_stream = true;   // HAYAI_HIP_BLOCK_STREAM=0: one-token Q8_0 / Q4_0 on the team kernels only
+    // HAYAI_HIP_BLOCK_STREAM_MIN: weight bytes from which it is used (Q8_0 300 x 512 5.1 us both
+    // ways, 1024 x 1024 5.6 us against 7.6)
+    size_t block_stream_min = (size_t)256 << 10;
     bool mmg = true;            // HAYAI_HIP_MMG=0: other formats' batches one token at a time
     // HAYAI_HIP_MOE_MMG_MIN: (token, slot) pairs per expert from which MoE runs on mmg.hip.
     // Against the grouped gather-GEMV, us: 128 experts 2048 x 768 4 pairs 161 : 148, 6.2 pairs
@@ -211,15 +215,21 @@ struct hh_engine {
 
     // Enqueue one GEMV y = W . x on the compute stream (all pointers device-visible).
     // xq_ws: room for a Q6_K GEMV's x digits (hh_ring_digits_bytes(n)); null: ws_xq.
+    // stream_ok: Q8_0 / Q4_0 may take the row stream (enqueue_bst).
     hh_status enqueue_gemv(int type, size_t m, size_t n, const uint8_t* w, const float* x, float* y,
-                           void* xq_ws = nullptr);
+                           void* xq_ws = nullptr, bool stream_ok = true);
+    // Q8_0 / Q4_0 matrix of one token as a row stream (block_stream.hip); w1: gate/up, with norm on
+    // RMSNorm(x); res: y = res + W . x.  HH_ERR_UNSUPPORTED_DEVICE when it does not fit.
+    hh_status enqueue_bst(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, const float* x, float* y,
+                          int act, const float* norm, float eps, const float* res);
     // Enqueue the fused or unfused gate/up + activation into h.
     // gu_ws: room for the unfused form's gate and up outputs (2 * d_ff floats, then the
     // GEMVs' x digits); null: ws_g / ws_u (/ ws_xq).
     hh_status enqueue_gateup(int type_g, int type_u, size_t d_ff, size_t d_model, const uint8_t* wg,
-                             const uint8_t* wu, const float* x, float* h, int act, float* gu_ws = nullptr);
+                             const uint8_t* wu, const float* x, float* h, int act, float* gu_ws = nullptr,
+                             bool stream_ok = true);
     hh_status enqueue_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, float* y);
-    bool small_ffn_shape(const hh_ffn_desc* d) const;  // the layer fits the one-launch FFN
+    bool small_layer(const hh_ffn_desc* d) const;  // the layer fits the one-launch FFN
     hh_status enqueue_small_ffn(const hh_ffn_desc* d, const uint8_t* wg, const uint8_t* wu, const uint8_t* wd,
                                 const float* x, float* y);
     hh_status enqueue_ffn_block(const hh_ffn_desc* d, const uint8_t* pack, const float* x, const float* norm,
