@@ -7,7 +7,7 @@
 // What bounds it: the weight stream.  The blocks are 34 and 18 bytes, and a lane that loads its
 // own block (gemv.hip) asks for 64 pieces at that stride, misaligned: the address units, not HBM,
 // set the pace (8B Q8_0 gate/up 41 us, 3.0 TB/s, here 28 us; down 30 us, 2.1 TB/s, here 16 us; a
-// block with RMSNorm and residual 78 -> 44 us, Q4_0 65 -> 33 us).  Here a wave copies a
+// block with RMSNorm and residual 78 -> 45 us, Q4_0 65 -> 35 us).  Here a wave copies a
 // whole row slice, 16 bytes per lane and contiguous, into its own LDS ring by global->LDS DMA
 // (no registers held, D rows in flight), and each lane then takes its two blocks from LDS: the
 // dwords that cover them and one v_alignbit each.  Rows start at any even address: a copy begins

@@ -698,7 +698,8 @@ hh_status hh_engine::enqueue_ffn_begin(const hh_ffn_desc* d, const uint8_t* pack
         digits = st == HH_OK;
     }
     if (st == HH_ERR_UNSUPPORTED_DEVICE)
-        st = enqueue_gateup(d->type_gate, d->type_up, d->d_ff, d->d_model, wg, wu, x, (float*)ws_h, d->act, nullptr, stream_ok);
+        st = enqueue_gateup(d->type_gate, d->type_up, d->d_ff, d->d_model, wg, wu, x, (float*)ws_h, d->act, nullptr,
+                            stream_ok);
     if (st != HH_OK) return st;
     ffn_stage = *d;
     ffn_stage_digits = digits;
@@ -731,8 +732,8 @@ hh_status hh_engine::enqueue_ffn_finish(const hh_ffn_desc* d, const uint8_t* pac
     }
     hh_status st = HH_ERR_UNSUPPORTED_DEVICE;
     if (ffn_stage_digits) st = enqueue_q4k(d->d_model, d->d_ff, wd, nullptr, nullptr, out, 0, false, ws_hq, nullptr);
-    if (st == HH_ERR_UNSUPPORTED_DEVICE) st = enqueue_gemv(d->type_down, d->d_model, d->d_ff, wd, (const float*)ws_h, out, nullptr,
-                                                         !small_layer(d));
+    if (st == HH_ERR_UNSUPPORTED_DEVICE)
+        st = enqueue_gemv(d->type_down, d->d_model, d->d_ff, wd, (const float*)ws_h, out, nullptr, !small_layer(d));
     if (st != HH_OK) return st;
     ffn_calls += 1;
     if (!res) return HH_OK;
@@ -949,8 +950,9 @@ hh_status hh_engine::enqueue_ffn_block(const hh_ffn_desc* d, const uint8_t* pack
         return HH_OK;
     }
     const size_t dm = d->d_model;
-    if (!small_layer(d)) {
-        // RMSNorm and the residual ride in the two halves where their kernels take them
+    if (!small_layer(d) && d->type_gate == d->type_up && (d->type_gate == HH_TYPE_Q8_0 || d->type_gate == HH_TYPE_Q4_0)) {
+        // the row stream takes RMSNorm and the residual along (other formats: the FFN kernels
+        // choose by the alignment of the normalized workspace below, not of x)
         HH_TRY(enqueue_ffn_begin(d, pack, x, norm, eps));
         return enqueue_ffn_finish(d, pack, y, x);
     }
@@ -1447,8 +1449,8 @@ hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, 
     const uint8_t* wg = pack + d->gate_off;
     const uint8_t* wu = pack + d->up_off;
     const uint8_t* wd = pack + d->down_off;
-    if (b < (small_ffn && small_layer(d) ? kMmgMinTokensSmallFfn : kMmgMinTokens) || d->type_gate != d->type_up || !mmg_ok(d->type_gate, df, dm, wg) ||
-        !mmg_ok(d->type_up, df, dm, wu) || !mmg_ok(d->type_down, dm, df, wd))
+    if (b < (small_ffn && small_layer(d) ? kMmgMinTokensSmallFfn : kMmgMinTokens) || d->type_gate != d->type_up ||
+        !mmg_ok(d->type_gate, df, dm, wg) || !mmg_ok(d->type_up, df, dm, wu) || !mmg_ok(d->type_down, dm, df, wd))
         return HH_ERR_UNSUPPORTED_DEVICE;
     const int types[] = {d->type_gate, d->type_down};
     const size_t ms[] = {df, dm}, ns[] = {dm, df};
