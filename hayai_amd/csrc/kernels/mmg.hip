@@ -31,11 +31,11 @@
 // shared by the workgroup's four waves.  A wave owns 64 weight rows (32 of gate and the same 32
 // of up), so each 1 KB token fragment read from LDS feeds two MFMAs.
 //
-// Modes (chosen by the token count alone, plan_mmg): h<TT>: TT tiles of 32 tokens, hi and lo as two MFMAs; s16: 16 tokens, hi in A rows
-// 0..15 and lo in rows 16..31 of one MFMA, added at the end.
+// Modes (chosen by the token count alone, plan_mmg): h<TT>: TT tiles of 32 tokens, hi and lo as
+// two MFMAs; s16: 16 tokens, hi in A rows 0..15 and lo in rows 16..31 of one MFMA, added at the end.
 //
 // What bounds it: at hundreds of tokens the matrix cores with the weight decode beside them (8B
-// FFN, 512 tokens, 2 x 180 GFLOP of hi and lo: 0.52 ms IQ2_XXS .. 0.78 ms Q8_0, 460 .. 690 TFLOP/s;
+// FFN, 512 tokens, 2 x 180 GFLOP of hi and lo: 0.44 ms IQ2_XXS .. 0.72 ms Q8_0, 500 .. 820 TFLOP/s;
 // one token at a time these took 12 .. 39 ms); at 4..16 tokens the weight stream's latency (8B
 // Q6_K FFN, 16 tokens: 106 us against 779 us).
 //
@@ -47,9 +47,6 @@
 // 0..7, half 1: lo).
 typedef float hh_f16v __attribute__((ext_vector_type(16)));
 
-#ifndef HH_MMG_VALU
-#define HH_MMG_VALU 0
-#endif
 enum { HH_MMG_H = 0, HH_MMG_S16 = 1, HH_MMG_F = 2 };
 
 struct hh_mmg_args {
@@ -116,30 +113,87 @@ struct hh_mmg_k {
 };
 
 // ---- weight formats -------------------------------------------------------------------
-// Raw: one chunk's bytes of one row as loaded (ready: what is taken from them once); load(p, ch, ...) of chunk ch of the row at p
-// (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
+// Raw: one chunk's bytes of one row as loaded (ready: what is taken from them once); load(p, ch,
+// ...) of chunk ch of the row at p (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
 // the d of the block that group g closes.  NB: B operands per step.
-struct hh_mmg_q4_0 {
-    static constexpr bool SUPER = false, MINS = false, TABLES = false;
-    static constexpr int NB = 1;
-    struct Raw {
-        uint2 q[4];
-        uint32_t d[4];
-    };
-    template <uint32_t HALF>
-    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
+// The 32-column formats: lane half h loads the two whole blocks 4 ch + 2 h, + 1 (consecutive
+// bytes: 3 loads for Q4_0, 5 for Q8_0, where a load of each half block and each d took 8), and
+// `ready` exchanges halves with the lane of the same row: then every lane has its half of all four.
+// With its 64 lanes in 64 places every load holds the address unit for as long as 64 lines take.
+// 8B FFN: 512 tokens Q8_0 888 -> 717 us, Q4_0 593 -> 455 us; 16 tokens Q4_0 92 -> 72 us.
+HH_DEV void hh_swap32(uint32_t& a, uint32_t& b) {  // a's upper 32 lanes with b's lower 32
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// Two blocks of QW code dwords each: w[0] low half d of the first, then its codes at half a dword,
+// w[QW] high half d of the second, then its codes.  After `ready` w[0 ..] groups 0, 2, w[QW] and dx
+// the four d, w[QW + 1 ..] groups 1, 3 (in place: a copy stays live beside it and spills).
+template <uint32_t QW>
+struct hh_mmg_pair {
+    static constexpr uint32_t BB = 4 * QW + 2;
+    uint32_t w[2 * QW + 1], dx;
+    HH_DEV static void put(uint32_t* o, uint4 v) { o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w; }
+    HH_DEV void load(const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
+        const uint32_t k = 4 * ch + 2 * h;
+        if (4 * ch + 4 <= nblk) {
+            const uint8_t* b = p + k * BB;
 #pragma unroll
-        for (uint32_t g = 0; g < 4; g++) {
-            const uint32_t k = 4 * ch + g;
-            const uint8_t* b = p + min(k, nblk - 1) * 18u;
-            r.q[g] = hh_ldu8(b + 2 + 8 * h);
-            r.d[g] = k < nblk ? hh_ld_u16(b) : 0u;
+            for (uint32_t i = 0; i < QW / 2; i++) put(w + 4 * i, hh_ldu16(b + 16 * i));
+            w[2 * QW] = hh_ldu4(b + 8 * QW);
+        } else {  // the row's end: block by block, d = 0 past it
+            uint32_t c[2][QW], d[2];
+#pragma unroll
+            for (uint32_t i = 0; i < 2; i++) {
+                const uint8_t* b = p + min(k + i, nblk - 1) * BB;
+                d[i] = k + i < nblk ? hh_ld_u16(b) : 0u;
+#pragma unroll
+                for (uint32_t j = 0; j < QW; j += 4) put(c[i] + j, hh_ldu16(b + 2 + 4 * j));
+            }
+            w[0] = d[0] | c[0][0] << 16;
+#pragma unroll
+            for (uint32_t i = 1; i < QW; i++) w[i] = __builtin_amdgcn_alignbit(c[0][i], c[0][i - 1], 16);
+            w[QW] = c[0][QW - 1] >> 16 | d[1] << 16;
+#pragma unroll
+            for (uint32_t i = 0; i < QW; i++) w[QW + 1 + i] = c[1][i];
         }
     }
-    HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
+    HH_DEV void ready() {
+        const uint32_t d = (w[0] & 0xFFFFu) | (w[QW] & 0xFFFF0000u);
+#pragma unroll
+        for (uint32_t i = 0; i < QW; i++) w[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], 16);
+        w[QW] = dx = d;
+        hh_swap32(w[QW], dx);
+#pragma unroll
+        for (uint32_t i = 0; i < QW / 2; i++) {
+            hh_swap32(w[i], w[QW / 2 + i]);
+            hh_swap32(w[QW + 1 + i], w[QW + 1 + QW / 2 + i]);
+        }
+    }
+    HH_DEV uint32_t code(int g, int i) const { return w[(g & 1 ? QW + 1 : 0) + (g & 2 ? QW / 2 : 0) + i]; }
+    HH_DEV float scale(int g) const {
+        const uint32_t d = g & 2 ? dx : w[QW];
+        return hh_f16(g & 1 ? d >> 16 : d & 0xFFFFu);
+    }
+};
+
+struct hh_mmg_q4_0 {
+    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true;
+    static constexpr int NB = 1;
+    typedef hh_mmg_pair<4> Raw;
+    template <uint32_t HALF>
+    HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
+        r.load(p, ch, h, nblk);
+    }
+    template <uint32_t HALF>
+    HH_DEV static void ready(Raw& r) {
+        r.ready();
+    }
+    HH_DEV static float scale(const Raw& r, int g) { return r.scale(g); }
     template <uint32_t HALF>
     HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
-        const uint32_t v[4] = {r.q[g].x, r.q[g].x >> 8, r.q[g].y, r.q[g].y >> 8};
+        const uint32_t v[4] = {r.code(g, 0), r.code(g, 0) >> 8, r.code(g, 1), r.code(g, 1) >> 8};
         hh_h2 o[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -154,26 +208,21 @@ struct hh_mmg_q4_0 {
 };
 
 struct hh_mmg_q8_0 {
-    static constexpr bool SUPER = false, MINS = false, TABLES = false;
+    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true;
     static constexpr int NB = 1;
-    struct Raw {
-        uint4 q[4];
-        uint32_t d[4];
-    };
+    typedef hh_mmg_pair<8> Raw;
     template <uint32_t HALF>
     HH_DEV static void load(Raw& r, const uint8_t* p, uint32_t ch, uint32_t h, uint32_t nblk) {
-#pragma unroll
-        for (uint32_t g = 0; g < 4; g++) {
-            const uint32_t k = 4 * ch + g;
-            const uint8_t* b = p + min(k, nblk - 1) * 34u;
-            r.q[g] = hh_ldu16(b + 2 + 16 * h);
-            r.d[g] = k < nblk ? hh_ld_u16(b) : 0u;
-        }
+        r.load(p, ch, h, nblk);
     }
-    HH_DEV static float scale(const Raw& r, int g) { return hh_f16(r.d[g]); }
+    template <uint32_t HALF>
+    HH_DEV static void ready(Raw& r) {
+        r.ready();
+    }
+    HH_DEV static float scale(const Raw& r, int g) { return r.scale(g); }
     template <uint32_t HALF>
     HH_DEV static void frag(const Raw& r, int g, int s, uint32_t, const char*, const hh_mmg_k& k, hh_h8* f) {
-        const uint32_t a = (s ? r.q[g].z : r.q[g].x) ^ 0x80808080u, b = (s ? r.q[g].w : r.q[g].y) ^ 0x80808080u;
+        const uint32_t a = r.code(g, 2 * s) ^ 0x80808080u, b = r.code(g, 2 * s + 1) ^ 0x80808080u;
         const hh_h2 z = hh_h2_all(1152.f);  // 1024 + (q + 128)
         f[0] = hh_h8_of(hh_bytes_h2<0, 1>(a) - z, hh_bytes_h2<2, 3>(a) - z, hh_bytes_h2<0, 1>(b) - z,
                         hh_bytes_h2<2, 3>(b) - z);
@@ -181,7 +230,7 @@ struct hh_mmg_q8_0 {
 };
 
 struct hh_mmg_q4_k {
-    static constexpr bool SUPER = true, MINS = true, TABLES = false;
+    static constexpr bool SUPER = true, MINS = true, TABLES = false, READY = true;
     static constexpr int NB = 1;
     struct Raw {
         uint4 q[2];
@@ -228,7 +277,7 @@ struct hh_mmg_q4_k {
 };
 
 struct hh_mmg_q6_k {
-    static constexpr bool SUPER = true, MINS = false, TABLES = false;
+    static constexpr bool SUPER = true, MINS = false, TABLES = false, READY = false;
     static constexpr int NB = 2;
     struct Raw {
         uint4 a, b, qh;
@@ -319,7 +368,7 @@ HH_DEV hh_h8 hh_mmg_iq_frag(uint4 grid, uint4 sign, uint32_t aux) {
 }
 
 struct hh_mmg_iq2_xxs {
-    static constexpr bool SUPER = true, MINS = false, TABLES = true;
+    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq2_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq2_table; }
@@ -346,7 +395,7 @@ struct hh_mmg_iq2_xxs {
 };
 
 struct hh_mmg_iq3_xxs {
-    static constexpr bool SUPER = true, MINS = false, TABLES = true;
+    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq3_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq3_table; }
@@ -776,7 +825,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     auto compute = [&](typename F::Raw* raw, auto buf_c) {
         constexpr uint32_t buf = decltype(buf_c)::value;
         constexpr bool open = buf == 0, close = buf == 1;
-        if constexpr (F::MINS) {
+        if constexpr (F::READY) {
 #pragma unroll
             for (int q = 0; q < 2; q++) F::template ready<buf>(raw[q]);
         }
@@ -845,16 +894,6 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         }
     };
 
-    // the matrix core's next operands are decoded while it works: one MFMA, then a few others
-    auto interleave = [&]() {
-        constexpr int N = 4 * 2 * 2 * TT * (NA + F::NB - 1);
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, HH_MMG_VALU, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-    };
     typename F::Raw raw[2][2];  // [buffer][row tile]
     constexpr hh_uint_c<0> B0{};
     constexpr hh_uint_c<1> B1{};
@@ -871,7 +910,6 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             for (int q = 0; q < 2; q++) F::template load<1>(raw[1][q], wp[q], ch + 1, h, nblk);
         }
         compute(raw[0], B0);
-        if (HH_MMG_VALU) interleave();
         if (!two) break;
         hh_mmg_sync();
         if (ch + 2 < c1) {
@@ -880,7 +918,6 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], ch + 2, h, nblk);
         }
         compute(raw[1], B1);
-        if (HH_MMG_VALU) interleave();
     }
 
     hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci);
