@@ -27,8 +27,8 @@
 // are contiguous in the block, and the stage is written in the order that gives:
 //   columns 16 h + 8 step + e  (Q8_0, Q4_K, Q6_K, IQ)   or   16 step + 8 h + e  (Q4_0),
 //   e natural (Q8_0, IQ) or 0 2 1 3 4 6 5 7 (nibble pairs of a dword).
-// Weights go from global memory to registers to the matrix core; only tokens pass through LDS,
-// shared by the workgroup's four waves.  A wave owns 64 weight rows (32 of gate and the same 32
+// Weights go from global memory to registers to the matrix core (Q4_K with one token tile by way
+// of LDS, hh_mmg_body); tokens pass through LDS, shared by the workgroup's four waves.  A wave owns 64 weight rows (32 of gate and the same 32
 // of up), so each 1 KB token fragment read from LDS feeds two MFMAs.
 //
 // Modes (chosen by the token count alone, plan_mmg): h<TT>: TT tiles of 32 tokens, hi and lo as
@@ -40,7 +40,7 @@
 // Q6_K FFN, 16 tokens: 106 us against 779 us).
 //
 // MoE (hh_mmg_moe_*): the (token, slot) pairs of an expert in tiles of 16 or 32, one launch over
-// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 259 us a layer.
+// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 246 us a layer.
 //
 // Token stages: [tile][128-column chunk][group 0..3][step 0..1][hi, lo][lane][8 f16], for Q4_K
 // followed after every second chunk by the sums [lane][8 f16] (lane half 0: hi of sub-blocks
@@ -48,6 +48,7 @@
 typedef float hh_f16v __attribute__((ext_vector_type(16)));
 
 enum { HH_MMG_H = 0, HH_MMG_S16 = 1, HH_MMG_F = 2 };
+#define HH_MMG_WSLOT 9216u  // a wave's 64 Q4_K rows of one superblock in LDS
 
 struct hh_mmg_args {
     const uint8_t* w0;       // GEMM: W; gate/up: W_gate
@@ -179,7 +180,7 @@ struct hh_mmg_pair {
 };
 
 struct hh_mmg_q4_0 {
-    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true;
+    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true, ROWS_LDS = false;
     static constexpr int NB = 1;
     typedef hh_mmg_pair<4> Raw;
     template <uint32_t HALF>
@@ -208,7 +209,7 @@ struct hh_mmg_q4_0 {
 };
 
 struct hh_mmg_q8_0 {
-    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true;
+    static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true, ROWS_LDS = false;
     static constexpr int NB = 1;
     typedef hh_mmg_pair<8> Raw;
     template <uint32_t HALF>
@@ -230,7 +231,7 @@ struct hh_mmg_q8_0 {
 };
 
 struct hh_mmg_q4_k {
-    static constexpr bool SUPER = true, MINS = true, TABLES = false, READY = true;
+    static constexpr bool SUPER = true, MINS = true, TABLES = false, READY = true, ROWS_LDS = true;
     static constexpr int NB = 1;
     struct Raw {
         uint4 q[2];
@@ -247,6 +248,13 @@ struct hh_mmg_q4_k {
         r.hd = hh_ld16(b);
         r.q[0] = hh_ld16(b + 16 + 64 * HALF + 16 * h);
         r.q[1] = hh_ld16(b + 48 + 64 * HALF + 16 * h);
+    }
+    // one row's superblock in LDS (both halves' raw)
+    HH_DEV static void load_lds(Raw& r0, Raw& r1, const char* b, uint32_t h) {
+        const uint4* v = reinterpret_cast<const uint4*>(b);
+        r0.hd = r1.hd = v[0];
+        r0.q[0] = v[1 + h], r0.q[1] = v[3 + h];
+        r1.q[0] = v[5 + h], r1.q[1] = v[7 + h];
     }
     HH_DEV static float scale(const Raw& r, int) { return hh_f16(r.hd.x & 0xFFFFu); }
     HH_DEV static float min_scale(const Raw& r) { return hh_f16(r.hd.x >> 16); }
@@ -277,7 +285,7 @@ struct hh_mmg_q4_k {
 };
 
 struct hh_mmg_q6_k {
-    static constexpr bool SUPER = true, MINS = false, TABLES = false, READY = false;
+    static constexpr bool SUPER = true, MINS = false, TABLES = false, READY = false, ROWS_LDS = false;
     static constexpr int NB = 2;
     struct Raw {
         uint4 a, b, qh;
@@ -368,7 +376,7 @@ HH_DEV hh_h8 hh_mmg_iq_frag(uint4 grid, uint4 sign, uint32_t aux) {
 }
 
 struct hh_mmg_iq2_xxs {
-    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false;
+    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false, ROWS_LDS = false;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq2_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq2_table; }
@@ -395,7 +403,7 @@ struct hh_mmg_iq2_xxs {
 };
 
 struct hh_mmg_iq3_xxs {
-    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false;
+    static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false, ROWS_LDS = false;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq3_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq3_table; }
@@ -744,7 +752,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     constexpr uint32_t CB = 8u * NA * 1024u;            // stage bytes of a (tile, chunk)
     constexpr uint32_t SUMS = F::MINS ? 1024u : 0u;
     constexpr uint32_t BUF = TT * (CB + SUMS);
-    constexpr uint32_t ROWS = MODE == HH_MMG_S16 ? 16 : 32;  // tokens per tile
+    constexpr bool WL = F::ROWS_LDS && TT == 1;
     extern __shared__ __attribute__((aligned(16))) char hh_smem[];
     const uint32_t tid = threadIdx.x, lane = tid % 64;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -897,6 +905,53 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     typename F::Raw raw[2][2];  // [buffer][row tile]
     constexpr hh_uint_c<0> B0{};
     constexpr hh_uint_c<1> B1{};
+    if constexpr (WL) {
+        // A superblock of the wave's 64 rows comes as nine runs of whole pieces, about 14 lines
+        // each, where twelve loads of a lane's own row took 64 lines each, and is on its way for
+        // two chunks instead of one.  Only where a workgroup has one token tile: two workgroups
+        // of a CU fit LDS beside each other so.  512-token MoE layer 258 -> 246 us.
+        char* const slot = hh_smem + 2 * BUF + wave * HH_MMG_WSLOT;
+        const uint8_t* src[9];  // piece 64 i + lane of the slot: row / 9, 16 bytes each
+#pragma unroll
+        for (uint32_t i = 0; i < 9; i++) {
+            const uint32_t p = 64 * i + lane, rr = p / 9, q = rr / 32;
+            const uint32_t at = GU ? grp * 128 + wave * 32 + rr % 32 : grp * 256 + wave * 64 + rr;
+            src[i] = (q ? a.w1 : a.w0) + ex + (size_t)min(at, a.m - 1) * a.row_bytes + (c0 >> 1) * 144u + p % 9 * 16u;
+        }
+        auto rows = [&]() {
+#pragma unroll
+            for (uint32_t i = 0; i < 9; i++) {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[i],
+                                                 (__attribute__((address_space(3))) void*)(slot + i * 1024u), 16, 0, 0);
+                src[i] += 144;
+            }
+        };
+        copy(c0, B0);
+        rows();
+        for (uint32_t ch = c0; ch < c1; ch += 2) {
+            hh_mmg_sync();  // chunk ch's tokens and the superblock's rows have landed, buffer 1 is free
+#pragma unroll
+            for (int q = 0; q < 2; q++) F::load_lds(raw[0][q], raw[1][q], slot + (q * 32 + r) * 144u, h);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot is read
+            asm volatile("" ::: "memory");
+            copy(ch + 1, B1);
+            const bool more = ch + 2 < c1;
+            if (more) rows();
+            compute(raw[0], B0);
+            asm volatile("" ::: "memory");
+            if (more)
+                __builtin_amdgcn_s_waitcnt(0x0079);  // vmcnt(9) lgkmcnt(0): the tokens; the rows stay in flight
+            else
+                __builtin_amdgcn_s_waitcnt(0x0070);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (more) copy(ch + 2, B0);
+            compute(raw[1], B1);
+        }
+        hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci);
+        return;
+    }
     copy(c0, B0);
 #pragma unroll
     for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], c0, h, nblk);
@@ -1127,7 +1182,7 @@ extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_su
     HH_MMG_KERNEL(FMT, h2, HH_MMG_H, 2, 2)
 HH_MMG_FORMAT(q4_0, 2)
 HH_MMG_FORMAT(q8_0, 2)
-HH_MMG_FORMAT(q4_k, 3)
+HH_MMG_FORMAT(q4_k, 2)
 HH_MMG_FORMAT(q6_k, 3)
 HH_MMG_FORMAT(iq2_xxs, 3)
 HH_MMG_FORMAT(iq3_xxs, 3)
@@ -1138,7 +1193,7 @@ HH_MMG_FORMAT(iq3_xxs, 3)
     extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_moe_##NAME##_gu(const hh_mmg_args a) {         \
         hh_mmg_body<hh_mmg_q4_k, MODE, 1, true, true>(a);                                                       \
     }
-HH_MMG_MOE(s16, HH_MMG_S16, 3)
-HH_MMG_MOE(h1, HH_MMG_H, 3)
+HH_MMG_MOE(s16, HH_MMG_S16, 2)
+HH_MMG_MOE(h1, HH_MMG_H, 2)
 extern "C" __global__ void __launch_bounds__(256, 2) hh_mmg_q4_k_f4(const hh_mmg_args a) { hh_mmf_body<false>(a); }
 extern "C" __global__ void __launch_bounds__(256, 2) hh_mmg_q4_k_f4_gu(const hh_mmg_args a) { hh_mmf_body<true>(a); }

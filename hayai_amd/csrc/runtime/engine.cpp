@@ -1272,6 +1272,8 @@ static size_t mmf_from(bool ffn, size_t m, size_t n) {
 // against 32, 6 tokens 43 against 32).
 constexpr size_t kMmgMinTokens = 4, kMmgMinTokensSmallFfn = 5;
 
+constexpr size_t kMmgRowsLds = 4 * 9216;  // Q4_K with one tile: a superblock of each wave's 64 rows
+
 struct MmgFmt {
     int type;
     bool super, mins, half_major, paired;
@@ -1317,7 +1319,7 @@ static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, 
     p.nch = (n + 127) / 128;
     const size_t chunk = (p.rows == 16 || single ? 8 : 16) * 1024, sums = f->mins ? 1024 : 0;
     p.tile_bytes = p.nch * chunk + p.nch / 2 * sums;
-    p.smem = 2 * p.tt * (chunk + sums) + f->tab_bytes;
+    p.smem = 2 * p.tt * (chunk + sums) + f->tab_bytes + (f->mins && p.tt == 1 ? kMmgRowsLds : 0);
     // splits: rounds of two workgroups per CU against the sums' traffic (8 bytes per output and
     // split at about 3 TB/s, and a launch)
     const size_t step = f->super ? 2 : 1, slots = 2 * cus;
@@ -1737,7 +1739,7 @@ hh_status hh_engine::enqueue_moe_mmg(const hh_moe_desc* d, const uint8_t* expert
     HH_TRY(kernel("hh_mmg_moe_conv", &fn));
     HH_TRY(launch(fn, (uint32_t)(tiles * (dm / 128)), 256, c));
     const std::string name = std::string("hh_mmg_moe_") + (rows == 16 ? "s16" : "h1");
-    const unsigned smem = 2 * ((rows == 16 ? 8192 : 16384) + 1024);
+    const unsigned smem = 2 * ((rows == 16 ? 8192 : 16384) + 1024) + kMmgRowsLds;
     auto product = [&](bool gu, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, float* out) {
         MmgArgs a{};
         a.w0 = w0;

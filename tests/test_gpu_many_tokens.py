@@ -99,6 +99,23 @@ def test_ffn(engine, types, d_model, d_ff, batch, act):
         assert np.max(np.abs(Y[b] - ref)) <= 2e-5 * np.max(np.abs(ref)), b
 
 
+@pytest.mark.parametrize("d_model,d_ff,batch", [(256, 256, 4), (512, 768, 17), (2304, 512, 16), (1280, 1792, 31),
+                                                (4096, 256, 70)])
+def test_q4_k_rows_through_lds(engine, d_model, d_ff, batch):
+    # gate/up with one token tile: one superblock, a short and a long run of them, splits of
+    # unequal length, 16- and 32-token tiles
+    types = (Q4_K, Q4_K, Q8_0)
+    print(f"[case] q4_k rows through lds {d_model}x{d_ff} batch={batch}", flush=True)
+    lay, ws, pack = make_pack(engine, types, d_model, d_ff, 66)
+    desc = engine.ffn_desc(types, d_model, d_ff, lay)
+    X = synth.normal(67, batch * d_model).reshape(batch, d_model)
+    Y = engine.ffn_batched(desc, pack, 0, X)
+    for b in range(batch):
+        ref = oracle.ffn(types, d_model, d_ff, *ws, X[b])
+        # as test_ffn
+        assert np.max(np.abs(Y[b] - ref)) <= 2e-5 * np.max(np.abs(ref)), b
+
+
 def test_in_place_and_unaligned_activations(engine):
     # x read and y written at 4-byte offsets, and y over x
     t, d_model, d_ff, batch = Q8_0, 160, 96, 9
