@@ -40,7 +40,7 @@
 // Q6_K FFN, 16 tokens: 106 us against 779 us).
 //
 // MoE (hh_mmg_moe_*): the (token, slot) pairs of an expert in tiles of 16 or 32, one launch over
-// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 246 us a layer.
+// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 228 us a layer.
 //
 // Token stages: [tile][128-column chunk][group 0..3][step 0..1][hi, lo][lane][8 f16], for Q4_K
 // followed after every second chunk by the sums [lane][8 f16] (lane half 0: hi of sub-blocks
@@ -682,11 +682,28 @@ HH_DEV void hh_mmg_sync() {
     asm volatile("" ::: "memory");
 }
 
+// What the outputs of a workgroup's N token rows need, into LDS while the first loads are on
+// their way: the factors back, and for MoE's down the pairs.  Read from memory at the end, four
+// rows at a time, each read's latency was in the way (MoE above: gate/up 128 -> 112 us, down
+// 78 -> 58).
+template <uint32_t N>
+struct __attribute__((aligned(16))) hh_mmg_tokens {
+    float down[N];
+    uint32_t pair[N];
+    HH_DEV void set(const hh_mmg_args& a, uint32_t tg, int4 rec, bool pairs) {
+        const uint32_t t = threadIdx.x;
+        if (t >= N) return;
+        down[t] = hh_mmg_down(a.amax[tg * N + t]);  // padded to whole tiles
+        if (pairs) pair[t] = (uint32_t)a.order[rec.y + min((int)t, rec.z - 1)];
+    }
+};
+
 // The sums of a wave's 64 weight rows and TT token tiles to memory (gate/up: the activation,
 // and the row group's largest |h| of each token).
 template <int MODE, int TT, bool GU, bool MOE>
 HH_DEV void hh_mmg_store(const hh_mmg_args& a, const hh_f16v (&sum)[2][TT], const uint32_t (&row)[2], int4 rec,
-                         uint32_t tg, uint32_t grp, uint32_t kci) {
+                         uint32_t tg, uint32_t grp, uint32_t kci,
+                         const hh_mmg_tokens<TT * (MODE == HH_MMG_S16 ? 16 : 32)>& tok) {
     constexpr uint32_t ROWS = MODE == HH_MMG_S16 ? 16 : 32;  // tokens per tile
     extern __shared__ __attribute__((aligned(16))) char hh_smem[];
     const uint32_t tid = threadIdx.x, lane = tid % 64;
@@ -702,34 +719,55 @@ HH_DEV void hh_mmg_store(const hh_mmg_args& a, const hh_f16v (&sum)[2][TT], cons
 #pragma unroll
         for (int i4 = 0; i4 < (MODE == HH_MMG_S16 ? 2 : 4); i4++) {
             const uint32_t in = 8 * i4 + 4 * h, t0 = (tg * TT + tt) * ROWS + in;
-            const float4 d4 = *reinterpret_cast<const float4*>(a.amax + t0);  // padded to whole tiles
-            const float dn[4] = {hh_mmg_down(d4.x), hh_mmg_down(d4.y), hh_mmg_down(d4.z), hh_mmg_down(d4.w)};
+            const float4 d4 = *reinterpret_cast<const float4*>(tok.down + tt * ROWS + in);
+            const float dn[4] = {d4.x, d4.y, d4.z, d4.w};
+            uint32_t to[4] = {t0, t0 + 1, t0 + 2, t0 + 3};
+            if constexpr (MOE && !GU) {  // the pairs
+                const uint4 p4 = *reinterpret_cast<const uint4*>(tok.pair + in);
+                to[0] = p4.x, to[1] = p4.y, to[2] = p4.z, to[3] = p4.w;
+            }
+            float v[2][4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                uint32_t t = t0 + k;
-                const bool live = MOE ? (int)(in + k) < rec.z : t < a.b;
-                if constexpr (MOE && !GU) t = (uint32_t)a.order[rec.y + min((int)(in + k), rec.z - 1)];  // the pair
-                float v[2];
+            for (int k = 0; k < 4; k++)
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
-                    v[q] = sum[q][tt][4 * i4 + k];
-                    if constexpr (MODE == HH_MMG_S16) v[q] += sum[q][tt][4 * i4 + k + 8];
-                    v[q] *= dn[k];
+                    v[q][k] = sum[q][tt][4 * i4 + k];
+                    if constexpr (MODE == HH_MMG_S16) v[q][k] += sum[q][tt][4 * i4 + k + 8];
+                    v[q][k] *= dn[k];
                 }
+            float hv[4];
+            if (fuse) {
+                // four at a time under one branch: each is a long chain
+                if (a.act == HH_ACT_GELU_TANH) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) hv[k] = hh_act_mul(v[0][k], v[1][k], HH_ACT_GELU_TANH);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) hv[k] = hh_act_mul(v[0][k], v[1][k], HH_ACT_SILU);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const bool live = MOE ? (int)(in + k) < rec.z : to[k] < a.b;
+                const size_t at = (size_t)to[k] * a.m;
                 if (fuse) {
-                    float hv = hh_act_mul(v[0], v[1], a.act);
-                    if (live && row[0] < a.m) out[(size_t)t * a.m + row[0]] = hv;
-                    // over the wave's 32 rows (the token is the same in a lane half)
-                    // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
-                    hv = row[0] < a.m ? fabsf(hv) : 0.f;
-                    hv = fmaxf(hv, hh_dpp<0xB1>(hv));   // quad_perm [1,0,3,2]
-                    hv = fmaxf(hv, hh_dpp<0x4E>(hv));   // quad_perm [2,3,0,1]
-                    hv = fmaxf(hv, hh_dpp<0x124>(hv));  // row_ror:4
-                    hv = fmaxf(hv, hh_dpp<0x128>(hv));  // row_ror:8
-                    if ((r & 15u) == 0) wmax[(r >> 4) * (TT * ROWS) + tt * ROWS + in + k] = hv;
+                    if (live && row[0] < a.m) out[at + row[0]] = hv[k];
                 } else if (live) {
-                    if (row[0] < a.m) out[(size_t)t * a.m + row[0]] = v[0];
-                    if (row[1] < a.m) out[(GU ? a.up_stride : 0) + (size_t)t * a.m + row[1]] = v[1];
+                    if (row[0] < a.m) out[at + row[0]] = v[0][k];
+                    if (row[1] < a.m) out[(GU ? a.up_stride : 0) + at + row[1]] = v[1][k];
+                }
+            }
+            if (fuse) {
+                // over the wave's 32 rows (a token is the same in a lane half)
+                // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    float x = row[0] < a.m ? fabsf(hv[k]) : 0.f;
+                    x = fmaxf(x, hh_dpp<0xB1>(x));   // quad_perm [1,0,3,2]
+                    x = fmaxf(x, hh_dpp<0x4E>(x));   // quad_perm [2,3,0,1]
+                    x = fmaxf(x, hh_dpp<0x124>(x));  // row_ror:4
+                    x = fmaxf(x, hh_dpp<0x128>(x));  // row_ror:8
+                    if ((r & 15u) == 0) wmax[(r >> 4) * (TT * ROWS) + tt * ROWS + in + k] = x;
                 }
             }
         }
@@ -753,6 +791,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
     constexpr uint32_t SUMS = F::MINS ? 1024u : 0u;
     constexpr uint32_t BUF = TT * (CB + SUMS);
     constexpr bool WL = F::ROWS_LDS && TT == 1;
+    __shared__ hh_mmg_tokens<TT * (MODE == HH_MMG_S16 ? 16 : 32)> tokens;
     extern __shared__ __attribute__((aligned(16))) char hh_smem[];
     const uint32_t tid = threadIdx.x, lane = tid % 64;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -928,6 +967,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         };
         copy(c0, B0);
         rows();
+        tokens.set(a, tg, rec, MOE && !GU);
         for (uint32_t ch = c0; ch < c1; ch += 2) {
             hh_mmg_sync();  // chunk ch's tokens and the superblock's rows have landed, buffer 1 is free
 #pragma unroll
@@ -949,12 +989,13 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
             if (more) copy(ch + 2, B0);
             compute(raw[1], B1);
         }
-        hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci);
+        hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci, tokens);
         return;
     }
     copy(c0, B0);
 #pragma unroll
     for (int q = 0; q < 2; q++) F::template load<0>(raw[0][q], wp[q], c0, h, nblk);
+    tokens.set(a, tg, rec, MOE && !GU);
     for (uint32_t ch = c0; ch < c1; ch += 2) {
         // chunk ch's tokens have landed for every wave, and buffer 1 is free
         hh_mmg_sync();
@@ -975,7 +1016,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         compute(raw[1], B1);
     }
 
-    hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci);
+    hh_mmg_store<MODE, TT, GU, MOE>(a, sum, row, rec, tg, grp, kci, tokens);
 }
 
 // ---- Q4_K, one f16 per token element --------------------------------------------------
@@ -999,6 +1040,7 @@ HH_DEV void hh_mmf_body(const hh_mmg_args& a) {
     const uint32_t tid = threadIdx.x, lane = tid % 64;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const uint32_t r = lane & 31u, h = lane >> 5;
+    __shared__ hh_mmg_tokens<TT * 32> tokens;
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     const uint32_t unit = slot / a.ttiles * 8u + xcd, tg = slot % a.ttiles;  // as hh_mmg_body
     if (unit >= a.groups * a.kc) return;
@@ -1105,6 +1147,7 @@ HH_DEV void hh_mmf_body(const hh_mmg_args& a) {
     copy(c0, B0);
 #pragma unroll
     for (int q = 0; q < 2; q++) F::load<0>(raw[0][q], wp[q], c0, h, 0);
+    tokens.set(a, tg, int4{}, false);
     for (uint32_t ch = c0; ch < c1; ch += 2) {
         hh_mmg_sync();
         copy(ch + 1, B1);
@@ -1126,7 +1169,7 @@ HH_DEV void hh_mmf_body(const hh_mmg_args& a) {
         for (int tt = 0; tt < TT; tt++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[q][tt][i] *= u[q];
-    hh_mmg_store<HH_MMG_F, TT, GU, false>(a, acc, row, int4{}, tg, grp, kci);
+    hh_mmg_store<HH_MMG_F, TT, GU, false>(a, acc, row, int4{}, tg, grp, kci, tokens);
 }
 
 struct hh_mmg_sum_args {
