@@ -1804,8 +1804,15 @@ hh_status hh_engine::enqueue_moe_ffn(const hh_moe_desc* d, const uint8_t* expert
                                    y + t0 * dm, logits ? logits + t0 * E : nullptr, bias));
         return HH_OK;
     }
+    // Pairs per active expert from which the matrix cores are faster (grouped : matrix cores, us):
+    // 128 experts of 2048 x 768, top 8: 2 pairs 93 : 111, 3 pairs 117 : 117, 4 pairs 136 : 120; 64 of
+    // 2048 x 1536: 2 pairs 92 : 105, 4 pairs 139 : 113; 64 of 2048 x 1024: 2 pairs 62 : 71, 4 pairs
+    // 91 : 77.  Where the experts leave CUs idle the fixed part weighs more: 16 of 1024 x 1536,
+    // 4 pairs 41 : 46; 16 of 1024 x 512, 5.5 pairs 36 : 39.
+    const size_t active = std::min(E, P);
+    const bool fills = active * (dm / 256) >= 2 * (size_t)props.multiProcessorCount && P * dm * df >= 400000000u;
     if (groups && mmg && P <= kMoeMaxPairs && dm / 64 <= 64 && df / 64 <= 64 && T > 1 &&
-        (double)P >= moe_mmg_min * (double)std::min(E, P)) {
+        (double)P >= (moe_mmg_min > 0 ? moe_mmg_min : fills ? 3.0 : 6.0) * (double)active) {
         const hh_status st = enqueue_moe_mmg(d, experts, x, T, ids, wts, y, logits, bias);
         if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }

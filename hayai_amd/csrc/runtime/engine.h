@@ -175,11 +175,9 @@ struct hh_engine {
     // ways, 1024 x 1024 5.6 us against 7.6)
     size_t block_stream_min = (size_t)256 << 10;
     bool mmg = true;            // HAYAI_HIP_MMG=0: other formats' batches one token at a time
-    // HAYAI_HIP_MOE_MMG_MIN: (token, slot) pairs per expert from which MoE runs on mmg.hip.
-    // Against the grouped gather-GEMV, us: 128 experts 2048 x 768 4 pairs 161 : 148, 6.2 pairs
-    // 166 : 205; 64 experts 1024 x 1280 4 pairs 76 : 80; 16 experts 1024 x 512 4 pairs 41 : 33,
-    // 6 pairs 41 : 40, 8 pairs 42 : 45.
-    double moe_mmg_min = 6;
+    // HAYAI_HIP_MOE_MMG_MIN: pairs per active expert from which a MoE layer takes the matrix cores
+    // (0: by the experts, enqueue_moe_ffn)
+    double moe_mmg_min = 0;
     size_t mmf_min = 0;         // HAYAI_HIP_MMF_MIN: all-Q4_K batches from which tokens are f16 (0: by the weights)
     size_t mmi_min = 17;        // HAYAI_HIP_MMI_MIN: fewest tokens per pass on the int8 kernels (>= 2)
     int mmi_d = 0;              // HAYAI_HIP_MMI_D: ring depth of the int8 f16-MFMA kernels (0: chosen)
