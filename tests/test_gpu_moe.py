@@ -312,9 +312,10 @@ def test_moe_grouped_at_the_pair_limit(engine, T):
     (2, 2, 512, 256, 48),     # every expert has every token: 32-pair tiles, the last of 16
     (3, 1, 256, 768, 200),    # uneven experts, row groups past the matrix
     (4, 3, 256, 256, 1400),   # 4200 pairs: two passes of the grouping
+    (128, 8, 1024, 1024, 48),  # 3 pairs an expert are enough where the experts fill the chip
 ])
 def test_moe_on_the_matrix_cores(engine, E, k, d_model, d_ff, T):
-    # From 6 pairs per expert the experts' products run in tiles of one expert's pairs; routed
+    # From 6 (or 3) pairs per expert the experts' products run in tiles of one expert's pairs; routed
     # on the GPU and from given ids with empty slots.
     print(f"[case] moe tiles E={E} k={k} {d_model}x{d_ff} T={T}", flush=True)
     buf, host, stride, offs = make_experts(engine, E, d_model, d_ff, 77)
