@@ -1266,6 +1266,16 @@ static size_t mmf_from(bool ffn, size_t m, size_t n) {
     return w >= (size_t)100 << 20 ? 65 : w >= (size_t)48 << 20 ? 97 : 136;
 }
 
+// The leading tokens of an all-Q4_K batch that may enter as one f16: those of the passes that
+// would take 8-bit tokens.  The last pass has fewer than mmi_min tokens where the batch leaves so
+// few over 64, and they keep the f32-accurate kernels (16 tokens or one), as in a short batch: of
+// an 8B FFN 3.7e-4 against 5e-4, of a product 2e-7 against 2.5e-4 (2-norm).
+size_t hh_engine::mmf_tokens(size_t batch) const {
+    if (!mmq || mmi_min > kMmMaxTokens) return 0;
+    const size_t last = batch % kMmMaxTokens;
+    return last < mmi_min ? batch - last : batch;
+}
+
 // From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
 // 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
 // one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
@@ -1489,11 +1499,13 @@ hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const ui
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_gemv(type, m, n, w, x + b * n, y + b * m));
         return HH_OK;
     }
-    if (mmq && batch >= (mmf_min ? mmf_min : mmf_from(false, m, n))) {
-        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y, true);
-        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    size_t done = 0;
+    if (batch >= (mmf_min ? mmf_min : mmf_from(false, m, n)) && mmf_tokens(batch)) {
+        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, mmf_tokens(batch), y, true);
+        if (st == HH_OK) done = mmf_tokens(batch);
+        else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
-    for (size_t b0 = 0; b0 < batch; b0 += kMmMaxTokens) {
+    for (size_t b0 = done; b0 < batch; b0 += kMmMaxTokens) {
         const size_t nb = std::min(kMmMaxTokens, batch - b0);
         if (nb == 1) {
             HH_TRY(enqueue_gemv(type, m, n, w, x + b0 * n, y + b0 * m));
@@ -1560,11 +1572,13 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_ffn(d, pack, x + b * dm, y + b * dm));
         return HH_OK;
     }
-    if (mmq && batch >= (mmf_min ? mmf_min : mmf_from(true, df, dm))) {
-        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y, true);
-        if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
+    size_t done = 0;
+    if (batch >= (mmf_min ? mmf_min : mmf_from(true, df, dm)) && mmf_tokens(batch)) {
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, mmf_tokens(batch), y, true);
+        if (st == HH_OK) done = mmf_tokens(batch);
+        else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
-    for (size_t b0 = 0; b0 < batch; b0 += kMmMaxTokens) {
+    for (size_t b0 = done; b0 < batch; b0 += kMmMaxTokens) {
         const size_t nb = std::min(kMmMaxTokens, batch - b0);
         if (nb == 1) {
             HH_TRY(enqueue_ffn(d, pack, x + b0 * dm, y + b0 * dm));

@@ -303,7 +303,8 @@ struct hh_engine {
     // the product of the staged tokens: GEMM (w1 null) into y [b][m], or gate/up + act into y
     hh_status mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b, float* y,
                           int act, bool h, bool single);
-    // single: one f16 per token element (Q4_K)
+    // single: one f16 per token element (Q4_K), for the first mmf_tokens of a batch
+    size_t mmf_tokens(size_t batch) const;
     hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y,
                                bool single);
     hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y,

@@ -185,7 +185,8 @@ void hh_pending_destroy(hh_pending* p);
  *     max|y| per token on N(0,1) activations (the tests bound it at 4%);
  *   - longer batches (from 65 to 144 tokens on, by the size of the weights), in passes of up to
  *     1024: each activation as one f16 of its token's own power-of-two scale, exact integer
- *     weights, f32 accumulation: measured 2.5e-4 of the f32 product (2-norm).
+ *     weights, f32 accumulation: measured 2.5e-4 of the f32 product (2-norm).  The 1..16 tokens
+ *     that such a batch has over a multiple of 64 are a pass of their own, at f32 accuracy.
  * Set HAYAI_HIP_MMQ=0 in the environment before creating the engine to keep f32
  * activations for every batch size (17 and more tokens then run one token at a time);
  * HAYAI_HIP_MMI_MIN=16 moves passes of 16 tokens onto the int8 form. */
@@ -295,7 +296,7 @@ hh_status hh_ffn_block_stack_dev(hh_engine* e, const hh_ffn_desc* d, const hh_bu
  * precision hh_gemv_batched states: passes of 17..64 tokens quantize x, and then h, to
  * int8 per 32-element block, which moves the FFN output by 3-13% of max|y| per token on
  * N(0,1) inputs (h is heavy-tailed; the tests bound it at 25%), longer batches enter x and h
- * as f16 (5e-4, 2-norm); passes of 2..16 tokens stay
+ * as f16 (5e-4, 2-norm; not the 1..16 tokens over a multiple of 64); passes of 2..16 tokens stay
  * within 1e-3 of the f32 FFN (h enters down as f16).  Other layers of quantized types (gate
  * and up alike) run gate/up(+act) and down on the matrix cores at f32 accuracy from 4 or 5
  * tokens on; what is left runs the single-token op per token.  _dev: device buffers, enqueue only; without: host x / y, blocking. */

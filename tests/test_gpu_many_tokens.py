@@ -200,3 +200,30 @@ def test_f16_ffn(f16_engine, d_model, d_ff, batch, act):
     worst = float(np.max(np.abs(Y - (f * u) @ D.T) / bound))
     print(f"  worst error / bound {worst:.3e}", flush=True)
     assert worst <= 1.0
+
+
+@pytest.mark.parametrize("m,n,batch", [(300, 512, 65), (257, 768, 66), (256, 2304, 80), (512, 512, 139)])
+def test_f16_leaves_a_short_last_pass(f16_engine, m, n, batch):
+    # the 1..16 tokens over a multiple of 64 are computed as in a batch of their own
+    print(f"[case] f16 tokens, last pass m={m} n={n} batch={batch}", flush=True)
+    at = batch // 64 * 64
+    w = synth.matrix(Q4_K, m, n, 68)
+    X = synth.normal(69, batch * n).reshape(batch, n)
+    Y = f16_engine.ggml_gemv_batched_q4_k(m, n, w, X, batch).reshape(batch, m)
+    last = f16_engine.ggml_gemv_batched_q4_k(m, n, w, X[at:], batch - at).reshape(-1, m)
+    np.testing.assert_array_equal(Y[at:], last)
+    lay, ws, pack = make_pack(f16_engine, (Q4_K,) * 3, n, 512, 70)
+    desc = f16_engine.ffn_desc((Q4_K,) * 3, n, 512, lay)
+    Y = f16_engine.ffn_batched(desc, pack, 0, X)
+    np.testing.assert_array_equal(Y[at:], f16_engine.ffn_batched(desc, pack, 0, X[at:]))
+
+
+def test_f16_starts_at_a_full_pass(f16_engine):
+    # 81 tokens: the last pass has 17, which would be 8-bit ones, and is f16 with the others
+    m, n, batch = 64, 512, 81
+    w = synth.matrix(Q4_K, m, n, 71)
+    X = synth.normal(72, batch * n).reshape(batch, n)
+    Y = f16_engine.ggml_gemv_batched_q4_k(m, n, w, X, batch).reshape(batch, m)
+    W, wide = parts(w, m, n)
+    X = X.astype(np.float64)
+    assert np.all(np.abs(Y - X @ W.T) <= np.abs(X) @ wide.T)
