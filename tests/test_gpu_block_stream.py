@@ -102,3 +102,17 @@ def test_zero_scale_past_the_slice(stream):
     w[3, -34:-32] = np.array([0x7C00], np.uint16).view(np.uint8)
     y = stream.ggml_gemv_dispatch(t, m, n, w, synth.normal(77, n))
     assert not np.isfinite(y[3]) and np.isfinite(np.delete(y, 3)).all()
+
+
+@pytest.mark.parametrize("m,n", [(40, 256), (5, 4096), (40, 5632), (9, 14336)])
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+def test_infinite_element_in_the_last_block(stream, t, m, n):
+    # lanes past a slice hold its last block of x: an infinity there counts once, as in IEEE sums
+    print(f"[case] block stream infinity type={t} m={m} n={n}", flush=True)
+    w = synth.matrix(t, m, n, 80)
+    x = synth.normal(81, n)
+    x[n - 3] = -np.inf
+    y = stream.ggml_gemv_dispatch(t, m, n, w, x)
+    W = oracle.dequant(t, w, m * n).reshape(m, n).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(y, (W * x.astype(np.float64)).sum(axis=1).astype(np.float32))
