@@ -458,11 +458,12 @@ struct hh_mmg_amax_args {
     uint32_t n, pad;
 };
 
-// amax in [2^(k-1), 2^k) -> up = 2^(10 - k): the largest magnitude into [512, 1024), so that a
-// sum of 32 elements stays below f16's largest value.  A token without a finite, non-zero
-// maximum keeps the factor 1 (its infinities stay infinities).
+// A token's amax: the largest of its finite magnitudes.  amax in [2^(k-1), 2^k) -> up = 2^(10 - k):
+// the largest magnitude into [512, 1024), so that a sum of 32 elements stays below f16's largest
+// value; infinities stay what they are under any factor.  A token of zeros keeps the factor 1.
+HH_DEV float hh_mmg_mag(float x) { return fabsf(x) < __builtin_inff() ? fabsf(x) : 0.f; }
 HH_DEV int hh_mmg_exp(float amax) {
-    if (!(amax > 0.f && amax < __builtin_inff())) return 0;
+    if (amax == 0.f) return 0;
     int k;
     (void)frexpf(amax, &k);
     return min(max(10 - k, -120), 120);
@@ -473,22 +474,27 @@ HH_DEV float hh_wave_max(float v) {
     return v;
 }
 
-// A workgroup of 256 threads: the largest magnitude of x[0, n) (NaN elements do not count).
-HH_DEV void hh_mmg_token_amax(const float* x, uint32_t n, float* amax) {
-    __shared__ float red[4];
+// A workgroup of 256 threads: the amax of x[0, n).
+template <class MAG>
+HH_DEV float hh_mmg_wave_amax(const float* x, uint32_t n, MAG mag) {
     float v = 0.f;
     if ((((uintptr_t)x | n) & 3u) == 0 && ((uintptr_t)x & 15u) == 0) {
         const float4* x4 = reinterpret_cast<const float4*>(x);
 #pragma unroll 4
         for (uint32_t i = threadIdx.x; i < n / 4; i += 256) {
             const float4 u = x4[i];
-            v = fmaxf(v, fmaxf(fmaxf(fabsf(u.x), fabsf(u.y)), fmaxf(fabsf(u.z), fabsf(u.w))));
+            v = fmaxf(v, fmaxf(fmaxf(mag(u.x), mag(u.y)), fmaxf(mag(u.z), mag(u.w))));
         }
     } else {
 #pragma unroll 4
-        for (uint32_t i = threadIdx.x; i < n; i += 256) v = fmaxf(v, fabsf(x[i]));
+        for (uint32_t i = threadIdx.x; i < n; i += 256) v = fmaxf(v, mag(x[i]));
     }
-    v = hh_wave_max(v);
+    return hh_wave_max(v);
+}
+HH_DEV void hh_mmg_token_amax(const float* x, uint32_t n, float* amax) {
+    __shared__ float red[4];
+    float v = hh_mmg_wave_amax(x, n, [](float e) { return fabsf(e); });  // (fmaxf leaves NaN out)
+    if (v == __builtin_inff()) v = hh_mmg_wave_amax(x, n, hh_mmg_mag);
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
     __syncthreads();
     if (threadIdx.x == 0) *amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -506,10 +512,11 @@ HH_DEV uint32_t hh_bf16(float v) {
     return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
 }
 
+// v = hi + lo.  An infinity is in lo, with the largest finite hi: hi meets Q6_K's remainders too, most
+// of which are 0, and lo only the codes' own products.
 HH_DEV void hh_mmg_split(float v, _Float16& hi, _Float16& lo) {
-    hi = (_Float16)v;
-    const float r = v - (float)hi;
-    lo = (_Float16)(r == r ? r : 0.f);  // an infinite v: hi carries it alone
+    hi = (_Float16)__builtin_amdgcn_fmed3f(v, -65504.f, 65504.f);
+    lo = (_Float16)(v - (float)hi);
 }
 
 // One chunk of one tile, by a workgroup of `threads`.  row(tok, &src, &up): the tile's token tok
@@ -554,7 +561,7 @@ HH_DEV void hh_mmg_conv_chunk(uint8_t* tile, const hh_mmg_conv_args& a, uint32_t
         for (int e = 0; e < 8; e++) {
             _Float16 x0, x1;
             hh_mmg_split(v[e], x0, x1);
-            hi[e] = x0;
+            hi[e] = a.single ? (_Float16)v[e] : x0;
             lo[e] = x1;
         }
         const uint32_t gs = g * 2 + step;
@@ -762,7 +769,7 @@ HH_DEV void hh_mmg_store(const hh_mmg_args& a, const hh_f16v (&sum)[2][TT], cons
                 // its two 16-lane rows by DPP: LDS shuffles here cost 10 us of a 150 us launch
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    float x = row[0] < a.m ? fabsf(hv[k]) : 0.f;
+                    float x = row[0] < a.m ? hh_mmg_mag(hv[k]) : 0.f;
                     x = fmaxf(x, hh_dpp<0xB1>(x));   // quad_perm [1,0,3,2]
                     x = fmaxf(x, hh_dpp<0x4E>(x));   // quad_perm [2,3,0,1]
                     x = fmaxf(x, hh_dpp<0x124>(x));  // row_ror:4
@@ -782,6 +789,13 @@ HH_DEV void hh_mmg_store(const hh_mmg_args& a, const hh_f16v (&sum)[2][TT], cons
             a.pmax[(size_t)grp * a.ldt + tg * (TT * ROWS) + tid] = v;
         }
     }
+}
+
+// Infinities as the largest finite values.
+HH_DEV hh_h8 hh_finite(hh_h8 v) {
+    const _Float16 m = (_Float16)65504.f;
+    const hh_h8 top = {m, m, m, m, m, m, m, m};
+    return __builtin_elementwise_max(__builtin_elementwise_min(v, top), -top);
 }
 
 template <class F, int MODE, int TT, bool GU, bool MOE = false>
@@ -892,6 +906,12 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
                     for (int tt = 0; tt < TT; tt++)
                         x[k][tt] = *reinterpret_cast<const hh_h8*>(st + tt * (CB + SUMS) + (g * 2 + s) * (NA * 1024) +
                                                                    k * 1024);
+                // what the weights' remainders meet: hi.  In s16 its tile holds lo too, and they are made
+                // finite here (8B Q6_K FFN, 16 tokens 80.7 -> 82.3 us; zeros for lo by way of LDS 87.6)
+                hh_h8 xrem[TT];
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++)
+                    xrem[tt] = F::NB > 1 && MODE == HH_MMG_S16 ? hh_finite(x[0][tt]) : x[0][tt];
                 // hi of every tile, then lo, then the weights' remainders: no product waits for
                 // the one before it
 #pragma unroll
@@ -906,7 +926,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
                                 for (int i = 0; i < 16; i++) c[i] = 0.f;
                             }
                             part[q][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                k < NA ? x[k][tt] : x[0][tt], wf[q][k < NA ? 0 : 1], c, 0, 0, 0);
+                                k < NA ? x[k][tt] : xrem[tt], wf[q][k < NA ? 0 : 1], c, 0, 0, 0);
                         }
             }
             if (!F::SUPER || (close && g == 3)) {
@@ -1205,7 +1225,7 @@ extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_su
     const float h = hh_act_mul(g, u, a.act);
     if (r < a.m) a.y[i] = h;
     __shared__ float red[4];
-    const float v = hh_wave_max(r < a.m ? fabsf(h) : 0.f);
+    const float v = hh_wave_max(r < a.m ? hh_mmg_mag(h) : 0.f);
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = v;
     __syncthreads();
     if (threadIdx.x == 0)

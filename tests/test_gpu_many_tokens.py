@@ -71,6 +71,29 @@ def test_tokens_of_any_size(engine, t):
     assert not np.isfinite(Y[4]).any()
 
 
+@pytest.mark.parametrize("batch", [7, 24, 64])  # the three tilings
+@pytest.mark.parametrize("t", FORMATS)
+def test_infinities_and_nan(engine, t, batch):
+    # as the sum of the products in IEEE arithmetic: an infinite element makes an output infinite, or
+    # NaN where its weight is 0, whatever its token's finite elements are
+    print(f"[case] infinities type={t} batch={batch}", flush=True)
+    m, n = 96, 768
+    w = synth.matrix(t, m, n, 56)
+    X = synth.normal(57, batch * n).reshape(batch, n)
+    X[1, n - 1] = np.inf
+    X[2, 5] = -np.inf
+    X[2, 300:] *= np.float32(1e9)  # finite, far above f16
+    X[3, 40] = np.nan
+    X[4, 9], X[4, 700] = np.inf, -np.inf
+    Y = engine.ggml_gemv_batched(t, m, n, w, X, batch).reshape(batch, m)
+    W = oracle.dequant(t, w, m * n).reshape(m, n).astype(np.float64)
+    fine = [0, 5, 6]
+    check(t, m, n, w, X[fine], Y[fine])
+    with np.errstate(invalid="ignore"):
+        for b in (1, 2, 3, 4):
+            np.testing.assert_array_equal(Y[b], (W * X[b].astype(np.float64)).sum(axis=1).astype(np.float32), str(b))
+
+
 def make_pack(engine, types, d_model, d_ff, cfg):
     shapes = [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]
     mats = [hayai_amd.QuantMatrix("m", c, r, t) for t, (r, c) in zip(types, shapes)]
