@@ -16,7 +16,8 @@
 // elements are scaled by one power of two (its largest magnitude into [512, 1024)) and split
 // into two f16, hi + lo, which carry 22 bits; products are summed in f32 by the matrix cores
 // over one scale block (32 or 256 columns), then d times that is added to the running sum.
-// Measured against 64 bits: 1e-7 to 4e-7, as the one-token f32 kernels.
+// Measured against 64 bits (2-norm): 6e-8 to 1.7e-7 a product, 1.5e-7 to 4e-7 an FFN; for rows that the
+// one-token kernels sum in f32 no more than theirs, by short sums (hh_mmg_fine, and at most 512 columns to a split).
 // The Q4_K minimum is dmin * sum_j m_j X_j with X_j the f32 sum of the token's 32 elements of
 // sub-block j, as hi + lo f16: one MFMA per superblock (k slots 0..7 hi, 8..15 lo).
 //
@@ -116,7 +117,8 @@ struct hh_mmg_k {
 // ---- weight formats -------------------------------------------------------------------
 // Raw: one chunk's bytes of one row as loaded (ready: what is taken from them once); load(p, ch,
 // ...) of chunk ch of the row at p (half h); frag(raw, g, s): the B operand of step s of the chunk's group g; scale(raw, g):
-// the d of the block that group g closes.  NB: B operands per step.
+// the d of the block that group g closes.  NB: B operands per step.  RUN: groups (32 columns) that
+// the matrix cores sum before d.
 // The 32-column formats: lane half h loads the two whole blocks 4 ch + 2 h, + 1 (consecutive
 // bytes: 3 loads for Q4_0, 5 for Q8_0, where a load of each half block and each d took 8), and
 // `ready` exchanges halves with the lane of the same row: then every lane has its half of all four.
@@ -181,6 +183,7 @@ struct hh_mmg_pair {
 
 struct hh_mmg_q4_0 {
     static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true, ROWS_LDS = false;
+    static constexpr int RUN = 1;
     static constexpr int NB = 1;
     typedef hh_mmg_pair<4> Raw;
     template <uint32_t HALF>
@@ -210,6 +213,7 @@ struct hh_mmg_q4_0 {
 
 struct hh_mmg_q8_0 {
     static constexpr bool SUPER = false, MINS = false, TABLES = false, READY = true, ROWS_LDS = false;
+    static constexpr int RUN = 1;
     static constexpr int NB = 1;
     typedef hh_mmg_pair<8> Raw;
     template <uint32_t HALF>
@@ -232,6 +236,7 @@ struct hh_mmg_q8_0 {
 
 struct hh_mmg_q4_k {
     static constexpr bool SUPER = true, MINS = true, TABLES = false, READY = true, ROWS_LDS = true;
+    static constexpr int RUN = 8;
     static constexpr int NB = 1;
     struct Raw {
         uint4 q[2];
@@ -286,6 +291,7 @@ struct hh_mmg_q4_k {
 
 struct hh_mmg_q6_k {
     static constexpr bool SUPER = true, MINS = false, TABLES = false, READY = false, ROWS_LDS = false;
+    static constexpr int RUN = 8;
     static constexpr int NB = 2;
     struct Raw {
         uint4 a, b, qh;
@@ -377,6 +383,7 @@ HH_DEV hh_h8 hh_mmg_iq_frag(uint4 grid, uint4 sign, uint32_t aux) {
 
 struct hh_mmg_iq2_xxs {
     static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false, ROWS_LDS = false;
+    static constexpr int RUN = 8;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq2_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq2_table; }
@@ -404,6 +411,7 @@ struct hh_mmg_iq2_xxs {
 
 struct hh_mmg_iq3_xxs {
     static constexpr bool SUPER = true, MINS = false, TABLES = true, READY = false, ROWS_LDS = false;
+    static constexpr int RUN = 8;
     static constexpr int NB = 1;
     static constexpr uint32_t TAB = sizeof(hh_mmg_iq3_tab);
     HH_DEV static const uint8_t* table() { return (const uint8_t*)&hh_mmg_iq3_table; }
@@ -433,6 +441,18 @@ struct hh_mmg_iq3_xxs {
                               *reinterpret_cast<const uint4*>(tab + 2048 + ((aux >> (7 * l)) & 127u) * 16), aux);
     }
 };
+
+// For rows that the one-token kernels sum in f32 (MmgForm::Fine): 64 columns (Q6_K, with its
+// remainders, 32) to a sum of the matrix cores, whose additions over 256 alone lose more than an
+// f32 product does.  2048 x 3840, 24 tokens, against 64 bits: IQ2_XXS 1.74e-7 -> 1.06e-7 (one token
+// 1.28e-7), Q6_K 1.82e-7 -> 1.05e-7 (1.13e-7).
+template <class F>
+struct hh_mmg_fine : F {
+    static constexpr int RUN = F::NB > 1 ? 1 : 2;
+};
+typedef hh_mmg_fine<hh_mmg_q6_k> hh_mmg_q6_k_fine;
+typedef hh_mmg_fine<hh_mmg_iq2_xxs> hh_mmg_iq2_xxs_fine;
+typedef hh_mmg_fine<hh_mmg_iq3_xxs> hh_mmg_iq3_xxs_fine;
 
 // ---- tokens -> stages -----------------------------------------------------------------
 
@@ -898,7 +918,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
                 hh_h8 wf[2][F::NB];
 #pragma unroll
                 for (int q = 0; q < 2; q++) F::template frag<buf>(raw[q], g, s, h, tab, kk, wf[q]);
-                const bool fresh = s == 0 && (F::SUPER ? open && g == 0 : true);
+                const bool fresh = s == 0 && (F::RUN == 8 ? open && g == 0 : g % F::RUN == 0);
                 hh_h8 x[NA][TT];
 #pragma unroll
                 for (int k = 0; k < NA; k++)
@@ -929,7 +949,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
                                 k < NA ? x[k][tt] : xrem[tt], wf[q][k < NA ? 0 : 1], c, 0, 0, 0);
                         }
             }
-            if (!F::SUPER || (close && g == 3)) {
+            if (F::RUN < 8 ? g % F::RUN == F::RUN - 1 : close && g == 3) {
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
                     const float d = F::scale(raw[q], g);
@@ -1203,24 +1223,31 @@ struct hh_mmg_sum_args {
     int32_t act;
     uint32_t ldt;
 };
+// s += v with c, what the additions have lost so far (Kahan): 4096 columns of Q8_0 in up to 32 splits,
+// 8 tokens, 1.28e-7 -> 7.8e-8 against 64 bits (one token 1.1e-7), in the same time.
+HH_DEV void hh_mmg_add(float& s, float& c, float v) {
+    const float y = v + c, t = s + y;
+    c = fabsf(t) < __builtin_inff() ? y - (t - s) : 0.f;
+    s = t;
+}
 // grid.y: tokens
 extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum(const hh_mmg_sum_args a) {
     const uint32_t r = blockIdx.x * 256 + threadIdx.x;
     if (r >= a.m) return;
     const uint64_t i = (uint64_t)blockIdx.y * a.m + r;
-    float s = 0.f;
+    float s = 0.f, c = 0.f;
 #pragma unroll 4
-    for (uint32_t k = 0; k < a.kc; k++) s += a.part[k * a.stride + i];
+    for (uint32_t k = 0; k < a.kc; k++) hh_mmg_add(s, c, a.part[k * a.stride + i]);
     a.y[i] = s;
 }
 extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_sum_args a) {
     const uint32_t r = blockIdx.x * 256 + threadIdx.x;
     const uint64_t i = (uint64_t)blockIdx.y * a.m + min(r, a.m - 1);
-    float g = 0.f, u = 0.f;
+    float g = 0.f, u = 0.f, gc = 0.f, uc = 0.f;
 #pragma unroll 4
     for (uint32_t k = 0; k < a.kc; k++) {
-        g += a.part[k * a.stride + i];
-        u += a.part[k * a.stride + a.up_stride + i];
+        hh_mmg_add(g, gc, a.part[k * a.stride + i]);
+        hh_mmg_add(u, uc, a.part[k * a.stride + a.up_stride + i]);
     }
     const float h = hh_act_mul(g, u, a.act);
     if (r < a.m) a.y[i] = h;
@@ -1239,9 +1266,11 @@ extern "C" __global__ void __launch_bounds__(256) hh_mmg_sum_act(const hh_mmg_su
     extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_##FMT##_##NAME##_gu(const hh_mmg_args a) {     \
         hh_mmg_body<hh_mmg_##FMT, MODE, TT, true>(a);                                                           \
     }
-#define HH_MMG_FORMAT(FMT, WPE)               \
+#define HH_MMG_ONE_TILE(FMT, WPE)             \
     HH_MMG_KERNEL(FMT, s16, HH_MMG_S16, 1, WPE) \
-    HH_MMG_KERNEL(FMT, h1, HH_MMG_H, 1, WPE)    \
+    HH_MMG_KERNEL(FMT, h1, HH_MMG_H, 1, WPE)
+#define HH_MMG_FORMAT(FMT, WPE) \
+    HH_MMG_ONE_TILE(FMT, WPE)   \
     HH_MMG_KERNEL(FMT, h2, HH_MMG_H, 2, 2)
 HH_MMG_FORMAT(q4_0, 2)
 HH_MMG_FORMAT(q8_0, 2)
@@ -1249,6 +1278,9 @@ HH_MMG_FORMAT(q4_k, 2)
 HH_MMG_FORMAT(q6_k, 3)
 HH_MMG_FORMAT(iq2_xxs, 3)
 HH_MMG_FORMAT(iq3_xxs, 3)
+HH_MMG_ONE_TILE(q6_k_fine, 2)  // (two tiles spill)
+HH_MMG_FORMAT(iq2_xxs_fine, 2)
+HH_MMG_FORMAT(iq3_xxs_fine, 2)
 #define HH_MMG_MOE(NAME, MODE, WPE)                                                                               \
     extern "C" __global__ void __launch_bounds__(256, WPE) hh_mmg_moe_##NAME(const hh_mmg_args a) {              \
         hh_mmg_body<hh_mmg_q4_k, MODE, 1, false, true>(a);                                                      \

@@ -1255,6 +1255,7 @@ struct MmgSumArgs {
     uint32_t ldt;
 };
 constexpr size_t kMmgMaxTokens = 1024;  // tokens per pass (bounds the workspaces)
+constexpr size_t kMmgFineBytes = (size_t)256 << 20;  // f32 rows: about the most bytes of a pass's split sums
 constexpr size_t kMmgLdt = kMmgMaxTokens + 64;  // tokens padded to whole tiles
 // All-Q4_K batches as f16 tokens (mode f) against passes of 64 8-bit tokens: from how many
 // tokens, by the weights.  FFN: 1024 x 2816 97 tokens 57 : 69 us, 512 x 1536 128 tokens 61 : 52,
@@ -1276,6 +1277,15 @@ size_t hh_engine::mmf_tokens(size_t batch) const {
     return last < mmi_min ? batch - last : batch;
 }
 
+// Is a one-token product of this matrix as accurate as f32 sums of f32 products?  (Q8_0, and Q6_K /
+// IQ where the ring kernels, whose x is 16-bit digits, do not take it.  Q4_0's team kernels
+// cancel, to twice the error of a batch here.)
+bool hh_engine::f32_rows(int type, size_t n, const uint8_t* w, const float* x) const {
+    if (type == HH_TYPE_Q8_0) return true;
+    const RingFmt* f = ring_fmt(type);
+    return f && type != HH_TYPE_Q4_K && (!ring || !ring_cols_ok(f, n) || (((uintptr_t)w | (uintptr_t)x) & 15u) != 0);
+}
+
 // From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
 // 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
 // one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
@@ -1287,14 +1297,18 @@ constexpr size_t kMmgRowsLds = 4 * 9216;  // Q4_K with one tile: a superblock of
 struct MmgFmt {
     int type;
     bool super, mins, half_major, paired;
+    int fine;            // hh_mmg_fine's kernels: none, of one token tile, all
     uint32_t align;      // of the weights
     uint32_t tab_bytes;  // LDS tables
     double work;         // MFMAs per step, relative
 };
 static const MmgFmt kMmgFmts[] = {
-    {HH_TYPE_Q4_0, false, false, false, true, 2, 0, 1.0},   {HH_TYPE_Q8_0, false, false, true, false, 2, 0, 1.0},
-    {HH_TYPE_Q4_K, true, true, true, true, 16, 0, 1.0},     {HH_TYPE_Q6_K, true, false, true, false, 2, 0, 1.5},
-    {HH_TYPE_IQ2_XXS, true, false, true, false, 2, 6144, 1.0}, {HH_TYPE_IQ3_XXS, true, false, true, false, 2, 4096, 1.0},
+    {HH_TYPE_Q4_0, false, false, false, true, 0, 2, 0, 1.0},
+    {HH_TYPE_Q8_0, false, false, true, false, 0, 2, 0, 1.0},
+    {HH_TYPE_Q4_K, true, true, true, true, 0, 16, 0, 1.0},
+    {HH_TYPE_Q6_K, true, false, true, false, 1, 2, 0, 1.5},
+    {HH_TYPE_IQ2_XXS, true, false, true, false, 2, 2, 6144, 1.0},
+    {HH_TYPE_IQ3_XXS, true, false, true, false, 2, 2, 4096, 1.0},
 };
 static const MmgFmt* mmg_fmt(int type) {
     for (const MmgFmt& f : kMmgFmts)
@@ -1302,22 +1316,29 @@ static const MmgFmt* mmg_fmt(int type) {
     return nullptr;
 }
 
+// f32 rows: the most chunks (128 columns) to one running sum; more are split and added exactly
+// (hh_mmg_add).  In a sum of 128 blocks the rounding of the additions alone is 2e-7 of the result:
+// 8B Q8_0 FFN, 200 tokens, 3.7e-7 against 64 bits, so 2.0e-7 (one token 2.0e-7; 6 chunks 2.15e-7).
+// That costs the splits' traffic: 512 tokens 675 -> 930 us, 200 tokens 341 -> 439, 77 tokens 268 -> 244;
+// 2048 x 5632 84 -> 84.  Q6_K's sums of 32 columns lose more: 2 chunks.
+static size_t mmg_run(const MmgFmt* f) { return f->fine == 1 ? 2 : 4; }
+
 // How a product of b tokens runs: tokens per MFMA tile (16: hi and lo as rows of one tile),
 // tiles per workgroup, and the split of the columns.
 struct MmgPlan {
     const char* mode;
     size_t rows, tt, tiles, ttiles, groups, nch, cpk, kc, stage, tile_bytes, smem;
 };
-// single: one f16 per token element (mode f)
-static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus, bool single) {
+static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus, MmgForm form) {
     MmgPlan p{};
     const size_t pad2 = (b + 63) / 64 * 64, pad1 = (b + 31) / 32 * 32;
     double us;  // of one chunk of one workgroup beside the others of its CU
+    const bool single = form == MmgForm::Single;
     if (single) {
         p.mode = "f4", p.rows = 32, p.tt = 4, us = 2.4;
     } else if (b <= 16) {
         p.mode = "s16", p.rows = 16, p.tt = 1, us = 0.7;
-    } else if ((double)pad1 * 1.2 <= (double)pad2) {
+    } else if ((double)pad1 * 1.2 <= (double)pad2 || (form == MmgForm::Fine && f->fine == 1)) {
         p.mode = "h1", p.rows = 32, p.tt = 1, us = 1.3;
     } else {
         p.mode = "h2", p.rows = 32, p.tt = 2, us = 2.2;
@@ -1334,7 +1355,8 @@ static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, 
     // split at about 3 TB/s, and a launch)
     const size_t step = f->super ? 2 : 1, slots = 2 * cus;
     double best = 1e300;
-    for (size_t kc = 1; kc <= std::min<size_t>(p.nch / step, 64); kc++) {
+    const size_t most = form == MmgForm::Fine ? mmg_run(f) : p.nch, least = (p.nch + most - 1) / most;
+    for (size_t kc = least; kc <= std::max(least, std::min<size_t>(p.nch / step, 64)); kc++) {
         size_t cpk = (p.nch + kc - 1) / kc;
         cpk = (cpk + step - 1) / step * step;
         const size_t real = (p.nch + cpk - 1) / cpk;
@@ -1361,10 +1383,10 @@ bool hh_engine::mmg_ok(int type, size_t m, size_t n, const void* w) const {
 
 // The workspaces of products (types, ms, ns, gate/up) over b tokens, in turn on one stream.
 hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus,
-                              int count, bool single) {
+                              int count, MmgForm form) {
     size_t s = 0, pb = 0;
     for (int i = 0; i < count; i++) {
-        const MmgPlan p = plan_mmg(mmg_fmt(types[i]), gus[i], ms[i], ns[i], b, (size_t)props.multiProcessorCount, single);
+        const MmgPlan p = plan_mmg(mmg_fmt(types[i]), gus[i], ms[i], ns[i], b, (size_t)props.multiProcessorCount, form);
         s = std::max(s, p.tiles * p.tile_bytes);
         if (p.kc > 1) pb = std::max(pb, p.kc * b * ms[i] * (gus[i] ? 2 : 1) * sizeof(float));
     }
@@ -1380,9 +1402,9 @@ hh_status hh_engine::mmg_grow(size_t b, const int* types, const size_t* ms, cons
 
 // h: the tokens are gate/up's output, whose largest magnitudes are there by so many row groups.
 hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h,
-                               bool single) {
+                               MmgForm form) {
     const MmgFmt* f = mmg_fmt(type);
-    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, single);
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, form);
     float* amax = (float*)ws_mg_f + (h ? kMmgLdt : 0);
     hipFunction_t fn;
     if (!h) {
@@ -1393,18 +1415,19 @@ hh_status hh_engine::mmg_stage(int type, bool gu, size_t m, size_t n, const floa
     return launch(fn, (uint32_t)(p.tiles * p.nch), 256,
                   MmgConvArgs{x, (uint8_t*)ws_mg_s, amax, h ? (float*)ws_mg_f + 2 * kMmgLdt : nullptr, p.tile_bytes,
                               (uint32_t)b, (uint32_t)n, (uint32_t)p.nch, (uint32_t)p.rows, f->mins, f->half_major,
-                              f->paired, (uint32_t)h, (uint32_t)kMmgLdt, single});
+                              f->paired, (uint32_t)h, (uint32_t)kMmgLdt, form == MmgForm::Single});
 }
 
 hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b,
-                                 float* y, int act, bool h, bool single) {
+                                 float* y, int act, bool h, MmgForm form) {
     const MmgFmt* f = mmg_fmt(type);
     const bool gu = w1 != nullptr;
-    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, single);
+    const MmgPlan p = plan_mmg(f, gu, m, n, b, (size_t)props.multiProcessorCount, form);
     size_t rb;
     HH_TRY(row_bytes(type, n, &rb));
     hipFunction_t fn;
-    HH_TRY(kernel(std::string("hh_mmg_") + format_of(type)->name + "_" + p.mode + (gu ? "_gu" : ""), &fn));
+    const char* fine = form == MmgForm::Fine && f->fine ? "_fine_" : "_";
+    HH_TRY(kernel(std::string("hh_mmg_") + format_of(type)->name + fine + p.mode + (gu ? "_gu" : ""), &fn));
     MmgArgs a{};
     a.w0 = w0;
     a.w1 = gu ? w1 : w0;
@@ -1441,22 +1464,31 @@ hh_status hh_engine::mmg_product(int type, size_t m, size_t n, const uint8_t* w0
     return HH_OK;
 }
 
+// Tokens per pass over m outputs of n columns (f32 rows: by their split sums; with half and a
+// quarter of kMmgFineBytes the 512 tokens above took 1030 and 1145 us).
+static size_t mmg_pass(const MmgFmt* f, MmgForm form, size_t m, size_t n) {
+    if (form != MmgForm::Fine) return kMmgMaxTokens;
+    const size_t splits = (n + 128 * mmg_run(f) - 1) / (128 * mmg_run(f));
+    return std::min(kMmgMaxTokens, std::max<size_t>(64, kMmgFineBytes / (splits * m * sizeof(float)) / 64 * 64));
+}
+
 hh_status hh_engine::enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b,
-                                      float* y, bool single) {
+                                      float* y, MmgForm form) {
     if (b < kMmgMinTokens || !mmg_ok(type, m, n, w)) return HH_ERR_UNSUPPORTED_DEVICE;
     const bool gu = false;
-    for (size_t nb : {std::min(b, kMmgMaxTokens), b % kMmgMaxTokens})  // a full pass and the last
-        if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1, single));
-    for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
-        const size_t nb = std::min(kMmgMaxTokens, b - b0);
-        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb, 0, single));
-        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0, false, single));
+    const size_t pass = mmg_pass(mmg_fmt(type), form, m, n);
+    for (size_t nb : {std::min(b, pass), b % pass})  // a full pass and the last
+        if (nb) HH_TRY(mmg_grow(nb, &type, &m, &n, &gu, 1, form));
+    for (size_t b0 = 0; b0 < b; b0 += pass) {
+        const size_t nb = std::min(pass, b - b0);
+        HH_TRY(mmg_stage(type, false, m, n, x + b0 * n, nb, 0, form));
+        HH_TRY(mmg_product(type, m, n, w, nullptr, nb, y + b0 * m, 0, false, form));
     }
     return HH_OK;
 }
 
 hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y,
-                                     bool single) {
+                                     MmgForm form) {
     const size_t dm = d->d_model, df = d->d_ff;
     const uint8_t* wg = pack + d->gate_off;
     const uint8_t* wu = pack + d->up_off;
@@ -1467,19 +1499,21 @@ hh_status hh_engine::enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, 
     const int types[] = {d->type_gate, d->type_down};
     const size_t ms[] = {df, dm}, ns[] = {dm, df};
     const bool gus[] = {true, false};
-    const size_t most = std::min(b, kMmgMaxTokens);
-    for (size_t nb : {most, b % kMmgMaxTokens})  // a full pass and the last
-        if (nb) HH_TRY(mmg_grow(nb, types, ms, ns, gus, 2, single));
+    const size_t pass = std::min(mmg_pass(mmg_fmt(d->type_gate), form, 2 * df, dm),
+                                 mmg_pass(mmg_fmt(d->type_down), form, dm, df)),
+                 most = std::min(b, pass);
+    for (size_t nb : {most, b % pass})  // a full pass and the last
+        if (nb) HH_TRY(mmg_grow(nb, types, ms, ns, gus, 2, form));
     const hh_status st = grow(&ws_mg_h, &ws_mg_h_cap, most * df * sizeof(float));
     if (st != HH_OK) return st == HH_ERR_OUT_OF_MEMORY ? HH_ERR_UNSUPPORTED_DEVICE : st;
-    for (size_t b0 = 0; b0 < b; b0 += kMmgMaxTokens) {
-        const size_t nb = std::min(kMmgMaxTokens, b - b0);
+    for (size_t b0 = 0; b0 < b; b0 += pass) {
+        const size_t nb = std::min(pass, b - b0);
         float* h = (float*)ws_mg_h;
-        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb, 0, single));
-        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act, false, single));
-        const size_t kc = plan_mmg(mmg_fmt(d->type_gate), true, df, dm, nb, (size_t)props.multiProcessorCount, single).kc;
-        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb, kc == 1 ? (df + 127) / 128 : (df + 255) / 256, single));
-        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0, true, single));
+        HH_TRY(mmg_stage(d->type_gate, true, df, dm, x + b0 * dm, nb, 0, form));
+        HH_TRY(mmg_product(d->type_gate, df, dm, wg, wu, nb, h, d->act, false, form));
+        const size_t kc = plan_mmg(mmg_fmt(d->type_gate), true, df, dm, nb, (size_t)props.multiProcessorCount, form).kc;
+        HH_TRY(mmg_stage(d->type_down, false, dm, df, h, nb, kc == 1 ? (df + 127) / 128 : (df + 255) / 256, form));
+        HH_TRY(mmg_product(d->type_down, dm, df, wd, nullptr, nb, y + b0 * dm, 0, true, form));
     }
     ffn_stage_valid = false;
     ffn_calls += 3 * b;
@@ -1493,7 +1527,8 @@ hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const ui
                       ((uintptr_t)x & 15u) == 0 && m <= 0xFFFFFFFFu && n <= 0xFFFFFFFFu;
     if (!mfma) {
         if (type != HH_TYPE_Q4_K) {
-            const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y, false);
+            const MmgForm form = f32_rows(type, n, w, x) ? MmgForm::Fine : MmgForm::Pair;
+            const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, batch, y, form);
             if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
         }
         for (size_t b = 0; b < batch; b++) HH_TRY(enqueue_gemv(type, m, n, w, x + b * n, y + b * m));
@@ -1501,7 +1536,7 @@ hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const ui
     }
     size_t done = 0;
     if (batch >= (mmf_min ? mmf_min : mmf_from(false, m, n)) && mmf_tokens(batch)) {
-        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, mmf_tokens(batch), y, true);
+        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, mmf_tokens(batch), y, MmgForm::Single);
         if (st == HH_OK) done = mmf_tokens(batch);
         else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
@@ -1544,7 +1579,10 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
                       mmr_ok(df, dm, batch, wg, wg, x) && mmr_ok(df, dm, batch, wu, wu, x) &&
                       (((uintptr_t)wd | (uintptr_t)x) & 15u) == 0;
     if (!mfma && !(d->type_gate == HH_TYPE_Q4_K && d->type_up == HH_TYPE_Q4_K && d->type_down == HH_TYPE_Q4_K)) {
-        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y, false);
+        // (without the ring kernels, gate/up of one format is one team kernel's, in f32)
+        const bool f32 = !ring_ok(d, wg, wu, wd, x) && d->type_gate != HH_TYPE_Q4_K && d->type_gate != HH_TYPE_Q4_0 &&
+                         f32_rows(d->type_down, df, wd, nullptr);
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, batch, y, f32 ? MmgForm::Fine : MmgForm::Pair);
         if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     if (q4km) {
@@ -1574,7 +1612,7 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
     }
     size_t done = 0;
     if (batch >= (mmf_min ? mmf_min : mmf_from(true, df, dm)) && mmf_tokens(batch)) {
-        const hh_status st = enqueue_mmg_ffn(d, pack, x, mmf_tokens(batch), y, true);
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, mmf_tokens(batch), y, MmgForm::Single);
         if (st == HH_OK) done = mmf_tokens(batch);
         else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
@@ -2022,7 +2060,9 @@ static std::vector<std::string> required_kernels() {
     for (const MmgFmt& f : kMmgFmts)
         for (const char* mode : {"s16", "h1", "h2"})
             for (const char* gu : {"", "_gu"})
-                k.push_back(std::string("hh_mmg_") + format_of(f.type)->name + "_" + mode + gu);
+                for (const char* fine : {"_", "_fine_"})
+                    if (!fine[1] || f.fine == 2 || (f.fine && std::string(mode) != "h2"))
+                        k.push_back(std::string("hh_mmg_") + format_of(f.type)->name + fine + mode + gu);
     for (const char* f : {"hh_bst_q8_0", "hh_bst_q4_0"})
         for (const char* v : {"_pair", "_wide", "_pair_gu", "_wide_gu"}) k.push_back(std::string(f) + v);
     k.push_back("hh_lut_gemv");

@@ -85,6 +85,9 @@ struct hh_event {
 };
 
 struct MoegArgs;
+// Tokens of mmg.hip's products: two f16 each, or one (Q4_K); Fine: two, and sums as accurate as f32
+// products summed in f32.
+enum class MmgForm { Pair, Single, Fine };
 
 struct hh_engine {
     int device = 0;
@@ -296,19 +299,19 @@ struct hh_engine {
     // any launch) when shape, type or alignment does not fit or the workspaces cannot be had.
     bool mmg_ok(int type, size_t m, size_t n, const void* w) const;
     hh_status mmg_grow(size_t b, const int* types, const size_t* ms, const size_t* ns, const bool* gus, int count,
-                       bool single);
+                       MmgForm form);
     // x [b][n] -> stages of `type`'s order (h: x is gate/up's output, its
     // largest magnitudes known by so many row groups)
-    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h, bool single);
+    hh_status mmg_stage(int type, bool gu, size_t m, size_t n, const float* x, size_t b, size_t h, MmgForm form);
     // the product of the staged tokens: GEMM (w1 null) into y [b][m], or gate/up + act into y
     hh_status mmg_product(int type, size_t m, size_t n, const uint8_t* w0, const uint8_t* w1, size_t b, float* y,
-                          int act, bool h, bool single);
-    // single: one f16 per token element (Q4_K), for the first mmf_tokens of a batch
-    size_t mmf_tokens(size_t batch) const;
+                          int act, bool h, MmgForm form);
+    size_t mmf_tokens(size_t batch) const;  // how many of an all-Q4_K batch's tokens may be single f16
+    bool f32_rows(int type, size_t n, const uint8_t* w, const float* x) const;
     hh_status enqueue_mmg_gemm(int type, size_t m, size_t n, const uint8_t* w, const float* x, size_t b, float* y,
-                               bool single);
+                               MmgForm form);
     hh_status enqueue_mmg_ffn(const hh_ffn_desc* d, const uint8_t* pack, const float* x, size_t b, float* y,
-                              bool single);
+                              MmgForm form);
     // MoE routing of T tokens (device pointers) and the grouped expert FFN.
     hh_status enqueue_moe_route(const hh_moe_desc* d, const float* logits, const float* bias, size_t T,
                                 int32_t* ids, float* wts);

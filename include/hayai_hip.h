@@ -173,7 +173,8 @@ void hh_pending_destroy(hh_pending* p);
  * outputs[b*m + r] = W[r] . inputs[b*n .. b*n+n) for b < batch.  Host weights and
  * activations, blocking.  Q4_K with batch >= 2 runs on the matrix cores in passes of up to
  * 64 tokens; the other quantized types with batch >= 4 in passes of up to 1024 tokens at f32
- * accuracy (measured within 4e-7 of the 64-bit product); F32 and F16 loop over tokens.
+ * accuracy (measured within 2e-7 of the 64-bit product, and no further than the same tokens one at
+ * a time); F32 and F16 loop over tokens.
  * Precision of the Q4_K passes:
  *   - passes of 2..16 tokens: f32 activations (as f16 hi + lo pairs), f32 accumulation:
  *     within ~1e-6 of the f32 product;

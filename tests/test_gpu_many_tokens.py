@@ -105,6 +105,51 @@ def make_pack(engine, types, d_model, d_ff, cfg):
     return lay, ws, pack
 
 
+def rms(err):
+    return float(np.sqrt(np.mean(err ** 2)))
+
+
+# where one token at a time is f32 products summed in f32 (Q8_0; Q6_K and IQ in rows of an odd
+# number of blocks): long and split columns, one workgroup's whole row, each tiling
+@pytest.mark.parametrize("t,m,n,batch", [
+    (Q8_0, 4160, 4096, 1000), (Q8_0, 2048, 8192, 24), (Q8_0, 2048, 4096, 8), (Q6_K, 2048, 3840, 24),
+    (Q6_K, 2048, 768, 40), (IQ2, 2048, 3840, 12), (IQ2, 2048, 2304, 64), (IQ3, 2048, 3840, 24),
+])
+def test_as_accurate_as_one_token(engine, t, m, n, batch):
+    print(f"[case] accuracy type={t} m={m} n={n} batch={batch}", flush=True)
+    w = synth.matrix(t, m, n, 74)
+    X = synth.normal(75, batch * n).reshape(batch, n)
+    rows = w.reshape(m, -1)[:2048]
+    Y = engine.ggml_gemv_batched(t, m, n, w, X, batch).reshape(batch, m)[:8, :2048]
+    one = np.stack([engine.ggml_gemv_dispatch(t, len(rows), n, rows.reshape(-1), x) for x in X[:8]])
+    ref = X[:8].astype(np.float64) @ oracle.dequant(t, rows.reshape(-1), rows.shape[0] * n).reshape(-1, n).T.astype(np.float64)
+    ours, theirs = rms(Y - ref), rms(one - ref)
+    print(f"  batch {ours:.3e} one at a time {theirs:.3e}", flush=True)
+    # 16384 outputs a side: the root mean squares of two equal errors are within 2 %
+    assert ours <= 1.04 * theirs
+
+
+@pytest.mark.parametrize("types,d_model,d_ff,batch", [((Q8_0,) * 3, 2048, 5632, 77), ((Q8_0,) * 3, 2048, 5632, 400),
+                                                      ((IQ3,) * 3, 2304, 3328, 40), ((Q6_K,) * 3, 2304, 3328, 70)])
+def test_ffn_as_accurate_as_one_token(engine, types, d_model, d_ff, batch):
+    print(f"[case] ffn accuracy {types} {d_model}x{d_ff} batch={batch}", flush=True)
+    lay, ws, pack = make_pack(engine, types, d_model, d_ff, 76)
+    desc = engine.ffn_desc(types, d_model, d_ff, lay)
+    X = synth.normal(77, batch * d_model).reshape(batch, d_model)
+    Y = engine.ffn_batched(desc, pack, 0, X)[:8]
+    one = np.stack([engine.ffn(desc, pack, 0, x) for x in X[:8]])
+    g, u, d = (oracle.dequant(t, w, r * c).reshape(r, c).astype(np.float64)
+               for t, w, (r, c) in zip(types, ws, [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]))
+    x = X[:8].astype(np.float64)
+    gate = x @ g.T
+    ref = (gate / (1 + np.exp(-gate)) * (x @ u.T)) @ d.T
+    ours, theirs = rms(Y - ref), rms(one - ref)
+    print(f"  batch {ours:.3e} one at a time {theirs:.3e}", flush=True)
+    # the sums lose what the one-token ones do, about 1e-7 a product; the 22 bits of x and of h add 4e-8
+    # each, independently: sqrt(1 + 0.4 ** 2) = 1.08, and 2 % between samples as above
+    assert ours <= 1.1 * theirs
+
+
 @pytest.mark.parametrize("types,d_model,d_ff,batch,act", [
     ((Q4_0,) * 3, 576, 1536, 5, 0), ((Q8_0,) * 3, 96, 160, 40, 0), ((Q6_K,) * 3, 768, 1280, 33, 1),
     ((Q4_K, Q4_K, Q6_K), 512, 1536, 70, 0), ((IQ2,) * 3, 512, 768, 16, 0), ((IQ3, IQ3, Q8_0), 256, 512, 17, 0),
