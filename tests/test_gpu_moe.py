@@ -273,13 +273,47 @@ def _engine_with_env(**env):
                 os.environ[k] = v
 
 
+@pytest.fixture(scope="module")
+def without_mmg():
+    eng = _engine_with_env(HAYAI_HIP_MMG="0")
+    yield eng
+    eng.close()
+
+
 @pytest.mark.parametrize("T", [512, 513])
 def test_moe_grouped_at_the_pair_limit(engine, T):
-    # 512 tokens x top-8 = 4096 (token, slot) pairs, the most the grouped kernels take in one
-    # call (every expert active, ~32 pairs each: several LDS passes per expert, records and
-    # rank masks at full size); 513 tokens go to the per-(token, expert) kernels instead.
+    # 512 tokens x top-8 = 4096 (token, slot) pairs, the most one grouping takes (every expert
+    # active, ~32 pairs each); 513 tokens are two passes, the second of one token.
     # Routed on the GPU (hh_moe_dev) and from given ids (hh_moe_ffn_dev): bit-identical, and
-    # each token against the oracle.
+    # each token against the oracle.  Here on the matrix cores, in tiles of one expert's pairs.
+    pair_limit(engine, T)
+
+
+@pytest.mark.parametrize("T", [512, 513])
+def test_moe_grouped_at_the_pair_limit_without_the_matrix_cores(without_mmg, T):
+    # the same on the grouped kernels: several LDS stages of pairs per expert, records at full size
+    pair_limit(without_mmg, T)
+
+
+def test_moe_grouped_with_one_crowded_expert(engine):
+    # 300 pairs on 128 experts are too few for the matrix cores (2.3 each), but half of them are one
+    # expert's: its grouped workgroups stage 150 pairs, in order, many times over
+    E, k, d_model, d_ff, T = 128, 2, 512, 256, 150
+    print(f"[case] moe crowded expert E={E} k={k} T={T}", flush=True)
+    buf, host, stride, offs = make_experts(engine, E, d_model, d_ff, 92)
+    d = engine.moe_desc(d_model, d_ff, E, k, stride, offs)
+    ids = np.stack([np.full(T, 5), (np.arange(T) % 127 + 6) % E], axis=1).astype(np.int32)
+    w = np.random.default_rng(12).uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    x = synth.normal(18, T * d_model).reshape(T, d_model)
+    y = engine.alloc(4 * T * d_model)
+    engine.moe_ffn_dev(d, buf, 0, engine.upload(x), 0, T, engine.upload(ids), 0, engine.upload(w), 0, y, 0)
+    Y = y.read(np.float32, T * d_model).reshape(T, d_model)
+    for t in range(T):
+        ref = oracle.moe_token(Q4_K, d_model, d_ff, host, stride, offs, ids[t], w[t], x[t])
+        assert np.max(np.abs(Y[t] - ref)) <= REL_TOL * np.max(np.abs(ref)), t
+
+
+def pair_limit(engine, T):
     E, k, d_model, d_ff = 128, 8, 256, 256
     oracle.set_threads(min(16, oracle.max_threads()))
     print(f"[case] moe pair limit E={E} k={k} {d_model}x{d_ff} T={T}", flush=True)
