@@ -935,8 +935,9 @@ hh_status hh_engine::enqueue_ffn_block_stack(const hh_ffn_desc* d, const uint8_t
 // The FFN residual block of one token: y = x + FFN(RMSNorm(x)) (ffn_apply,
 // crates/hayai-core/src/hybrid_infer.rs:883-936, with rms_norm of
 // crates/hayai-cpu/src/attention.rs:142-147).  The ring kernels fuse both neighbours: gate/up
-// normalizes x while quantizing it, down adds the residual as it stores y.  Other layouts
-// run RMSNorm, the FFN and the residual add as three steps.  y may be x.
+// normalizes x while quantizing it, down adds the residual as it stores y; so does the Q8_0 / Q4_0 row
+// stream, as it brings x into LDS.  Other layouts, and small layers, run RMSNorm, the FFN and the
+// residual add as three steps.  y may be x.
 hh_status hh_engine::enqueue_ffn_block(const hh_ffn_desc* d, const uint8_t* pack, const float* x, const float* norm,
                                        float eps, float* y) {
     const uint8_t* wg = pack + d->gate_off;
@@ -1572,8 +1573,9 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
     const uint8_t* wd = pack + d->down_off;
     const bool mfma = d->type_gate == HH_TYPE_Q4_K && d->type_up == HH_TYPE_Q4_K && d->type_down == HH_TYPE_Q4_K &&
                       batch >= 2 && !q4k_generic && (((uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd | (uintptr_t)x) & 15u) == 0;
-    // Q4_K_M layers (Q4_K gate/up, Q6_K down): gate and up for all tokens as weight-stream MFMA
-    // GEMMs, the activation over [batch][d_ff], then the Q6_K ring GEMV per token.
+    // Q4_K_M layers (Q4_K gate/up, Q6_K down) that mmg.hip does not take (HAYAI_HIP_MMG=0, or no memory
+    // for its workspaces): gate and up for all tokens as weight-stream MFMA GEMMs, the activation over
+    // [batch][d_ff], then the Q6_K ring GEMV per token.
     const bool q4km = d->type_gate == HH_TYPE_Q4_K && d->type_up == HH_TYPE_Q4_K && d->type_down == HH_TYPE_Q6_K &&
                       batch >= 4 && batch <= kMmrMaxTokens && df % 512 == 0 && !capturing &&
                       mmr_ok(df, dm, batch, wg, wg, x) && mmr_ok(df, dm, batch, wu, wu, x) &&

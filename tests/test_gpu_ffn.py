@@ -447,9 +447,26 @@ def test_small_ffn_one_launch_equals_two_launches(engine, types, d_model, d_ff):
 
 @pytest.mark.parametrize("batch", [2, 4, 16])
 def test_q4k_m_batched_ffn_matches_oracle(engine, batch):
-    # Batched tokens through a Q4_K_M layer: gate/up as weight-stream MFMA GEMMs, the
-    # activation, the Q6_K ring GEMV per token (batch >= 4; batch 2 runs the one-token op per
-    # token); each token against the oracle.
+    # Batched tokens through a Q4_K_M layer: gate/up + activation and down on the matrix cores
+    # (mmg.hip, batch >= 4; batch 2 runs the one-token op per token); each token against the oracle.
+    q4k_m_batched(engine, batch)
+
+
+@pytest.mark.parametrize("batch", [2, 4, 16, 17])
+def test_q4k_m_batched_ffn_without_mmg(monkeypatch, batch):
+    # HAYAI_HIP_MMG=0: 4..16 tokens with gate/up as weight-stream MFMA GEMMs, the activation, and the
+    # Q6_K ring GEMV per token; fewer and more one token at a time
+    monkeypatch.setenv("HAYAI_HIP_MMG", "0")
+    eng = hayai_amd.HipEngine(0)
+    try:
+        Y, one = q4k_m_batched(eng, batch)
+        if batch in (2, 17):
+            np.testing.assert_array_equal(Y, one)
+    finally:
+        eng.close()
+
+
+def q4k_m_batched(engine, batch):
     types, d_model, d_ff = (12, 12, 14), 4096, 14336
     print(f"[case] q4_k_m batched B={batch}", flush=True)
     oracle.set_threads(min(16, oracle.max_threads()))
@@ -463,3 +480,4 @@ def test_q4k_m_batched_ffn_matches_oracle(engine, batch):
         worst = max(worst, rel_err(Y[b], ref))
     print(f"  worst per-token rel_err {worst:.3e}", flush=True)
     assert worst <= REL_TOL, worst
+    return Y, np.stack([engine.ffn(desc, pack, 0, x) for x in X])
