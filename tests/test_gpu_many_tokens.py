@@ -109,11 +109,13 @@ def rms(err):
     return float(np.sqrt(np.mean(err ** 2)))
 
 
-# where one token at a time is f32 products summed in f32 (Q8_0; Q6_K and IQ in rows of an odd
-# number of blocks): long and split columns, one workgroup's whole row, each tiling
+# where one token at a time is f32 products summed in f32 (Q8_0, Q4_0; Q6_K and IQ in rows of an odd
+# number of blocks): long and split columns, one workgroup's whole row, each tiling; and where it is
+# 16-bit digits (the last three), which a lost lo operand, 2^-12 of x, would pass by ten times
 @pytest.mark.parametrize("t,m,n,batch", [
     (Q8_0, 4160, 4096, 1000), (Q8_0, 2048, 8192, 24), (Q8_0, 2048, 4096, 8), (Q6_K, 2048, 3840, 24),
     (Q6_K, 2048, 768, 40), (IQ2, 2048, 3840, 12), (IQ2, 2048, 2304, 64), (IQ3, 2048, 3840, 24),
+    (Q4_0, 2048, 4096, 24), (Q4_0, 2048, 8192, 8), (Q6_K, 2048, 4096, 64), (IQ2, 2048, 4096, 24), (IQ3, 2048, 2048, 9),
 ])
 def test_as_accurate_as_one_token(engine, t, m, n, batch):
     print(f"[case] accuracy type={t} m={m} n={n} batch={batch}", flush=True)
