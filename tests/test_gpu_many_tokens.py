@@ -109,21 +109,33 @@ def rms(err):
     return float(np.sqrt(np.mean(err ** 2)))
 
 
-# where one token at a time is f32 products summed in f32 (Q8_0, Q4_0; Q6_K and IQ in rows of an odd
-# number of blocks): long and split columns, one workgroup's whole row, each tiling; and where it is
+@pytest.fixture(scope="module")
+def team_kernels():
+    import os
+    os.environ["HAYAI_HIP_BLOCK_STREAM"] = "0"  # Q8_0 / Q4_0 too
+    try:
+        eng = hayai_amd.HipEngine(0)
+    finally:
+        del os.environ["HAYAI_HIP_BLOCK_STREAM"]
+    yield eng
+    eng.close()
+
+
+# where the team kernels' one token at a time is f32 products summed in f32 (Q8_0, Q4_0; Q6_K and IQ
+# in rows of an odd number of blocks): long and split columns, one workgroup's whole row, each tiling; and where it is
 # 16-bit digits (the last three), which a lost lo operand, 2^-12 of x, would pass by ten times
 @pytest.mark.parametrize("t,m,n,batch", [
     (Q8_0, 4160, 4096, 1000), (Q8_0, 2048, 8192, 24), (Q8_0, 2048, 4096, 8), (Q6_K, 2048, 3840, 24),
     (Q6_K, 2048, 768, 40), (IQ2, 2048, 3840, 12), (IQ2, 2048, 2304, 64), (IQ3, 2048, 3840, 24),
     (Q4_0, 2048, 4096, 24), (Q4_0, 2048, 8192, 8), (Q6_K, 2048, 4096, 64), (IQ2, 2048, 4096, 24), (IQ3, 2048, 2048, 9),
 ])
-def test_as_accurate_as_one_token(engine, t, m, n, batch):
+def test_as_accurate_as_one_token(engine, team_kernels, t, m, n, batch):
     print(f"[case] accuracy type={t} m={m} n={n} batch={batch}", flush=True)
     w = synth.matrix(t, m, n, 74)
     X = synth.normal(75, batch * n).reshape(batch, n)
     rows = w.reshape(m, -1)[:2048]
     Y = engine.ggml_gemv_batched(t, m, n, w, X, batch).reshape(batch, m)[:8, :2048]
-    one = np.stack([engine.ggml_gemv_dispatch(t, len(rows), n, rows.reshape(-1), x) for x in X[:8]])
+    one = np.stack([team_kernels.ggml_gemv_dispatch(t, len(rows), n, rows.reshape(-1), x) for x in X[:8]])
     ref = X[:8].astype(np.float64) @ oracle.dequant(t, rows.reshape(-1), rows.shape[0] * n).reshape(-1, n).T.astype(np.float64)
     ours, theirs = rms(Y - ref), rms(one - ref)
     print(f"  batch {ours:.3e} one at a time {theirs:.3e}", flush=True)
@@ -133,13 +145,14 @@ def test_as_accurate_as_one_token(engine, t, m, n, batch):
 
 @pytest.mark.parametrize("types,d_model,d_ff,batch", [((Q8_0,) * 3, 2048, 5632, 77), ((Q8_0,) * 3, 2048, 5632, 400),
                                                       ((IQ3,) * 3, 2304, 3328, 40), ((Q6_K,) * 3, 2304, 3328, 70)])
-def test_ffn_as_accurate_as_one_token(engine, types, d_model, d_ff, batch):
+def test_ffn_as_accurate_as_one_token(engine, team_kernels, types, d_model, d_ff, batch):
     print(f"[case] ffn accuracy {types} {d_model}x{d_ff} batch={batch}", flush=True)
     lay, ws, pack = make_pack(engine, types, d_model, d_ff, 76)
     desc = engine.ffn_desc(types, d_model, d_ff, lay)
     X = synth.normal(77, batch * d_model).reshape(batch, d_model)
     Y = engine.ffn_batched(desc, pack, 0, X)[:8]
-    one = np.stack([engine.ffn(desc, pack, 0, x) for x in X[:8]])
+    _, _, own = make_pack(team_kernels, types, d_model, d_ff, 76)
+    one = np.stack([team_kernels.ffn(desc, own, 0, x) for x in X[:8]])
     g, u, d = (oracle.dequant(t, w, r * c).reshape(r, c).astype(np.float64)
                for t, w, (r, c) in zip(types, ws, [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]))
     x = X[:8].astype(np.float64)
