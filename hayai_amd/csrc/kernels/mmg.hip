@@ -17,7 +17,8 @@
 // into two f16, hi + lo, which carry 22 bits; products are summed in f32 by the matrix cores
 // over one scale block (32 or 256 columns), then d times that is added to the running sum.
 // Measured against 64 bits (2-norm): 6e-8 to 1.7e-7 a product, 1.5e-7 to 4e-7 an FFN; for rows that the
-// one-token kernels sum in f32 no more than theirs, by short sums (hh_mmg_fine, and at most 512 columns to a split).
+// one-token kernels sum in f32 no more than theirs, by short sums (hh_mmg_fine, and at most 512
+// columns to a split).
 // The Q4_K minimum is dmin * sum_j m_j X_j with X_j the f32 sum of the token's 32 elements of
 // sub-block j, as hi + lo f16: one MFMA per superblock (k slots 0..7 hi, 8..15 lo).
 //
@@ -29,19 +30,22 @@
 //   columns 16 h + 8 step + e  (Q8_0, Q4_K, Q6_K, IQ)   or   16 step + 8 h + e  (Q4_0),
 //   e natural (Q8_0, IQ) or 0 2 1 3 4 6 5 7 (nibble pairs of a dword).
 // Weights go from global memory to registers to the matrix core (Q4_K with one token tile by way
-// of LDS, hh_mmg_body); tokens pass through LDS, shared by the workgroup's four waves.  A wave owns 64 weight rows (32 of gate and the same 32
-// of up), so each 1 KB token fragment read from LDS feeds two MFMAs.
+// of LDS, hh_mmg_body); tokens pass through LDS, shared by the workgroup's four waves.  A wave owns
+// 64 weight rows (32 of gate and the same 32 of up), so each 1 KB token fragment read from LDS
+// feeds two MFMAs.
 //
 // Modes (chosen by the token count alone, plan_mmg): h<TT>: TT tiles of 32 tokens, hi and lo as
 // two MFMAs; s16: 16 tokens, hi in A rows 0..15 and lo in rows 16..31 of one MFMA, added at the end.
 //
-// What bounds it: at hundreds of tokens the matrix cores with the weight decode beside them (8B
-// FFN, 512 tokens, 2 x 180 GFLOP of hi and lo: 0.44 ms IQ2_XXS .. 0.72 ms Q8_0, 500 .. 820 TFLOP/s;
-// one token at a time these took 12 .. 39 ms); at 4..16 tokens the weight stream's latency (8B
-// Q6_K FFN, 16 tokens: 106 us against 779 us).
+// What bounds it: at hundreds of tokens the matrix cores, busy for 45 to 49 % of a CU's active cycles
+// (Q4_K, Q6_K), with the weight decode beside them at two waves per SIMD.  8B FFN, 512 tokens, 2 x 180
+// GFLOP of hi and lo: 0.43 ms IQ2_XXS, 0.60 ms Q6_K, 0.93 ms Q8_0 with its splits, 390 .. 840 TFLOP/s
+// (one token at a time these took 12 .. 39 ms).  With few tokens the loads: a lane's row is a line of
+// its own in every instruction (Q8_0, 77 tokens: matrix cores 13 % busy, waits 24 %); at 4..16 tokens
+// the weight stream's latency (8B Q6_K FFN, 16 tokens: 82 us against 779 us).
 //
 // MoE (hh_mmg_moe_*): the (token, slot) pairs of an expert in tiles of 16 or 32, one launch over
-// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 228 us a layer.
+// every (tile, row group).  128 experts of 2048 x 768, 512 tokens: 1220 -> 225 us a layer.
 //
 // Token stages: [tile][128-column chunk][group 0..3][step 0..1][hi, lo][lane][8 f16], for Q4_K
 // followed after every second chunk by the sums [lane][8 f16] (lane half 0: hi of sub-blocks
@@ -123,7 +127,7 @@ struct hh_mmg_k {
 // bytes: 3 loads for Q4_0, 5 for Q8_0, where a load of each half block and each d took 8), and
 // `ready` exchanges halves with the lane of the same row: then every lane has its half of all four.
 // With its 64 lanes in 64 places every load holds the address unit for as long as 64 lines take.
-// 8B FFN: 512 tokens Q8_0 888 -> 717 us, Q4_0 593 -> 455 us; 16 tokens Q4_0 92 -> 72 us.
+// When it was made, 8B FFN: 512 tokens Q8_0 888 -> 717 us, Q4_0 593 -> 455 us; 16 tokens Q4_0 92 -> 72.
 HH_DEV void hh_swap32(uint32_t& a, uint32_t& b) {  // a's upper 32 lanes with b's lower 32
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     a = r[0];
@@ -132,7 +136,8 @@ HH_DEV void hh_swap32(uint32_t& a, uint32_t& b) {  // a's upper 32 lanes with b'
 
 // Two blocks of QW code dwords each: w[0] low half d of the first, then its codes at half a dword,
 // w[QW] high half d of the second, then its codes.  After `ready` w[0 ..] groups 0, 2, w[QW] and dx
-// the four d, w[QW + 1 ..] groups 1, 3 (in place: a copy stays live beside it and spills).
+// the four d, w[QW + 1 ..] groups 1, 3 (in place, for a copy would stay live beside it: two token
+// tiles of Q8_0 are at 256 registers and spill about ten even so).
 template <uint32_t QW>
 struct hh_mmg_pair {
     static constexpr uint32_t BB = 4 * QW + 2;
@@ -988,7 +993,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
         // A superblock of the wave's 64 rows comes as nine runs of whole pieces, about 14 lines
         // each, where twelve loads of a lane's own row took 64 lines each, and is on its way for
         // two chunks instead of one.  Only where a workgroup has one token tile: two workgroups
-        // of a CU fit LDS beside each other so.  512-token MoE layer 258 -> 246 us.
+        // of a CU fit LDS beside each other so.  512-token MoE layer 258 -> 246 us when it was made.
         char* const slot = hh_smem + 2 * BUF + wave * HH_MMG_WSLOT;
         const uint8_t* src[9];  // piece 64 i + lane of the slot: row / 9, 16 bytes each
 #pragma unroll
@@ -1067,7 +1072,7 @@ HH_DEV void hh_mmg_body(const hh_mmg_args& a) {
 // is multiplied by d_before / d (f32), and the products stay those of exact integers sc q.  In
 // the same units the minimum is -(dmin / d) m_j X_j, whose factors enter the bf16 matrix core as
 // two bf16 each (f32's range, 16 bits).  8B FFN, 512 tokens: 558 us as 8 passes of 8-bit tokens,
-// 294 us here (613 TFLOP/s); error against 64 bits 1.2e-2 -> 5e-4.  A superblock with d = 0 keeps the unit before it and
+// 269 us here (669 TFLOP/s, matrix cores 45 % busy); error against 64 bits 1.2e-2 -> 5e-4.  A superblock with d = 0 keeps the unit before it and
 // zero scales.
 typedef __bf16 hh_b8 __attribute__((ext_vector_type(8)));
 

@@ -1333,7 +1333,10 @@ struct MmgPlan {
 static MmgPlan plan_mmg(const MmgFmt* f, bool gu, size_t m, size_t n, size_t b, size_t cus, MmgForm form) {
     MmgPlan p{};
     const size_t pad2 = (b + 63) / 64 * 64, pad1 = (b + 31) / 32 * 32;
-    double us;  // of one chunk of one workgroup beside the others of its CU
+    // What a chunk of one workgroup counts against a round's fixed 3 and the splits' traffic, found by
+    // trial.  It is not a chunk's time, which with two workgroups on a CU is (rocprofv3) 5.7 us of f4,
+    // 4.3 of Q4_K h2, 7.3 of Q6_K h2, 5 of Q8_0 h1.
+    double us;
     const bool single = form == MmgForm::Single;
     if (single) {
         p.mode = "f4", p.rows = 32, p.tt = 4, us = 2.4;
