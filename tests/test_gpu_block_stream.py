@@ -127,3 +127,41 @@ def test_infinite_element_in_the_last_block(stream, t, m, n):
     W = oracle.dequant(t, w, m * n).reshape(m, n).astype(np.float64)
     with np.errstate(invalid="ignore"):
         np.testing.assert_array_equal(y, (W * x.astype(np.float64)).sum(axis=1).astype(np.float32))
+
+
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+def test_captured_blocks_replay(engine, t):
+    # two residual blocks and a product on the row stream in one graph: every replay, with eager
+    # calls between them, gives the eager bits
+    d_model, d_ff = 2048, 5632
+    shapes = [(d_ff, d_model), (d_ff, d_model), (d_model, d_ff)]
+    lay = hayai_amd.LayerPackLayout.ffn_only(*[hayai_amd.QuantMatrix("m", c, r, t) for r, c in shapes])
+    ws = [synth.matrix(t, r, c, synth.seed_for(82, t, i)) for i, (r, c) in enumerate(shapes)]
+    pack = engine.alloc(lay.total)
+    for w, off in zip(ws, (lay.gate_off, lay.up_off, lay.down_off)):
+        pack.write(w, off)
+    desc = engine.ffn_desc((t,) * 3, d_model, d_ff, lay)
+    x, norm = engine.upload(synth.normal(83, d_model)), engine.upload(np.ones(d_model, np.float32))
+    y, z = engine.alloc(4 * d_model), engine.alloc(4 * d_ff)
+
+    def step():
+        engine.ffn_block_dev(desc, pack, 0, norm, 0, 1e-5, x, 0, y, 0)
+        engine.ffn_block_dev(desc, pack, 0, norm, 0, 1e-5, y, 0, y, 0)
+        engine.gemv_dev(t, d_ff, d_model, pack, lay.gate_off, y, 0, z, 0)
+
+    step()
+    engine.sync()
+    want = y.read(np.float32, d_model), z.read(np.float32, d_ff)
+    g = engine.capture(step)
+    for k in range(4):
+        x.write(synth.normal(84 + k, d_model), 0)  # other inputs in the same buffer
+        step()
+        engine.sync()
+        eager = y.read(np.float32, d_model), z.read(np.float32, d_ff)
+        assert not np.array_equal(eager[0], want[0])
+        y.write(np.zeros(d_model, np.float32), 0)
+        g.launch()
+        engine.sync()
+        np.testing.assert_array_equal(y.read(np.float32, d_model), eager[0])
+        np.testing.assert_array_equal(z.read(np.float32, d_ff), eager[1])
+    g.free()
