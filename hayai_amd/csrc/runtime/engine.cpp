@@ -1258,14 +1258,15 @@ struct MmgSumArgs {
 constexpr size_t kMmgMaxTokens = 1024;  // tokens per pass (bounds the workspaces)
 constexpr size_t kMmgFineBytes = (size_t)256 << 20;  // f32 rows: about the most bytes of a pass's split sums
 constexpr size_t kMmgLdt = kMmgMaxTokens + 64;  // tokens padded to whole tiles
-// All-Q4_K batches as f16 tokens (mode f) against passes of 64 8-bit tokens: from how many
-// tokens, by the weights.  FFN: 1024 x 2816 97 tokens 57 : 69 us, 512 x 1536 128 tokens 61 : 52,
-// 160 tokens 62 : 70.  One matrix: 128256 x 2048 65 tokens 93 : 166, 32000 x 2048 97 tokens
-// 61 : 69, 4096 x 4096 128 tokens 43 : 39, 200 tokens 43 : 69.
+// All-Q4_K batches as f16 tokens (mode f) against passes of 64 8-bit tokens, of batches past one
+// such pass: from how many tokens (mmf_tokens of the batch), by the weights.  FFN: 1024 x 2816 97
+// tokens 57 : 69 us, 512 x 1536 128 tokens 61 : 52, 160 tokens 62 : 70.  One matrix: 128256 x 2048 64
+// tokens and one more 113 : 157, 96 tokens 86 : 207, 32000 x 2048 97 tokens 61 : 69, 4096 x 4096 128
+// tokens 43 : 39.
 static size_t mmf_from(bool ffn, size_t m, size_t n) {
     const size_t w = m * n;
     if (ffn) return w >= (size_t)2 << 20 ? 97 : 144;
-    return w >= (size_t)100 << 20 ? 65 : w >= (size_t)48 << 20 ? 97 : 136;
+    return w >= (size_t)100 << 20 ? 64 : w >= (size_t)48 << 20 ? 97 : 136;
 }
 
 // The leading tokens of an all-Q4_K batch that may enter as one f16: those of the passes that
@@ -1287,8 +1288,8 @@ bool hh_engine::f32_rows(int type, size_t n, const uint8_t* w, const float* x) c
     return f && type != HH_TYPE_Q4_K && (!ring || !ring_cols_ok(f, n) || (((uintptr_t)w | (uintptr_t)x) & 15u) != 0);
 }
 
-// From how many tokens: below 4 the one-token kernels are as fast (8B Q6_K FFN: 2 tokens 100 us,
-// 4 tokens 202 us against 103; 8B Q4_K_M: 4 tokens 91 against 86), and a layer with the
+// From how many tokens: below 4 the one-token kernels are as fast or nearly (8B Q6_K FFN: 2 tokens 100 us,
+// 4 tokens 197 us against 81; 8B Q4_K_M: 4 tokens 89 against 61), and a layer with the
 // one-launch FFN (small_ffn.hip, 7 us a token) gains from 5 (576 x 1536 Q4_0: 4 tokens 29 us
 // against 32, 6 tokens 43 against 32).
 constexpr size_t kMmgMinTokens = 4, kMmgMinTokensSmallFfn = 5;
@@ -1539,9 +1540,10 @@ hh_status hh_engine::enqueue_gemv_batched(int type, size_t m, size_t n, const ui
         return HH_OK;
     }
     size_t done = 0;
-    if (batch >= (mmf_min ? mmf_min : mmf_from(false, m, n)) && mmf_tokens(batch)) {
-        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, mmf_tokens(batch), y, MmgForm::Single);
-        if (st == HH_OK) done = mmf_tokens(batch);
+    const size_t nf = mmf_tokens(batch);
+    if (nf && (mmf_min ? batch >= mmf_min : batch > kMmMaxTokens && nf >= mmf_from(false, m, n))) {
+        const hh_status st = enqueue_mmg_gemm(type, m, n, w, x, nf, y, MmgForm::Single);
+        if (st == HH_OK) done = nf;
         else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     for (size_t b0 = done; b0 < batch; b0 += kMmMaxTokens) {
@@ -1616,9 +1618,10 @@ hh_status hh_engine::enqueue_ffn_batched(const hh_ffn_desc* d, const uint8_t* pa
         return HH_OK;
     }
     size_t done = 0;
-    if (batch >= (mmf_min ? mmf_min : mmf_from(true, df, dm)) && mmf_tokens(batch)) {
-        const hh_status st = enqueue_mmg_ffn(d, pack, x, mmf_tokens(batch), y, MmgForm::Single);
-        if (st == HH_OK) done = mmf_tokens(batch);
+    const size_t nf = mmf_tokens(batch);
+    if (nf && (mmf_min ? batch >= mmf_min : batch > kMmMaxTokens && nf >= mmf_from(true, df, dm))) {
+        const hh_status st = enqueue_mmg_ffn(d, pack, x, nf, y, MmgForm::Single);
+        if (st == HH_OK) done = nf;
         else if (st != HH_ERR_UNSUPPORTED_DEVICE) return st;
     }
     for (size_t b0 = done; b0 < batch; b0 += kMmMaxTokens) {
